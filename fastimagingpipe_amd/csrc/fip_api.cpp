@@ -665,17 +665,14 @@ int fip_autotune(size_t image_size, size_t num_baselines, float cell_size, int r
         const int rows[3] = {1, 2, 4};
         const int tiles[2] = {32, 64};
         double tm[kStCount];
-        for (int ci = 0; ci < 3; ++ci) {
-            for (int pers = 0; pers < 2; ++pers) {
-                Tuning t = best;
-                t.stage1_records = records[ci];
-                t.persistent = pers;
-                if (int rc = measure(t, tm)) return rc;
-                if (tm[kStGridFft] < best_s1) {
-                    best_s1 = tm[kStGridFft];
-                    best.stage1_records = t.stage1_records;
-                    best.persistent = t.persistent;
-                }
+        best.persistent = 0;
+        for (int r : records) {
+            Tuning t = best;
+            t.stage1_records = r;
+            if (int rc = measure(t, tm)) return rc;
+            if (tm[kStGridFft] < best_s1) {
+                best_s1 = tm[kStGridFft];
+                best.stage1_records = r;
             }
         }
         for (int r : rows) {

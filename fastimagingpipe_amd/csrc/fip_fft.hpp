@@ -165,18 +165,67 @@ __device__ __forceinline__ void static_for(F&& f)
     static_for_impl(f, std::make_integer_sequence<int, N>{});
 }
 
+// Sums and differences whose operands may be known zeros (ZA, ZB): the
+// compiler keeps x + 0 for the sign of zero, so a pruned transform leaves
+// them out itself.
+template <bool ZA, bool ZB> __device__ __forceinline__ float2 cadd_z(float2 a, float2 b)
+{
+    if constexpr (ZB) return a;
+    else if constexpr (ZA) return b;
+    else return cadd(a, b);
+}
+template <bool ZA, bool ZB> __device__ __forceinline__ float2 csub_z(float2 a, float2 b)
+{
+    if constexpr (ZB) return a;
+    else if constexpr (ZA) return make_float2(-b.x, -b.y);
+    else return csub(a, b);
+}
+// Radix 4 with the inputs whose bit is set in MASK; the others are zeros.
+template <unsigned MASK>
+__device__ __forceinline__ void bfly4_masked(float2* v)
+{
+    constexpr bool z0 = !(MASK & 1u), z1 = !(MASK & 2u), z2 = !(MASK & 4u), z3 = !(MASK & 8u);
+    const float2 a = cadd_z<z0, z2>(v[0], v[2]), b = csub_z<z0, z2>(v[0], v[2]);
+    const float2 c = cadd_z<z1, z3>(v[1], v[3]), d = cmul_i(csub_z<z1, z3>(v[1], v[3]));
+    constexpr bool za = z0 && z2, zc = z1 && z3;
+    v[0] = cadd_z<za, zc>(a, c);
+    v[2] = csub_z<za, zc>(a, c);
+    v[1] = cadd_z<za, zc>(b, d);
+    v[3] = csub_z<za, zc>(b, d);
+}
+
+// Inputs 0..LO-1 and R-HI..R-1 of a radix-R butterfly, as a bit mask (every
+// bit where that is all of them).
+template <int R, int LO, int HI>
+constexpr unsigned band_mask()
+{
+    if (LO + HI >= R) return 0xffffffffu;
+    const unsigned all = R >= 32 ? 0xffffffffu : ((1u << R) - 1u);
+    return (((1u << LO) - 1u) | ~((1u << (R - HI)) - 1u)) & all;
+}
+
 // Composite radix R = A * B in registers (Cooley-Tukey): input r = B r1 + r2,
 // output s = s1 + A s2; A-point DFTs over r1, rotation by
-// exp(+2 pi i r2 s1 / R), then B-point DFTs over r2.
+// exp(+2 pi i r2 s1 / R), then B-point DFTs over r2.  With A = 4, inputs
+// whose bit is clear in MASK are taken as zeros and not read.
 template <int A, int B>
 struct BflyAB {
+    template <unsigned MASK = 0xffffffffu>
     static __device__ __forceinline__ void run(float2* v)
     {
         constexpr int R = A * B;
         float2 x[B][A];
         static_for<B>([&](auto r2) {
             static_for<A>([&](auto r1) { x[r2][r1] = v[B * r1 + r2]; });
-            Bfly<A>::run(x[r2]);
+            static_assert(A == 4 || MASK == 0xffffffffu, "pruned inputs need 4-point DFTs first");
+            if constexpr (A == 4 && MASK != 0xffffffffu) {
+                constexpr int q = decltype(r2)::value;
+                constexpr unsigned m = ((MASK >> q) & 1u) | (((MASK >> (B + q)) & 1u) << 1) |
+                                       (((MASK >> (2 * B + q)) & 1u) << 2) | (((MASK >> (3 * B + q)) & 1u) << 3);
+                bfly4_masked<m>(x[r2]);
+            } else {
+                Bfly<A>::run(x[r2]);
+            }
             static_for<A>([&](auto s1) { x[r2][s1] = rot<R, decltype(r2)::value * decltype(s1)::value>(x[r2][s1]); });
         });
         static_for<A>([&](auto s1) {
@@ -191,6 +240,20 @@ template <> struct Bfly<6> : BflyAB<2, 3> {};
 template <> struct Bfly<12> : BflyAB<4, 3> {};
 template <> struct Bfly<16> : BflyAB<4, 4> {};
 template <> struct Bfly<24> : BflyAB<8, 3> {};
+template <> struct Bfly<32> : BflyAB<4, 8> {};
+
+// Butterfly of radix R with zero inputs outside MASK, where the radix has a
+// pruned form (4-point DFTs first); the others read every input.
+constexpr bool bfly_prunes(int R) { return R == 12 || R == 16 || R == 32; }
+template <int R, unsigned MASK>
+__device__ __forceinline__ void bfly_masked(float2* v)
+{
+    static_assert(bfly_prunes(R) || MASK == 0xffffffffu, "no pruned form of this radix");
+    if constexpr (bfly_prunes(R))
+        Bfly<R>::template run<MASK>(v);
+    else
+        Bfly<R>::run(v);
+}
 
 // ----------------------------------------------------------------- FFT plans
 // Radix lists for N = 3 * 2^k.  The host twiddle generator walks the same
@@ -199,9 +262,13 @@ template <> struct Bfly<24> : BflyAB<8, 3> {};
 // waves per workgroup hide the LDS and barrier latency of each stage.  Each
 // stage is one LDS round trip and two barriers, so these lengths take the
 // fewest stages that keep a butterfly's registers within occupancy: radix 16
-// and 12 in registers (three stages for 768 to 3072, four for 6144 and
-// 12288) measured 3-13% faster than radix 8/4/3/2 lists of five or six
-// stages.
+// and 12 in registers (three stages for 384 to 6144, four for 12288) measured
+// 3-13% faster than radix 8/4/3/2 lists of five or six stages, and 6144 as
+// 32, 16, 12 took the column kernel from 99 to 83 us at 4096^2 against
+// 16, 16, 2, 12 (one LDS round trip less; the radix-32 stage fills three of
+// the eight waves, which the CU's other workgroups cover).  Every list ends in radix 12: the last stage's outputs then lie
+// N/12 apart, so a crop to the central two thirds is four whole outputs
+// dropped per butterfly, and the kept ones leave from registers.
 template <int NT, int... Rs>
 struct PlanDef {
     static constexpr int nt = NT;
@@ -213,15 +280,15 @@ template <int N> struct FftPlan;
     template <> struct FftPlan<N_> : PlanDef<NT_, __VA_ARGS__> { \
         static constexpr int n = N_;                           \
     }
-FIP_PLAN(48, 64, 8, 2, 3);
-FIP_PLAN(96, 64, 8, 4, 3);
-FIP_PLAN(192, 64, 8, 8, 3);
-FIP_PLAN(384, 64, 8, 8, 2, 3);
-FIP_PLAN(768, 64, 16, 12, 4);
+FIP_PLAN(48, 64, 4, 12);
+FIP_PLAN(96, 64, 8, 12);
+FIP_PLAN(192, 64, 16, 12);
+FIP_PLAN(384, 64, 8, 4, 12);
+FIP_PLAN(768, 64, 16, 4, 12);
 FIP_PLAN(1536, 128, 16, 8, 12);
 FIP_PLAN(3072, 256, 16, 16, 12);
-FIP_PLAN(6144, 512, 16, 16, 12, 2);
-FIP_PLAN(12288, 1024, 16, 16, 12, 4);
+FIP_PLAN(6144, 512, 32, 16, 12);
+FIP_PLAN(12288, 1024, 16, 16, 4, 12);
 #undef FIP_PLAN
 
 // Padded LDS offsets of the R elements of a butterfly relative to the padded
@@ -245,82 +312,120 @@ template <int Ns, int R> struct StoreOff {
 
 // One Stockham stage of radix R with Ns = product of earlier radices.
 // tw points at this stage's twiddles laid out [r-1][k], k < Ns.  Threads
-// t >= NT of a larger workgroup take no butterfly but reach both barriers.
-template <int N, int NT, int R, int Ns>
-__device__ __forceinline__ void fft_stage(float2* __restrict__ buf, const float2* __restrict__ tw, int t)
+// t >= NT of a larger workgroup (whole waves, NT a multiple of 64) take no
+// butterfly but reach the barriers.
+//
+// The first stage's inputs come from load(j, v): v[r] = x[j + r N/R], and the
+// last stage's outputs go to store(j, v): X[j + r N/R] = v[r] (there Ns = N/R,
+// so j is the output index's low part); every other exchange goes through buf.
+// LoadLds / StoreLds say whether load reads or store writes LDS that this
+// transform (or its caller's data in the same memory) uses, which needs a
+// barrier between the reads and the writes.  MASK: the first stage's inputs
+// that can be non-zero (load need not set the others).
+template <class P, int S, int Ns, int TwOff, bool LoadLds, bool StoreLds, unsigned MASK, class Load, class Store>
+__device__ __forceinline__ void fft_stage(float2* __restrict__ buf, const float2* __restrict__ tw, int t,
+                                          const Load& load, const Store& store)
 {
+    constexpr int N = P::n, NT = P::nt, R = P::radix[S];
+    constexpr bool first = S == 0, last = S + 1 == P::nstages;
     constexpr int NB = N / R;                    // butterflies in this stage
     constexpr int BPT = (NB + NT - 1) / NT;      // butterflies per thread
-    constexpr bool exact = (NB % NT) == 0;
-    const bool act = t < NT;
-    float2 v[BPT][R];
-    // Twiddles do not depend on the data: issue their (L1/L2-resident) loads
-    // before the LDS loads and the barrier so their latency is hidden.
-    float2 w[BPT][R > 1 ? R - 1 : 1];
-    if (Ns > 1) {
+    // The two barriers around the exchange of in-place data.
+    constexpr bool mid = (!first || LoadLds) && (!last || StoreLds), end = !last || StoreLds;
+    auto body = [&](auto ALL) {
+        constexpr bool all = decltype(ALL)::value;   // every thread here has all its butterflies
+        float2 v[BPT][R];
+        // Twiddles do not depend on the data: issue their (L1/L2-resident)
+        // loads before the LDS loads and the barrier so their latency is
+        // hidden.
+        float2 w[BPT][R > 1 ? R - 1 : 1];
+        if (Ns > 1) {
+#pragma unroll
+            for (int b = 0; b < BPT; ++b) {
+                const int j = t + b * NT;
+                const int k = (all || j < NB) ? j % Ns : 0;
+#pragma unroll
+                for (int r = 1; r < R; ++r) w[b][r - 1] = (tw + TwOff)[(r - 1) * Ns + k];
+            }
+        }
 #pragma unroll
         for (int b = 0; b < BPT; ++b) {
             const int j = t + b * NT;
-            const int k = (exact || j < NB) ? j % Ns : 0;
+            if (all || (t < NT && j < NB)) {
+                if constexpr (first) {
+                    load(j, v[b]);
+                } else if constexpr (LoadOff<NB>::ok) {
+                    const float2* p = buf + lds_pad(j);
 #pragma unroll
-            for (int r = 1; r < R; ++r) w[b][r - 1] = tw[(r - 1) * Ns + k];
-        }
-    }
+                    for (int r = 0; r < R; ++r) v[b][r] = p[LoadOff<NB>::at(r)];
+                } else {
 #pragma unroll
-    for (int b = 0; b < BPT; ++b) {
-        const int j = t + b * NT;
-        if (act && (exact || j < NB)) {
-            if constexpr (LoadOff<NB>::ok) {
-                const float2* p = buf + lds_pad(j);
-#pragma unroll
-                for (int r = 0; r < R; ++r) v[b][r] = p[LoadOff<NB>::at(r)];
-            } else {
-#pragma unroll
-                for (int r = 0; r < R; ++r) v[b][r] = buf[lds_pad(j + r * NB)];
+                    for (int r = 0; r < R; ++r) v[b][r] = buf[lds_pad(j + r * NB)];
+                }
             }
         }
-    }
-    __syncthreads();
+        if constexpr (mid) __syncthreads();
 #pragma unroll
-    for (int b = 0; b < BPT; ++b) {
-        const int j = t + b * NT;
-        if (act && (exact || j < NB)) {
-            const int k = j % Ns;
-            if (Ns > 1) {
+        for (int b = 0; b < BPT; ++b) {
+            const int j = t + b * NT;
+            if (all || (t < NT && j < NB)) {
+                const int k = j % Ns;
+                if (Ns > 1) {
 #pragma unroll
-                for (int r = 1; r < R; ++r) v[b][r] = cmul(v[b][r], w[b][r - 1]);
-            }
-            Bfly<R>::run(v[b]);
-            const int base = (j / Ns) * Ns * R + k;
-            if constexpr (StoreOff<Ns, R>::ok) {
-                float2* p = buf + lds_pad(base);
+                    for (int r = 1; r < R; ++r) v[b][r] = cmul(v[b][r], w[b][r - 1]);
+                }
+                bfly_masked<R, first ? MASK : 0xffffffffu>(v[b]);
+                if constexpr (last) {
+                    store(j, v[b]);
+                } else {
+                    const int base = (j / Ns) * Ns * R + k;
+                    if constexpr (StoreOff<Ns, R>::ok) {
+                        float2* p = buf + lds_pad(base);
 #pragma unroll
-                for (int r = 0; r < R; ++r) p[StoreOff<Ns, R>::at(r)] = v[b][r];
-            } else {
+                        for (int r = 0; r < R; ++r) p[StoreOff<Ns, R>::at(r)] = v[b][r];
+                    } else {
 #pragma unroll
-                for (int r = 0; r < R; ++r) buf[lds_pad(base + r * Ns)] = v[b][r];
+                        for (int r = 0; r < R; ++r) buf[lds_pad(base + r * Ns)] = v[b][r];
+                    }
+                }
             }
         }
+        if constexpr (end) __syncthreads();
+    };
+    // Where the butterflies fill whole waves, the waves without one only take
+    // the barriers (a wave-uniform branch: every wave of the workgroup reaches
+    // each barrier once), so no register is merged across the branch.
+    constexpr bool exact = (NB % NT) == 0;
+    if constexpr (exact) {
+        if (__builtin_amdgcn_readfirstlane(t) < NT) {
+            body(std::true_type{});
+        } else {
+            if constexpr (mid) __syncthreads();
+            if constexpr (end) __syncthreads();
+        }
+    } else if constexpr (BPT == 1 && NB % 64 == 0) {
+        if (__builtin_amdgcn_readfirstlane(t) < NB) {
+            body(std::true_type{});
+        } else {
+            if constexpr (mid) __syncthreads();
+            if constexpr (end) __syncthreads();
+        }
+    } else {
+        body(std::false_type{});
     }
-    __syncthreads();
+    if constexpr (!last)
+        fft_stage<P, S + 1, Ns * R, TwOff + (Ns > 1 ? (R - 1) * Ns : 0), LoadLds, StoreLds, MASK>(buf, tw, t, load,
+                                                                                                  store);
 }
 
-template <class P, int S, int Ns, int TwOff, bool Done = (S >= P::nstages)>
-struct FftRun {
-    static __device__ __forceinline__ void run(float2* buf, const float2* tw, int t)
-    {
-        constexpr int R = P::radix[S];
-        fft_stage<P::n, P::nt, R, Ns>(buf, tw + TwOff, t);
-        constexpr int next_off = TwOff + (Ns > 1 ? (R - 1) * Ns : 0);
-        FftRun<P, S + 1, Ns * R, next_off>::run(buf, tw, t);
-    }
-};
-
-// Terminates the stage recursion once all radices are consumed.
-template <class P, int S, int Ns, int TwOff>
-struct FftRun<P, S, Ns, TwOff, true> {
-    static __device__ __forceinline__ void run(float2*, const float2*, int) {}
-};
+// Inverse FFT of length N between load and store (see fft_stage) with buf
+// (lds_len(N) entries) for the exchanges.
+template <int N, bool LoadLds, bool StoreLds, unsigned MASK = 0xffffffffu, class Load, class Store>
+__device__ __forceinline__ void fft_inverse_io(float2* buf, const float2* __restrict__ tw, int t, const Load& load,
+                                               const Store& store)
+{
+    fft_stage<FftPlan<N>, 0, 1, 0, LoadLds, StoreLds, MASK>(buf, tw, t, load, store);
+}
 
 // Inverse FFT of the N-point padded LDS array buf.  Caller must have a
 // workgroup barrier between filling buf and this call; on return the result
@@ -328,7 +433,18 @@ struct FftRun<P, S, Ns, TwOff, true> {
 template <int N>
 __device__ __forceinline__ void fft_inverse(float2* buf, const float2* __restrict__ tw, int t)
 {
-    FftRun<FftPlan<N>, 0, 1, 0>::run(buf, tw, t);
+    using P = FftPlan<N>;
+    constexpr int R0 = P::radix[0], R1 = P::radix[P::nstages - 1];
+    fft_inverse_io<N, true, true>(
+        buf, tw, t,
+        [&](int j, float2* v) {
+#pragma unroll
+            for (int r = 0; r < R0; ++r) v[r] = buf[lds_pad(j + r * (N / R0))];
+        },
+        [&](int j, const float2* v) {
+#pragma unroll
+            for (int r = 0; r < R1; ++r) buf[lds_pad(j + r * (N / R1))] = v[r];
+        });
 }
 
 // Number of twiddle entries the plan of length N uses (N - 1).

@@ -108,7 +108,7 @@ struct WorkView {
     float2* kt;        // [S][I/kKTile][M+1][kKTile]
     float* pre;        // [S][I][I] corrected image before re-projection
     float* img;        // [S][I][I] re-projected images
-    unsigned* work;    // [1] persistent-kernel work counter
+    unsigned* work;    // [1] cleared with the counters
     unsigned* pmax;    // [pmax_words(S)] spread slots of the image maxima
     size_t stride;
 };
@@ -118,7 +118,7 @@ struct Tuning {
     int stage1_records;   // gridding records per thread held in registers (2, 4, 8)
     int stage2_rows;    // image rows per stage-2 workgroup (1, 2, 4)
     int splat_tile;     // target tile edge of the splat (32 or 64)
-    int persistent;     // stage 1 as a persistent work-queue kernel
+    int persistent;     // accepted and kept; the column kernel has one launch form
 };
 
 // Stage ids for timing.

@@ -461,39 +461,41 @@ __global__ __launch_bounds__(256) void k_scatter(const VisRec* __restrict__ rec,
 
 // ---------------------------------------------------------------- stage 1
 
-// One visibility record prepared for a column: the column weight
-// ES((col - p2)/4)/2 (the Hermitian fold's 1/2) and the scale are folded
-// into its value; the row taps are applied per LDS band.
+// One visibility record prepared for a column.  The column weight
+// ES((col - p2)/4)/2 (the Hermitian fold's 1/2) is folded into its value.
+// Rows are counted from -g/2 (u = row + g/2); taps in ascending u: the first
+// row u0 and the tap distances X_j = j - 3 - f, j = 0..7 (and j = 8 where the
+// position is an integer: f = 1).  A mirrored record contributes conj(v) at
+// row -r, whose taps are those of the position -p1: f = 1 - frac.  A record
+// whose taps reach the grid's edge is marked (edge): its taps are clipped and
+// a mirrored tap at -g/2 stays there, so each one is placed by itself.
 struct ColRec {
-    int b1;
-    float f1, vr, vi;
-    bool mirror, live;
+    int b1, u0;
+    float f, vr, vi;
+    int nine;
+    bool mirror, edge, live;
 };
 
 // Taps follow FIPkernels.cu:213-243: r in [ceil(p-4), floor(p+4)] clipped to
-// [-g/2, g/2-1].  A mirrored record contributes conj(v) at row -r.
-__device__ __forceinline__ ColRec prep_rec(const VisRec& r, int col, bool mirror, int M, float fscale)
+// [-g/2, g/2-1].
+__device__ __forceinline__ ColRec prep_rec(const VisRec& r, int col, bool mirror, int M)
 {
     ColRec c;
     c.b1 = r.b1;
-    c.f1 = r.f1;
     c.mirror = mirror;
+    const bool frac = r.f1 > 0.0f;
+    c.nine = frac ? 0 : 1;
+    c.f = frac ? (mirror ? 1.0f - r.f1 : r.f1) : 1.0f;
+    const int lo1 = r.b1 - 4 + (frac ? 1 : 0), hi1 = r.b1 + 4;
+    c.u0 = M + (mirror ? -hi1 : lo1);
+    c.edge = lo1 <= -M || hi1 >= M;
     const int lo2 = max(r.b2 - 4 + (r.f2 > 0.0f ? 1 : 0), -M);
     const int hi2 = min(r.b2 + 4, M - 1);
-    c.live = (col >= lo2 && col <= hi2);
-    const float w2 = c.live ? es_f(((float)(col - r.b2) - r.f2) * 0.25f) * 0.5f * fscale : 0.0f;
+    c.live = col >= lo2 && col <= hi2 && lo1 < M && hi1 >= -M;
+    const float w2 = c.live ? es_f(((float)(col - r.b2) - r.f2) * 0.25f) * 0.5f : 0.0f;
     c.vr = r.vr * w2;
     c.vi = (mirror ? -r.vi : r.vi) * w2;
     return c;
-}
-
-// Grid rows are grouped in at most kScaleBlocks blocks of at least 16 rows
-// (by the index r mod G of row r); each block has its own power-of-two scale.
-constexpr int kScaleBlocks = 96;
-
-__device__ __forceinline__ int tap_row(const ColRec& c, int t1, int M)
-{
-    return c.mirror ? ((t1 == -M) ? -M : -t1) : t1;
 }
 
 // floor(x) and floor(x + 0.5) as int32 in one instruction each (the compiler
@@ -511,53 +513,89 @@ __device__ __forceinline__ int cvt_round_half_up_i32(float x)
     return r;
 }
 
-// ES inside its support, |x| <= 1 (as es_f without the range test).
-__device__ __forceinline__ float es_in(float x)
+// ES of a tap distance X in cells, |X| <= 4 (as es_f without the range test):
+// 2^(C sqrt(1 - X^2/16) - C) with the 1/16 moved into the constants (powers
+// of two, so the same roundings).
+__device__ __forceinline__ float es_tap(float X)
 {
     constexpr float C = (float)(kBeta * 1.4426950408889634);
-    return __builtin_amdgcn_exp2f(fmaf(C, __builtin_amdgcn_sqrtf(fmaf(-x, x, 1.0f)), -C));
+    return __builtin_amdgcn_exp2f(fmaf(0.25f * C, __builtin_amdgcn_sqrtf(fmaf(-X, X, 16.0f)), -C));
 }
 
+// Shape of the column kernel.  Rows are grouped in blocks of RBS rows, each
+// with its own power-of-two scale: at least 16 rows, so that the nine taps of
+// a record reach at most two blocks, and at most 96 blocks.
+//
+// NC copies of the int32 column spread the taps that several lanes of a wave
+// put on one row (the uv coverage is dense at the centre: a fifth of a hot
+// column's records share one cell at 256^2) over NC addresses; the sums are
+// integers, so adding the copies up is exact.  As many copies as keep the
+// column under 25 KB.
+//
+// NX threads are launched and the FFT takes the first NT.  A column with more
+// than two records per FFT thread is gridded by as many waves as give each
+// thread two (the uv coverage is concentrated: at 2048^2 with 32640
+// visibilities the median column holds 118 records and the fullest 4152, and
+// with 256 threads that one workgroup ran 33 us, the whole launch); the other
+// waves end at once and free their slots.  Where the FFT itself takes 512
+// threads or more the launch has workgroups enough to hide the full columns,
+// and waves that only end would halve the workgroups per CU.
+template <int G>
+struct ColShape {
+    static constexpr int M = G / 2, I = 2 * G / 3, h = I / 2;
+    static constexpr int NT = FftPlan<G>::nt;
+    static constexpr int NX = G <= 96 ? 512 : (G <= 1536 ? 1024 : (NT < 512 ? 512 : NT));
+    static constexpr int RBS = (G / 96 > 16) ? G / 96 : 16;
+    static constexpr int NBLK = G / RBS;
+    static constexpr int NC = G <= 384 ? 8 : (G <= 768 ? 4 : (G <= 1536 ? 2 : 1));
+    static constexpr int MC = 16;   // copies of a block's mass
+    // Waves per SIMD the registers must leave room for: what the LDS allows
+    // (three workgroups per CU at g = 6144, one at 12288).
+    static constexpr int waves = G >= 12288 ? 4 : (G >= 6144 ? 6 : 2);
+    static constexpr int acc_bytes = 2 * G * NC * (int)sizeof(int);
+    static constexpr int fft_bytes = lds_len(G) * (int)sizeof(float2);
+    static constexpr int bytes = acc_bytes > fft_bytes ? acc_bytes : fft_bytes;
+    static constexpr int mass_bytes = NBLK * MC * (int)sizeof(unsigned long long);
+    static_assert(G % RBS == 0 && M % RBS == 0 && NBLK <= 96, "scale blocks");
+    static_assert(mass_bytes <= acc_bytes && acc_bytes % 16 == 0 && mass_bytes % 16 == 0, "mass inside the column");
+    static_assert(NT <= NX && NBLK <= NT * 2, "one round of block scales");
+};
+
 // Row taps of one prepared record, accumulated as integers into the LDS
-// column (re, im interleaved; row r at padded index of r mod G), each scaled
-// by its block's power of two.  A mirrored record adds at row -t1 (mod G,
-// which also maps the edge tap t1 = -g/2 onto itself).  The tap offsets
-// (t1 - p1)/4 step by 1/4 from the first tap; each contribution is rounded
-// half up to an integer.  rbs is a power of two.
-__device__ __forceinline__ void grid_taps(const ColRec& c, int M, int G, int rbs, const float* sc, int* col)
+// column (re [0, G), im [G, 2G), each row NC copies; this lane's copy), each
+// scaled by its block's power of two and rounded half up.  Away from the
+// grid's edge a record's rows are one run u0..u0+7 (u0+8), so every tap is
+// one LDS address plus a constant.  It reaches at most two scale blocks, both
+// read once: taps from row `cross` on take the second.
+template <int G>
+__device__ __forceinline__ void grid_taps(const ColRec& c, const float* sc, int* col)
 {
-    const int lo1 = max(c.b1 - 4 + (c.f1 > 0.0f ? 1 : 0), -M);
-    const int hi1 = min(c.b1 + 4, M - 1);
-    float x = ((float)(lo1 - c.b1) - c.f1) * 0.25f;
-    const int sgn = c.mirror ? -1 : 1;
-    int row = sgn * lo1;   // the tap row sgn * t1, stepped with t1
-    // The taps' rows are one contiguous run of r mod G, so they reach at most
-    // two scale blocks: the first tap's and the last tap's.  Both scales are
-    // read once; each tap selects its own, so no tap waits on an LDS read
-    // (which would also wait for the previous taps' atomics).
-    const int ra = row, rz = sgn * hi1;
-    const unsigned ba = (unsigned)(ra < 0 ? ra + G : ra) / (unsigned)rbs;
-    const unsigned bz = (unsigned)(rz < 0 ? rz + G : rz) / (unsigned)rbs;
-    const float sca = sc[ba], scz = sc[bz];
-    auto tap = [&]() {
-        const int idx = row < 0 ? row + G : row;
-        const int q = 2 * lds_pad(idx);
-        const float wk = es_in(x) * ((unsigned)idx / (unsigned)rbs == ba ? sca : scz);
-        atomicAdd(&col[q], cvt_round_half_up_i32(c.vr * wk));
-        atomicAdd(&col[q + 1], cvt_round_half_up_i32(c.vi * wk));
-        x += 0.25f;
-        row += sgn;
-    };
-    // 8 taps (9 where the position is an integer), fewer only at the grid's
-    // edge: the first eight need no bound test (3% faster at 4096^2, 7% at
-    // 2048^2 with the ES form above, than one test per tap).
-    const int n = hi1 - lo1 + 1;
-    if (n >= 8) {
+    using Sh = ColShape<G>;
+    constexpr int NC = Sh::NC, M = Sh::M;
+    const int cp = NC > 1 ? (int)(threadIdx.x & (NC - 1)) : 0;
+    if (!c.edge) {
+        const unsigned ba = (unsigned)c.u0 / (unsigned)Sh::RBS, bz = (unsigned)(c.u0 + 8) / (unsigned)Sh::RBS;
+        const float sca = sc[ba], scz = sc[min(bz, (unsigned)Sh::NBLK - 1)];
+        const int cross = (int)((ba + 1) * (unsigned)Sh::RBS) - c.u0;
+        int* p = col + c.u0 * NC + cp;
+        auto tap = [&](int j) {
+            const float X = (float)(j - 3) - c.f;
+            const float wk = es_tap(X) * (j < cross ? sca : scz);
+            atomicAdd(p + j * NC, cvt_round_half_up_i32(c.vr * wk));
+            atomicAdd(p + (G + j) * NC, cvt_round_half_up_i32(c.vi * wk));
+        };
 #pragma unroll
-        for (int j = 0; j < 8; ++j) tap();
-        if (n == 9) tap();
-    } else {
-        for (int j = 0; j < n; ++j) tap();
+        for (int j = 0; j < 8; ++j) tap(j);
+        if (c.nine) tap(8);
+        return;
+    }
+    for (int j = 0; j < 8 + c.nine; ++j) {
+        const int t1 = c.mirror ? c.b1 + 4 - j : c.b1 - 3 - c.nine + j;   // the record's own row
+        if (t1 < -M || t1 > M - 1) continue;
+        const int u = (c.mirror ? (t1 == -M ? -M : -t1) : t1) + M;
+        const float wk = es_tap((float)(j - 3) - c.f) * sc[u / Sh::RBS];
+        atomicAdd(col + u * NC + cp, cvt_round_half_up_i32(c.vr * wk));
+        atomicAdd(col + (G + u) * NC + cp, cvt_round_half_up_i32(c.vi * wk));
     }
 }
 
@@ -565,17 +603,32 @@ __device__ __forceinline__ void grid_taps(const ColRec& c, int M, int G, int rbs
 // mass of every scale block its taps touch (at most two).  The mass is 64-bit:
 // a column holds up to two records per visibility (its direct and mirrored
 // buckets), so a 32-bit sum of up to 4096 units per record would wrap after
-// about 2^19 visibilities at one uv point.
-__device__ __forceinline__ void tap_mass(const ColRec& c, int M, int G, int rbs, float qs, unsigned long long* mass)
+// about 2^19 visibilities at one uv point.  Each block's mass is kept in MC
+// copies, one per lane modulo MC: nearly all records of a full column lie in
+// the few blocks around row 0, where a single word per block would serialise
+// the wave.
+template <int G>
+__device__ __forceinline__ void tap_mass(const ColRec& c, float qs, unsigned long long* mass)
 {
-    const int lo1 = max(c.b1 - 4 + (c.f1 > 0.0f ? 1 : 0), -M);
-    const int hi1 = min(c.b1 + 4, M - 1);
-    if (lo1 > hi1) return;
+    using Sh = ColShape<G>;
     const unsigned long long q = (unsigned long long)ceilf(fmaxf(fabsf(c.vr), fabsf(c.vi)) * qs);
-    const int ra = tap_row(c, lo1, M), rb = tap_row(c, hi1, M);
-    const int ba = (ra < 0 ? ra + G : ra) / rbs, bb = (rb < 0 ? rb + G : rb) / rbs;
-    atomicAdd(&mass[ba], q);
-    if (bb != ba) atomicAdd(&mass[bb], q);
+    int ba, bz;
+    if (!c.edge) {
+        ba = c.u0 / Sh::RBS;
+        bz = (c.u0 + 7 + c.nine) / Sh::RBS;
+    } else {
+        const int lo1 = max(c.b1 - 3 - c.nine, -Sh::M), hi1 = min(c.b1 + 4, Sh::M - 1);
+        const int a = c.mirror ? (lo1 == -Sh::M ? -Sh::M : -lo1) : lo1;
+        ba = (a + Sh::M) / Sh::RBS;
+        bz = ((c.mirror ? (hi1 == -Sh::M ? -Sh::M : -hi1) : hi1) + Sh::M) / Sh::RBS;
+        // a clipped mirrored run that starts at -g/2 goes on at the other end
+        if (c.mirror && lo1 == -Sh::M && hi1 > lo1) {
+            const int bn = (-(lo1 + 1) + Sh::M) / Sh::RBS;
+            if (bn != bz) atomicAdd(&mass[bn * Sh::MC + (threadIdx.x & (Sh::MC - 1))], q);
+        }
+    }
+    atomicAdd(&mass[ba * Sh::MC + (threadIdx.x & (Sh::MC - 1))], q);
+    if (bz != ba) atomicAdd(&mass[bz * Sh::MC + (threadIdx.x & (Sh::MC - 1))], q);
 }
 
 // Record ranges of column c: direct buckets cc-4..cc+4 and mirrored buckets
@@ -594,25 +647,24 @@ __device__ __forceinline__ int4 column_ranges(const int* __restrict__ bst, int c
     return r;
 }
 
-// Threads of a stage-1 workgroup: the column FFT's own count, or 512 where
-// that count is below 256 (g <= 1536), so that a column with many records
-// still spreads its gridding over eight waves; the extra threads idle
-// through the FFT stages.  (A floor of 512 for g = 3072 measured slower.)
-template <int G>
-constexpr int stage1_threads()
-{
-    return FftPlan<G>::nt < 256 ? 512 : FftPlan<G>::nt;
-}
-
+// Grids column c of snapshot s into LDS, transforms it and stores its I
+// cropped rows.  Bound by VALU issue at 4096^2 (the FFT is two thirds of its
+// instructions) and by the fullest columns' passes up to 2048^2.  Rows
+// counted from -g/2, so that a record's taps are one address plus constants,
+// the transform reading the integers and storing the crop from registers, and
+// extra waves for full columns took it from 105.6 to 83 us (4096^2, 130816
+// visibilities), 35 to 25 us (2048^2, 32640), 562 to 473 us (8192^2, 523776)
+// and 12.2 to 8 us (256^2, 2016) for three snapshots.  smem: ColShape<G>::bytes of LDS, used in turn as the blocks'
+// masses, the int32 column and the FFT's exchange buffer.  KR records per
+// thread are held in registers at a time.
 template <int G, int KR>
 __device__ __forceinline__ void stage1_column(int s, int c, int4 rg, const VisRec* __restrict__ sorted,
-                                              const SnapMeta& m,
-                                              const float2* __restrict__ tw,
-                                              float2* __restrict__ kt, size_t stride, int I, float2* fb,
-                                              unsigned long long* mass, float* sc, float* isc)
+                                              const SnapMeta& m, const float2* __restrict__ tw,
+                                              float2* __restrict__ kt, size_t stride, unsigned char* smem, float* sc,
+                                              float* isc)
 {
-    constexpr int NT = stage1_threads<G>();
-    constexpr int M = G / 2;
+    using Sh = ColShape<G>;
+    constexpr int NT = Sh::NT, M = Sh::M, RBS = Sh::RBS, NC = Sh::NC;
     const int t = threadIdx.x;
 
     const VisRec* vs = sorted + (size_t)s * stride;
@@ -620,6 +672,9 @@ __device__ __forceinline__ void stage1_column(int s, int c, int4 rg, const VisRe
     const int cm = (c == 0) ? 0 : ((c == M) ? -M : -c);      // mirrored column
     const int d0 = rg.x, d1 = rg.y, m0 = rg.z, m1 = rg.w;
     const int nd = d1 - d0, ntot = nd + (m1 - m0);
+    // Threads that grid (whole waves; every condition on them is uniform).
+    const int na = min(max((ntot / KR + 63) & ~63, NT), Sh::NX);
+    if (t >= na) return;
 
     // Exact integer accumulation with one power-of-two scale per block of
     // rows.  Pass 1 adds, per block, an upper bound of the magnitudes of the
@@ -631,47 +686,61 @@ __device__ __forceinline__ void stage1_column(int s, int c, int4 rg, const VisRe
     const float maxv = __uint_as_float(m.maxv_bits);
     const float amax = fmaxf(0.5f * maxv, 1e-30f);   // |v| ES / 2 <= amax
     const float qs = 4096.0f / amax;
-    // At least 16 rows per block, so the 9 taps of a record reach at most two
-    // blocks (two ends of a contiguous run of r mod G); at most kScaleBlocks.
-    constexpr int RBS = (G / kScaleBlocks > 16) ? G / kScaleBlocks : 16;
-    static_assert(G % RBS == 0 && G / RBS <= kScaleBlocks, "scale blocks");
 
     // Direct records (buckets cc-4..cc+4) then mirrored ones (cm-4..cm+4) in
-    // one numbering; each thread holds KR of them in registers at a time.
+    // one numbering.  A column whose records do not fit the registers walks
+    // them in passes, the next pass's records loaded under this one's work.
+    const int step = KR * na;
+    VisRec rn[KR];
     ColRec cr[KR];
-    auto load = [&](int base) {
-        VisRec r[KR];
+    auto fetch = [&](int base) {
 #pragma unroll
         for (int k = 0; k < KR; ++k) {
-            const int n = base + k * NT + t;
-            if (n < ntot) r[k] = vs[n < nd ? d0 + n : m0 + (n - nd)];
+            const int n = base + k * na + t;
+            if (n < ntot) rn[k] = vs[n < nd ? d0 + n : m0 + (n - nd)];
         }
+    };
+    auto prep = [&](int base) {
 #pragma unroll
         for (int k = 0; k < KR; ++k) {
-            const int n = base + k * NT + t;
+            const int n = base + k * na + t;
             if (n < ntot)
-                cr[k] = prep_rec(r[k], n < nd ? cc : cm, n >= nd, M, 1.0f);
+                cr[k] = prep_rec(rn[k], n < nd ? cc : cm, n >= nd, M);
             else
                 cr[k].live = false;
         }
     };
-    const bool resident = ntot <= KR * NT;
-    if (resident) load(0);
-    int* col = reinterpret_cast<int*>(fb);
-    for (int i = t; i < G; i += NT) fb[lds_pad(i)] = make_float2(0.0f, 0.0f);   // integer zero too
-    for (int i = t; i < kScaleBlocks; i += NT) mass[i] = 0ull;
-    __syncthreads();
-    for (int base = 0; base < ntot; base += KR * NT) {
-        if (!resident) load(base);
-#pragma unroll
-        for (int k = 0; k < KR; ++k)
-            if (cr[k].live) tap_mass(cr[k], M, G, RBS, qs, mass);
+    const bool resident = ntot <= step;
+    fetch(0);
+    unsigned long long* mass = reinterpret_cast<unsigned long long*>(smem);
+    int* col = reinterpret_cast<int*>(smem);
+    {
+        int4* z = reinterpret_cast<int4*>(smem);
+        for (int i = t; i < Sh::acc_bytes / 16; i += na) z[i] = make_int4(0, 0, 0, 0);
     }
     __syncthreads();
-    for (int i = t; i < kScaleBlocks; i += NT) {
+    for (int base = 0; base < ntot; base += step) {
+        prep(base);
+        if (base + step < ntot) fetch(base + step);
+#pragma unroll
+        for (int k = 0; k < KR; ++k)
+            if (cr[k].live) tap_mass<G>(cr[k], qs, mass);
+    }
+    if (!resident) fetch(0);
+    __syncthreads();
+    for (int i = t; i < Sh::NBLK; i += na) {
+        // One thread per block adds the copies up (starting at its own bank)
+        // and leaves them zero for the column that shares their memory.
+        unsigned long long sum = 0ull;
+#pragma unroll
+        for (int k = 0; k < Sh::MC; ++k) {
+            unsigned long long* q = mass + i * Sh::MC + ((k + i) & (Sh::MC - 1));
+            sum += *q;
+            *q = 0ull;
+        }
         // bound = mass * amax / 4096 (+ one unit per record of rounding slack
         // is already inside the ceil); 2^e > bound.
-        const float bound = (float)mass[i] * (amax / 4096.0f) * 1.0001f;
+        const float bound = (float)sum * (amax / 4096.0f) * 1.0001f;
         int e = 0;
         frexpf(fmaxf(bound, 1e-30f), &e);
         const int k = min(29 - e, 120);   // empty blocks: any finite scale
@@ -679,53 +748,85 @@ __device__ __forceinline__ void stage1_column(int s, int c, int4 rg, const VisRe
         isc[i] = ldexpf(1.0f, -k);
     }
     __syncthreads();
-    for (int base = 0; base < ntot; base += KR * NT) {
-        if (!resident) load(base);
+    for (int base = 0; base < ntot; base += step) {
+        if (!resident) {
+            prep(base);
+            if (base + step < ntot) fetch(base + step);
+        }
 #pragma unroll
         for (int k = 0; k < KR; ++k)
-            if (cr[k].live) grid_taps(cr[k], M, G, RBS, sc, col);
+            if (cr[k].live) grid_taps<G>(cr[k], sc, col);
     }
     __syncthreads();
-    const int rlo = -m.r1max, rhi = min(m.r1max, M - 1);
-    for (int i = rlo + t; i <= rhi; i += NT) {
-        const int idx = i < 0 ? i + G : i;
-        const int q = lds_pad(idx);
-        const int re = col[2 * q], im = col[2 * q + 1];
-        const float k = isc[idx / RBS];
-        fb[q] = make_float2((float)re * k, (float)im * k);
+    if (t >= NT) return;
+    // Column FFT straight from the integer column: element n of the transform
+    // is grid row n (n < g/2) or n - g, i.e. u = (n + g/2) mod g, so a
+    // butterfly's inputs lie N/R apart here too.
+    //
+    // Crop y in [-h, h): outputs n < h are rows n, n >= g - h rows n - g, and
+    // with the last radix a multiple of 3 and h = g/3 those are whole
+    // outputs of each butterfly, stored from its registers.  The row
+    // correction 1/(c(|y|) norm) is a factor per image row, applied by the
+    // row pass (one load per row there instead of one per row and column
+    // here).
+    constexpr int R0 = FftPlan<G>::radix[0], NB0 = G / R0;
+    constexpr int R1 = FftPlan<G>::radix[FftPlan<G>::nstages - 1], NS1 = G / R1;
+    static_assert(R0 % 2 == 0 && R1 % 3 == 0 && NS1 % kKTile == 0 && Sh::h % kKTile == 0, "column plan");
+    float2* fb = reinterpret_cast<float2*>(smem);
+    float2* ks = kt + (size_t)s * ((size_t)Sh::I * (M + 1)) + (size_t)c * kKTile;
+    // NZ: inputs 0..NZ-1 and R0-NZ..R0-1 are read, rows |r| < NZ NB0.
+    auto transform = [&](auto NZ) {
+        constexpr int nz = decltype(NZ)::value;
+        constexpr unsigned mask = band_mask<R0, nz, nz>();
+        fft_inverse_io<G, true, false, mask>(
+            fb, tw, t,
+            [&](int j, float2* v) {
+#pragma unroll
+                for (int r = 0; r < R0; ++r) {
+                    if (!((mask >> r) & 1u)) continue;
+                    const int q0 = NB0 * ((r + R0 / 2) % R0), u = j + q0;
+                    int re = 0, im = 0;
+#pragma unroll
+                    for (int q = 0; q < NC; ++q) {
+                        re += col[u * NC + q];
+                        im += col[(G + u) * NC + q];
+                    }
+                    const float k = NB0 % RBS == 0 ? isc[j / RBS + q0 / RBS] : isc[u / RBS];
+                    v[r] = make_float2((float)re * k, (float)im * k);
+                }
+            },
+            [&](int j, const float2* v) {
+                float2* o = ks + (size_t)(j / kKTile) * (M + 1) * kKTile + (j % kKTile);
+#pragma unroll
+                for (int r = 0; r < R1; ++r) {
+                    if (r >= R1 / 3 && r < 2 * R1 / 3) continue;
+                    const int yp = r < R1 / 3 ? NS1 * r + Sh::h : NS1 * r - G + Sh::h;   // plus j
+                    o[(size_t)(yp / kKTile) * (M + 1) * kKTile] = v[r];
+                }
+            });
+    };
+    // Rows beyond +-r1max hold no tap.  A band within 9/32 of the grid on
+    // either side (baselines up to 0.28 of the sampling rate, the usual
+    // imaging; the widest uv coverage is 0.5) needs 9/16 of the first
+    // stage's inputs, and its butterflies drop the zeros.
+    constexpr int NZ = bfly_prunes(R0) ? (9 * R0 + 31) / 32 : R0 / 2;
+    if constexpr (NZ < R0 / 2) {
+        if (m.r1max < NZ * NB0) {
+            transform(std::integral_constant<int, NZ>{});
+            return;
+        }
     }
-    __syncthreads();
-    fft_inverse<G>(fb, tw, t);
-    // Crop y in [-h, h).  The row correction 1/(c(|y|) norm) is a factor per
-    // image row, applied by the row pass (one load per row there instead of
-    // one per row and column here).
-    const int h = I / 2;
-    float2* ks = kt + (size_t)s * ((size_t)I * (M + 1));
-    // Two consecutive rows per thread and one 16-byte store: with yp even the
-    // pair shares a K-tile run (kKTile is even) at a 16-byte offset, and its
-    // LDS slots are adjacent (an even index and the next one never straddle
-    // a padding slot; h and G are even, so y and its wrap keep the parity).
-    static_assert(kKTile % 2 == 0, "row pairs inside a K-tile run");
-#pragma unroll 2
-    for (int yp = 2 * t; yp < I; yp += 2 * NT) {
-        const int y = yp - h;
-        const int q = lds_pad(y < 0 ? y + G : y);
-        const float2 v0 = fb[q], v1 = fb[q + 1];
-        *reinterpret_cast<float4*>(ks + ((size_t)(yp / kKTile) * (M + 1) + c) * kKTile + (yp % kKTile)) =
-            make_float4(v0.x, v0.y, v1.x, v1.y);
-    }
+    transform(std::integral_constant<int, R0 / 2>{});
 }
 
 template <int G, int KR>
-__global__ __launch_bounds__(stage1_threads<G>(), (stage1_threads<G>() >= 1024 ? 1 : 2)) void k_stage1(const VisRec* __restrict__ sorted,
-                                                            const int* __restrict__ bstart,
-                                                            const SnapMeta* __restrict__ meta,
-                                                            const float2* __restrict__ tw,
-                                                            float2* __restrict__ kt, size_t stride, int I)
+__global__ __launch_bounds__(ColShape<G>::NX, ColShape<G>::waves) void k_stage1(
+    const VisRec* __restrict__ sorted, const int* __restrict__ bstart, const SnapMeta* __restrict__ meta,
+    const float2* __restrict__ tw, float2* __restrict__ kt, size_t stride)
 {
-    __shared__ float2 fb[lds_len(G)];
-    __shared__ unsigned long long mass[kScaleBlocks];
-    __shared__ float sc[kScaleBlocks], isc[kScaleBlocks];
+    using Sh = ColShape<G>;
+    __shared__ __align__(16) unsigned char smem[Sh::bytes];
+    __shared__ float sc[Sh::NBLK], isc[Sh::NBLK];
     // Column-major over snapshots: the heavily populated low columns of
     // every snapshot are dispatched first, so none of them ends the launch.
     const int S = (int)(gridDim.x / (G / 2 + 1));
@@ -736,36 +837,7 @@ __global__ __launch_bounds__(stage1_threads<G>(), (stage1_threads<G>() >= 1024 ?
     const int4 rg = column_ranges<G>(bstart + (size_t)s * (G + 1), c);
     const SnapMeta m = meta[s];
     if (c > m.rmax) return;
-    stage1_column<G, KR>(s, c, rg, sorted, m, tw, kt, stride, I, fb, mass, sc, isc);
-}
-
-// Persistent form: a fixed grid pulls (snapshot, column) items from a
-// counter until all S*(M+1) items are claimed; every workgroup exits.
-template <int G, int KR>
-__global__ __launch_bounds__(stage1_threads<G>()) void k_stage1_persistent(
-    const VisRec* __restrict__ sorted, const int* __restrict__ bstart, const SnapMeta* __restrict__ meta,
-    const float2* __restrict__ tw, float2* __restrict__ kt, size_t stride,
-    int I, int S, unsigned* work)
-{
-    __shared__ float2 fb[lds_len(G)];
-    __shared__ unsigned long long mass[kScaleBlocks];
-    __shared__ float sc[kScaleBlocks], isc[kScaleBlocks];
-    __shared__ unsigned item;
-    constexpr unsigned per = G / 2 + 1;
-    const unsigned total = (unsigned)S * per;
-    for (;;) {
-        if (threadIdx.x == 0) item = atomicAdd(work, 1u);
-        __syncthreads();
-        const unsigned it = item;
-        __syncthreads();
-        if (it >= total) break;
-        const int s = (int)(it % (unsigned)S), c = (int)(it / (unsigned)S);
-        const int4 rg = column_ranges<G>(bstart + (size_t)s * (G + 1), c);
-        const SnapMeta m = meta[s];
-        if (c > m.rmax) continue;
-        stage1_column<G, KR>(s, c, rg, sorted, m, tw, kt, stride, I, fb, mass, sc, isc);
-        __syncthreads();
-    }
+    stage1_column<G, KR>(s, c, rg, sorted, m, tw, kt, stride, smem, sc, isc);
 }
 
 // ---------------------------------------------------------------- stage 2
@@ -1835,21 +1907,10 @@ hipError_t launch_scatter(const WorkView& w, const PlanTables& p, int S, int nma
 }
 
 template <int G, int KR>
-static void stage1_dispatch(const WorkView& w, const PlanTables& p, int S, bool persistent, hipStream_t st)
+static void stage1_dispatch(const WorkView& w, const PlanTables& p, int S, hipStream_t st)
 {
-    constexpr int NT = stage1_threads<G>();
-    if (persistent) {
-        int dev = 0, ncu = 0, per_cu = 0;
-        (void)hipGetDevice(&dev);
-        (void)hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
-        (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_stage1_persistent<G, KR>, NT, 0);
-        const int nb = max(1, ncu * max(per_cu, 1));
-        hipLaunchKernelGGL((k_stage1_persistent<G, KR>), dim3(nb), dim3(NT), 0, st, w.sorted, w.bstart, w.meta,
-                           p.tw_g, w.kt, w.stride, p.I, S, w.work);
-    } else {
-        hipLaunchKernelGGL((k_stage1<G, KR>), dim3((G / 2 + 1) * S), dim3(NT), 0, st, w.sorted, w.bstart, w.meta,
-                           p.tw_g, w.kt, w.stride, p.I);
-    }
+    hipLaunchKernelGGL((k_stage1<G, KR>), dim3((G / 2 + 1) * S), dim3(ColShape<G>::NX), 0, st, w.sorted, w.bstart,
+                       w.meta, p.tw_g, w.kt, w.stride);
 }
 
 // Records per thread held in registers while a column is gridded.
@@ -1857,11 +1918,11 @@ template <int G>
 static void stage1_pick(const WorkView& w, const PlanTables& p, int S, const Tuning& tu, hipStream_t st)
 {
     if (tu.stage1_records >= 8)
-        stage1_dispatch<G, 8>(w, p, S, tu.persistent != 0, st);
+        stage1_dispatch<G, 8>(w, p, S, st);
     else if (tu.stage1_records <= 2)
-        stage1_dispatch<G, 2>(w, p, S, tu.persistent != 0, st);
+        stage1_dispatch<G, 2>(w, p, S, st);
     else
-        stage1_dispatch<G, 4>(w, p, S, tu.persistent != 0, st);
+        stage1_dispatch<G, 4>(w, p, S, st);
 }
 
 hipError_t launch_stage1(const WorkView& w, const PlanTables& p, int S, const Tuning& tu, hipStream_t st)

@@ -249,9 +249,10 @@ int fip_stage_times_reset(void);
 
 /* ---- launch tuning and autotuner ---------------------------------------- */
 /* Measure candidate launch configurations (gridding records per thread,
- * rows per C2R workgroup, splat tile, persistent gridding) on synthetic data
- * of the given shape, keep the fastest for that image size, and write it to
- * *choice (4 ints: records, rows, tile, persistent; may be NULL). */
+ * rows per C2R workgroup, splat tile) on synthetic data of the given shape,
+ * keep the fastest for that image size, and write it to *choice (4 ints:
+ * records, rows, tile, persistent; may be NULL).  persistent is kept for
+ * callers that set it; the gridding has one launch form. */
 int fip_autotune(size_t image_size, size_t num_baselines, float cell_size,
                  int reps, int *choice);
 /* Force a launch configuration for an image size (choice as above). */

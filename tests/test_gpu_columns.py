@@ -1,0 +1,68 @@
+"""The column kernel at the edges of its cases: the gridded band on either side
+of the pruned transform's limit, taps clipped at the grid's edge, integer
+positions, mirrored records, and (for its exactness) columns of more records
+than its threads hold.
+"""
+import numpy as np
+import pytest
+
+from tests.inputs import rel_rms, rotation
+
+pytestmark = pytest.mark.gpu
+
+
+def positions(kind, g, rng):
+    """Grid positions [n, 2] (row, column)."""
+    m = g // 2
+    if kind.startswith("band"):   # rows up to just inside / outside 9/32 of the grid
+        limit = (9 * g) // 32 + (-4 if kind == "band_in" else 3)
+        p = rng.uniform(-0.4, 0.4, (500, 2)) * g
+        p[:, 0] = np.clip(p[:, 0], 5 - limit, limit - 5)
+        p[:2, 0] = limit - 4.5, 4.5 - limit
+        return p
+    if kind == "edge":   # taps clipped, wrapped by the mirror, or wholly outside
+        e = np.array([-m - 5, -m - 3.7, -m - 0.2, -m, -m + 0.3, -m + 3, -m + 3.9, m - 4.1, m - 3, m - 0.5, m, m + 3.2])
+        p = np.stack(np.meshgrid(e, np.concatenate([e, rng.uniform(-m, m, 8)])), -1).reshape(-1, 2)
+        return np.concatenate([p, p[:, ::-1]])
+    if kind == "integer":   # nine taps per axis
+        return 3.0 * rng.integers(-m // 3, m // 3 + 1, (500, 2))
+    raise ValueError(kind)
+
+
+@pytest.mark.parametrize("image", [64, 128, 256, 512, 1024])
+@pytest.mark.parametrize("kind", ["band_in", "band_out", "edge", "integer"])
+def test_columns_match_oracle(fip, oracle, image, kind):
+    rng = np.random.default_rng(image + sum(map(ord, kind)))
+    g = fip.grid_size(image)
+    cell = 2.0 ** -14 * 64 / image   # cell * g = 3 * 2^-9: multiples of 3 are exact positions
+    p = positions(kind, g, rng)
+    n = p.shape[0]
+    B = (p / (cell * g)).astype(np.float32)
+    vr, vi = rng.standard_normal((2, n)).astype(np.float32)
+    V = rotation(0.1, 0.3, 0.2).astype(np.float32)
+    pre, _, _ = fip.image(vr, vi, B, V, n, image, 1, cell)
+    ref, _, _ = oracle.image(vr, vi, B, V, image, cell, want_pre=True)
+    err = rel_rms(pre[0], ref)
+    print(f"{kind} {image}: pre rel-rms {err:.2e}")
+    # The bound of the image test at these sizes, whose inputs have the same
+    # spread of magnitudes (5e-6, its measured 8.6e-7 times five).
+    assert err < 5e-6
+
+
+@pytest.mark.parametrize("image,n", [(64, 9000), (256, 9000), (1024, 9000), (2048, 9000)])
+def test_crowded_columns_do_not_depend_on_the_order(fip, image, n):
+    """Records near one axis, several passes of a column's threads: the sums
+    are integers, so any order of the visibilities gives the same bits."""
+    rng = np.random.default_rng(image)
+    g = fip.grid_size(image)
+    cell = 2.0 ** -14 * 64 / image
+    p = np.stack([rng.uniform(-0.45, 0.45, n) * g, rng.uniform(-6, 6, n)], -1)
+    p[::2, 0] = rng.normal(0, 3, n // 2)
+    B = (p / (cell * g)).astype(np.float32)
+    vr, vi = rng.standard_normal((2, n)).astype(np.float32)
+    V = rotation(0.1, 0.3, 0.2).astype(np.float32)
+    k = rng.permutation(n)
+    a = fip.image(vr, vi, B, V, n, image, 1, cell)[0]
+    b = fip.image(vr[k], vi[k], B[k], V, n, image, 1, cell)[0]
+    assert np.isfinite(a).all()
+    assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
