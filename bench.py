@@ -68,8 +68,9 @@ def rmax_of(B, cell, g):
 def stage_bytes(nbl, image, g, rmax, tile, nsnap=3, nwin=1, fused=False):
     """Algorithmic HBM bytes per launch of each stage: every input read once and
     every output written once, for the nsnap snapshots (nwin windows) one launch
-    processes.  Visibility records are 24 B (two bucket/offset pairs + complex
-    value), the column-transformed grid holds rmax+1 complex columns of I rows.
+    processes.  "bin" is the whole front end: inputs in, records in column order
+    out.  Visibility records are 24 B (two tap/offset pairs + complex value),
+    the column-transformed grid holds rmax+1 complex columns of I rows.
     fused: the last snapshot's splat carries the trigger (splat_trigger reads
     its corrected image and the window's first two images, and writes three
     terms per trigger tile; the trigger stage turns the terms into the tLISI)."""
@@ -77,10 +78,7 @@ def stage_bytes(nbl, image, g, rmax, tile, nsnap=3, nwin=1, fused=False):
     kcols = rmax + 1
     un2 = (I // tile) ** 2
     b = {
-        "reset": nsnap * (g * 4 + 64),
-        "bin": nsnap * nbl * (4 + 4 + 8 + 24 + 8),
-        "scan": nsnap * (g * 4 + (g + 1) * 4),
-        "scatter": nsnap * nbl * (8 + 24 + 24),
+        "bin": nsnap * (nbl * (4 + 4 + 8 + 24) + (g // 2 + 14) * 4),
         "grid_colfft": nsnap * (nbl * 24 + kcols * I * 8),
         "row_c2r": nsnap * (kcols * I * 8 + I * I * 4),
         "splat": nsnap * (I * I * 4 * 2),

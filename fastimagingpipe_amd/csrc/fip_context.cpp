@@ -78,23 +78,20 @@ void PinnedBuf::release()
 
 // ---------------------------------------------------------------- work
 
-// Bytes of each work buffer for S snapshots, in the order rec, bkslot,
-// sorted, hist, bstart, meta, geom, kt, pre, img, work, pmax.
+// Bytes of each work buffer for S snapshots, in the order rec, sorted,
+// bstart, meta, geom, kt, pre, img, pmax.
 void work_sizes(int S, size_t stride, const PlanTables& p, size_t out[kWorkBufs])
 {
     const size_t s = (size_t)S;
     const size_t nvis = s * stride;
     const size_t sizes[kWorkBufs] = {nvis * sizeof(VisRec),                          // rec
-                                     nvis * sizeof(int2),                            // bkslot
                                      nvis * sizeof(VisRec),                          // sorted
-                                     s * p.G * sizeof(int),                          // hist
-                                     s * (p.G + 1) * sizeof(int),                    // bstart
+                                     s * bstart_words(p.G) * sizeof(int),            // bstart
                                      s * sizeof(SnapMeta),                           // meta
                                      s * sizeof(SnapGeom),                           // geom
                                      s * (size_t)p.I * (p.M + 1) * sizeof(float2),   // kt
                                      s * (size_t)p.I * p.I * sizeof(float),          // pre
                                      s * (size_t)p.I * p.I * sizeof(float),          // img
-                                     256,                                            // work
                                      pmax_words(S) * sizeof(unsigned)};              // pmax
     std::copy(sizes, sizes + kWorkBufs, out);
 }
@@ -110,8 +107,7 @@ size_t Work::bytes(int S, size_t stride, const PlanTables& p) const
 
 int Work::ensure(int S, size_t stride, const PlanTables& p)
 {
-    DevBuf* const all[kWorkBufs] = {&rec, &bkslot, &sorted, &hist, &bstart, &meta,
-                                    &geom, &kt, &pre, &img, &work, &pmax};
+    DevBuf* const all[kWorkBufs] = {&rec, &sorted, &bstart, &meta, &geom, &kt, &pre, &img, &pmax};
     size_t want[kWorkBufs];
     work_sizes(S, stride, p, want);
     for (int i = 0; i < kWorkBufs; ++i) {
@@ -127,16 +123,13 @@ WorkView Work::view(size_t stride) const
 {
     WorkView v;
     v.rec = rec.as<VisRec>();
-    v.bkslot = bkslot.as<int2>();
     v.sorted = sorted.as<VisRec>();
-    v.hist = hist.as<int>();
     v.bstart = bstart.as<int>();
     v.meta = meta.as<SnapMeta>();
     v.geom = geom.as<SnapGeom>();
     v.kt = kt.as<float2>();
     v.pre = pre.as<float>();
     v.img = img.as<float>();
-    v.work = work.as<unsigned>();
     v.pmax = pmax.as<unsigned>();
     v.stride = stride;
     return v;
@@ -147,10 +140,8 @@ WorkView snapshot_view(const WorkView& w, int s, const PlanTables& p)
     const size_t S = (size_t)s;
     WorkView v = w;
     v.rec = w.rec + S * w.stride;
-    v.bkslot = w.bkslot + S * w.stride;
     v.sorted = w.sorted + S * w.stride;
-    v.hist = w.hist + S * p.G;
-    v.bstart = w.bstart + S * (p.G + 1);
+    v.bstart = w.bstart + S * bstart_words(p.G);
     v.meta = w.meta + S;
     v.geom = w.geom + S;
     v.kt = w.kt + S * (size_t)p.I * (p.M + 1);
@@ -162,7 +153,7 @@ WorkView snapshot_view(const WorkView& w, int s, const PlanTables& p)
 
 void Work::release()
 {
-    for (DevBuf* b : {&rec, &bkslot, &sorted, &hist, &bstart, &meta, &geom, &kt, &pre, &img, &work, &pmax})
+    for (DevBuf* b : {&rec, &sorted, &bstart, &meta, &geom, &kt, &pre, &img, &pmax})
         b->release();
     ++gen;
 }
@@ -347,10 +338,7 @@ int imaging_sequence(Context* C, const PlanTables& p, const WorkView& w, const I
 {
     // r1r2_scale = cell * g (FIPkernels.cu:584), kept in FP64.
     const double scale = (double)cell * (double)p.G;
-    FIP_STAGE(C, kStReset, st, launch_reset(in, w, p, S, cell, norm_dev, norm_const, st));
-    FIP_STAGE(C, kStBin, st, launch_bin(in, w, p, S, nmax, scale, st));
-    FIP_STAGE(C, kStScan, st, launch_scan(w, p, S, st));
-    FIP_STAGE(C, kStScatter, st, launch_scatter(w, p, S, nmax, st));
+    FIP_STAGE(C, kStBin, st, launch_bin(in, w, p, S, nmax, cell, scale, norm_dev, norm_const, st));
     FIP_STAGE(C, kStGridFft, st, launch_stage1(w, p, S, tu, st));
     FIP_STAGE(C, kStRowC2R, st, launch_stage2(w, p, S, tu, st));
     const int ns = S - ndefer;

@@ -57,14 +57,14 @@ void plan_host_tables(size_t image, PlanHostTables& t);
 // Launch parameters used until the autotuner or fip_set_tuning picks others.
 Tuning default_tuning(size_t image);
 
-// Work buffers in the order rec, bkslot, sorted, hist, bstart, meta, geom,
-// kt, pre, img, work, pmax: their byte sizes for S snapshots.
-constexpr int kWorkBufs = 12;
+// Work buffers in the order rec, sorted, bstart, meta, geom, kt, pre, img,
+// pmax: their byte sizes for S snapshots.
+constexpr int kWorkBufs = 9;
 void work_sizes(int S, size_t stride, const PlanTables& p, size_t out[kWorkBufs]);
 
 // Work buffers sized for S snapshots of one image size and stride.
 struct Work {
-    DevBuf rec, bkslot, sorted, hist, bstart, meta, geom, kt, pre, img, work, pmax;
+    DevBuf rec, sorted, bstart, meta, geom, kt, pre, img, pmax;
     // Bumped whenever any buffer is reallocated or released: a captured graph
     // that baked in the old addresses must not be replayed after that.
     unsigned long long gen = 0;
@@ -131,7 +131,7 @@ private:
 // The work buffers of snapshot s of `w` as a one-snapshot view.
 WorkView snapshot_view(const WorkView& w, int s, const PlanTables& p);
 
-// Enqueue reset..splat / the trigger on explicit tables and buffers; C (may
+// Enqueue bin..splat / the trigger on explicit tables and buffers; C (may
 // be null) only adds the profiling events.  The splats of the view's last
 // ndefer snapshots are left to the caller's fused trigger launches
 // (fused_trigger_sequence for FIpipe's third snapshot).
@@ -150,7 +150,7 @@ int fused_trigger_sequence(Context* C, const PlanTables& p, const WorkView& w, i
 int pipe_sequence(Context* C, const PlanTables& p, const WorkView& w, const InputView& in, int nmax, float cell,
                   const Tuning& tu, const int* win_dev, int tile, float* out_dev, hipStream_t st);
 
-// Enqueue reset..splat for S snapshots described by `in` into `w`.
+// Enqueue bin..splat for S snapshots described by `in` into `w`.
 int run_imaging(Context& C, const Plan& P, Work& W, const InputView& in, int S, int nmax, float cell,
                 const int* norm_dev, int norm_const, const Tuning& tu, hipStream_t st);
 // Enqueue the trigger over windows `win_dev` (3 ints each) into out_dev.

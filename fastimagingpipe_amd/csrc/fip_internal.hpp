@@ -18,17 +18,26 @@ constexpr int kSupport = 8;
 // divide it).
 constexpr int kKTile = 8;
 
-// One binned visibility: integer floor and FP32 fraction of each grid
-// coordinate (computed from an FP64 product B * cell * g), and the weighted
+// One binned visibility: per axis the first tap, whether it has nine taps
+// (an integer position) instead of eight, and the FP32 fraction of the
+// position (computed from an FP64 product B * cell * g; 1 where it is an
+// integer), so that tap j lies at the distance j - 3 - f; and the weighted
 // visibility.  24 bytes.
 struct VisRec {
-    int b1;
+    int row;    // first row tap << 2 | nine << 1 | (its taps reach the grid's edge)
     float f1;
-    int b2;
+    int col;    // first column tap << 1 | nine
     float f2;
     float vr;
     float vi;
 };
+
+// A snapshot's visibilities are sorted in at most kMaxSegs segments, one
+// workgroup each, then merged; per snapshot and segment the largest
+// |column tap|, |row tap| and weighted magnitude (float bits).
+constexpr int kMaxSegs = 64;
+// Words of one snapshot's key offsets.
+size_t bstart_words(int G);
 
 // Image maxima are gathered in spread slots: per snapshot, kMaxSlots slots
 // for the corrected image before re-projection (slot set 0) and kMaxSlots for
@@ -47,14 +56,13 @@ size_t pmax_index(int s, int set, int slot);    // word of one slot
 
 // Per-snapshot scalars produced and consumed on the device.
 struct SnapMeta {
-    int ngrid;            // visibilities with at least one grid tap
     int rmax;             // largest |column tap|: stage 1 covers c = 0..rmax
     int r1max;            // largest |row tap|: rows of the gridded band
     unsigned maxv_bits;   // max(|re|,|im|) of weighted visibilities (float bits)
     unsigned maxp_bits;   // max of the corrected image before re-projection (k_max_finalize)
     unsigned maxd_bits;   // max of the re-projected image, maxall entry (k_trigger, k_max_finalize)
     int norm_n;           // N used by the splat's 1/N (num_baselines)
-    int nvis;             // visibilities present in this snapshot
+    int pad[2];
 };
 
 // Per-snapshot re-projection geometry (FP64, from the V matrix).
@@ -98,19 +106,28 @@ struct PlanTables {
 
 // Work buffers for a batch of up to S snapshots of one shape.
 struct WorkView {
-    VisRec* rec;       // [S*stride]
-    int2* bkslot;      // [S*stride]
-    VisRec* sorted;    // [S*stride]
-    int* hist;         // [S*G]
-    int* bstart;       // [S*(G+1)]
+    VisRec* rec;       // [S*stride] each segment in column order
+    VisRec* sorted;    // [S*stride] each snapshot in column order
+    int* bstart;       // [S][bstart_words] key offsets of each snapshot
     SnapMeta* meta;    // [S]
     SnapGeom* geom;    // [S]
     float2* kt;        // [S][I/kKTile][M+1][kKTile]
     float* pre;        // [S][I][I] corrected image before re-projection
     float* img;        // [S][I][I] re-projected images
-    unsigned* work;    // [1] cleared with the counters
     unsigned* pmax;    // [pmax_words(S)] spread slots of the image maxima
     size_t stride;
+};
+
+// The front end's part of the work buffers, with its segments.
+struct BinView {
+    VisRec *rec, *sorted;
+    int *boff, *seg;   // per snapshot: key offsets [segment][keys + 1]; extents [3][kMaxSegs]
+    int* bstart;
+    SnapMeta* meta;
+    SnapGeom* geom;
+    unsigned* pmax;
+    size_t stride, boff_stride, seg_stride;
+    int nseg, chunk;   // segments and visibilities per segment
 };
 
 // Tunable launch parameters (the autotuner picks among these).
@@ -121,7 +138,8 @@ struct Tuning {
     int persistent;     // accepted and kept; the column kernel has one launch form
 };
 
-// Stage ids for timing.
+// Stage ids for timing.  kStBin is the whole front end; reset, scan and scatter
+// keep their places in the list of stages and are never counted.
 enum Stage {
     kStReset = 0,
     kStBin,
@@ -137,12 +155,9 @@ enum Stage {
 const char* stage_name(int st);
 
 // Kernel launchers (fip_kernels.hip).  All launch asynchronously on stream.
-hipError_t launch_reset(const InputView& in, const WorkView& w, const PlanTables& p, int S,
-                        float cell, const int* norm_n_host, int norm_n_const, hipStream_t st);
-hipError_t launch_bin(const InputView& in, const WorkView& w, const PlanTables& p, int S,
-                      int nmax, double scale, hipStream_t st);
-hipError_t launch_scan(const WorkView& w, const PlanTables& p, int S, hipStream_t st);
-hipError_t launch_scatter(const WorkView& w, const PlanTables& p, int S, int nmax, hipStream_t st);
+// nmax: largest visibility count of the batch.
+hipError_t launch_bin(const InputView& in, const WorkView& w, const PlanTables& p, int S, int nmax, float cell,
+                      double scale, const int* norm_n_dev, int norm_n_const, hipStream_t st);
 hipError_t launch_stage1(const WorkView& w, const PlanTables& p, int S, const Tuning& tu,
                          hipStream_t st);
 hipError_t launch_stage2(const WorkView& w, const PlanTables& p, int S, const Tuning& tu,

@@ -1,12 +1,11 @@
 // HIP kernels of the FIP-TOI imaging-and-trigger path for gfx950 (CDNA4).
 //
-// Per batch of S snapshots the path runs eight launches (each covers all S
+// Per batch of S snapshots the path runs these launches (each covers all S
 // snapshots):
-//   reset    zero histograms / per-snapshot scalars, FP64 re-projection geometry
-//   bin      weighting (FIPkernels.cu:188-195), FP64 uv scaling, column-bucket
-//            histogram with per-visibility slots
-//   scan     exclusive scan of the bucket histogram
-//   scatter  visibilities into bucket order (counting sort by grid column)
+//   bin      weighting (FIPkernels.cu:188-195), FP64 uv scaling, each segment of
+//            a snapshot's visibilities sorted by grid column; per snapshot the
+//            FP64 re-projection geometry and cleared maximum slots
+//   merge    a snapshot's segments into one column order (not for one segment)
 //   stage1   per uv column c >= 0: deterministic integer LDS gridding of the
 //            Hermitian-folded grid column (FIPkernels.cu:197-245) and its
 //            length-g inverse FFT along the row axis, cropped to I rows
@@ -50,21 +49,6 @@ __device__ __forceinline__ unsigned* max_slot(unsigned* pm, int s, int set, int 
 }
 size_t pmax_words(int S) { return (size_t)S * kPmaxPer; }
 size_t pmax_index(int s, int set, int slot) { return max_slot_index(s, set, slot); }
-
-// exp(beta*(sqrt(1-x^2)-1)) (FIPkernels.cu:67-71), 0 for |x| > 1, as
-// 2^(C s - C) with C = beta log2 e and s = sqrt(1 - x^2) (1 - x^2 by one FMA,
-// hardware sqrt and exp2, ~1 ulp each).  s <= 1 carries an absolute error of
-// ~1e-7, so the exponent's error stays below ~2e-6 (C = 22.2) and the relative
-// error of ES below ~1.5e-6 at every x.  The form without the subtraction,
-// exp(-beta x^2 / (1 + s)), is no more accurate at this precision and costs
-// a reciprocal and three more instructions per tap.
-__device__ __forceinline__ float es_f(float x)
-{
-    constexpr float C = (float)(kBeta * 1.4426950408889634);
-    const float q = fmaf(-x, x, 1.0f);
-    if (q < 0.0f) return 0.0f;
-    return __builtin_amdgcn_exp2f(fmaf(C, __builtin_amdgcn_sqrtf(q), -C));
-}
 
 template <class T> __device__ __forceinline__ float vis_to_f(const void* p, size_t i);
 template <> __device__ __forceinline__ float vis_to_f<float>(const void* p, size_t i)
@@ -148,315 +132,375 @@ __device__ __forceinline__ int xcd_remap(int bid, int nb)
     return x * per + min(x, rem) + k;
 }
 
-__device__ __forceinline__ long long to_fixed(float x)
-{
-    return (long long)rintf(x);   // |x| < 2^62 by construction; exact for |x| >= 2^24
-}
-
-// ----------------------------------------------------------------- reset
-
-__global__ void k_reset(const float* __restrict__ vin, const int* __restrict__ nvis, int n_const,
-                        const int* __restrict__ norm_n, int norm_const, SnapMeta* meta, SnapGeom* geom,
-                        int* hist, unsigned* work, unsigned* pmax, int S, int G, int I, float cell)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < S * G) hist[i] = 0;
-    if (i < S * 2 * kMaxSlots) *max_slot(pmax, i / (2 * kMaxSlots), 0, i % (2 * kMaxSlots)) = 0u;
-    if (i == 0) work[0] = 0u;
-    if (i < S) {
-        SnapMeta m;
-        m.ngrid = 0;
-        m.rmax = -1;
-        m.r1max = -1;
-        m.maxv_bits = 0u;
-        m.maxp_bits = 0u;
-        m.maxd_bits = 0u;
-        m.nvis = nvis ? nvis[i] : n_const;
-        m.norm_n = norm_n ? norm_n[i] : norm_const;
-        meta[i] = m;
-
-        // Re-projection geometry (coordschange FIPkernels.cu:289-299 and the
-        // closed form of p2p :301-376), FP64 from the float V matrix.
-        const float* V = vin + (size_t)i * 9;
-        const double v00 = V[0], v01 = V[1], v10 = V[3], v11 = V[4];
-        const double v20 = V[6], v21 = V[7], v22 = V[8];
-        const double a22 = fabs(v22);
-        SnapGeom gm;
-        gm.m00 = -v00 / a22;
-        gm.m01 = v10 / a22;
-        gm.m10 = -v01 / a22;
-        gm.m11 = v11 / a22;
-        const double det = gm.m00 * gm.m11 - gm.m01 * gm.m10;
-        gm.i00 = gm.m11 / det;
-        gm.i01 = -gm.m01 / det;
-        gm.i10 = -gm.m10 / det;
-        gm.i11 = gm.m00 / det;
-        gm.im00 = fabs(gm.m00) > 1e-12 ? 1.0 / gm.m00 : 0.0;
-        gm.im10 = fabs(gm.m10) > 1e-12 ? 1.0 / gm.m10 : 0.0;
-        const double xi = v20 / v22, eta = v21 / v22;
-        const double delta = (double)cell;
-        gm.sx = -xi / delta;
-        gm.sy = eta / delta;
-        gm.delta = delta;
-        gm.sin_on = (xi * xi + eta * eta != 0.0) ? 1 : 0;
-        // Singular values of the affine part, and the largest direction-cosine
-        // radius any source or target can reach.
-        const double h = (double)(I / 2);
-        const double tr = gm.m00 * gm.m00 + gm.m01 * gm.m01 + gm.m10 * gm.m10 + gm.m11 * gm.m11;
-        const double dd = fabs(det);
-        const double disc = sqrt(fmax(0.0, tr * tr - 4.0 * dd * dd));
-        const double smax = sqrt(0.5 * (tr + disc)), smin = sqrt(fmax(0.0, 0.5 * (tr - disc)));
-        const double rmax = delta * (smax * h * 1.4142135623730951 + 4.0 + h);
-        const double kap = sqrt(xi * xi + eta * eta) * rmax / sqrt(fmax(1e-300, 1.0 - rmax * rmax));
-        gm.kappa = kap;
-        if (!(rmax < 0.9) || !(kap < 0.5) || !isfinite(det) || det == 0.0) {
-            gm.curv = -1.0;   // no usable bound: the splat scans whole images
-        } else {
-            gm.curv = kap;
-        }
-        // A pixel receives splat weight from the sources mapped into the open
-        // 2 x 2 square around it.  The map expands by at least
-        // smin (1 - kappa), so they lie in a set of diameter
-        // 2 sqrt(2) / (smin (1 - kappa)), which holds at most (d + 1)^2
-        // integer points.  Without a usable bound every pixel of the image
-        // counts.
-        {
-            const double den = smin * (1.0 - kap);
-            double cap = (gm.curv >= 0.0 && den > 0.0) ? 2.8284271247461903 / den + 1.0 : 0.0;
-            cap = cap * cap;
-            const double all = (double)I * (double)I;
-            gm.ccap = (int)fmin(gm.curv >= 0.0 && den > 0.0 ? ceil(cap) : all, fmin(all, 1073741824.0));
-            gm.ccap = max(gm.ccap, 1);
-        }
-        // n' = 1 - sqrt(1 - r^2) = r^2 (1/2 + r^2/8 + r^4/16 + 5 r^6/128 + ...);
-        // for r^2 <= 0.01 the terms after r^8 are below 3e-12 of n'.
-        // The splat takes this series along each group of 8 consecutive
-        // sources of a row (k = 0..7) from its quadratic Taylor model in k.
-        // r^2 is quadratic in k with |dr^2/dk| <= 2 r d and d2r^2/dk2 = 2 d^2,
-        // d = cell |(m00, m10)|; for r <= 0.1 the series' third k-derivative
-        // is at most 0.31 d^3, so the model's remainder at k <= 7 is at most
-        // 17.6 d^3 in n', 17.6 d^3 max(|sx|, |sy|) in pixels.  The series
-        // form is taken only where that is at most 5e-8 px (a tenth of an FP32
-        // ulp of the splat's local positions); otherwise the closed form per
-        // source.
-        const double dcol = delta * sqrt(gm.m00 * gm.m00 + gm.m10 * gm.m10);
-        const double qerr = 18.0 * dcol * dcol * dcol * fmax(fabs(gm.sx), fabs(gm.sy));
-        gm.series = (rmax * rmax <= 0.01 && qerr <= 5e-8) ? 1 : 0;
-        gm.pad = 0;
-        geom[i] = gm;
-    }
-}
-
-// ------------------------------------------------------------------- bin
-
-// Threads of a bin workgroup and visibilities per thread (a workgroup bins
-// kBinThreads * kBinVpt visibilities).  Large workgroups keep the number of
-// per-workgroup bucket flushes (global atomics) low; 16 waves each keep the
-// CUs busy although a step has only ~100 workgroups.
-constexpr int kBinThreads = 1024;
-constexpr int kBinVpt = 4;
-// Largest grid size: bounds the bucket counts one bin or scan thread holds.
+// Largest grid size: bounds the keys one scan thread holds.
 constexpr int kMaxGrid = 12288;
 
-// Block-privatised column histogram: slots within the block come from LDS
-// atomics, then one global atomic per non-empty bucket reserves the block's
-// range, so the hot central buckets see one global atomic per block instead
-// of one per visibility.
-template <class VT>
-__global__ __launch_bounds__(kBinThreads) void k_bin(InputView in, VisRec* __restrict__ rec, int2* __restrict__ bs,
-                                             int* __restrict__ hist, SnapMeta* __restrict__ meta, int G,
-                                             double scale)
+// ------------------------------------------------------------- front end
+
+// Re-projection geometry of one snapshot from its V matrix (vin, 9 floats).
+__device__ SnapGeom snap_geometry(const float* __restrict__ vin, int I, float cell)
 {
-    extern __shared__ int lh[];   // G ints: local counts, then block bases
-    constexpr int NW = kBinThreads / 64;
-    __shared__ int sh_i[3][NW];
-    __shared__ unsigned sh_u[NW];
-    const int s = blockIdx.y;
-    const int ns = in.nvis ? in.nvis[s] : in.n_const;
+    // Re-projection geometry (coordschange FIPkernels.cu:289-299 and the
+    // closed form of p2p :301-376), FP64 from the float V matrix.
+    const float* V = vin;
+    const double v00 = V[0], v01 = V[1], v10 = V[3], v11 = V[4];
+    const double v20 = V[6], v21 = V[7], v22 = V[8];
+    const double a22 = fabs(v22);
+    SnapGeom gm;
+    gm.m00 = -v00 / a22;
+    gm.m01 = v10 / a22;
+    gm.m10 = -v01 / a22;
+    gm.m11 = v11 / a22;
+    const double det = gm.m00 * gm.m11 - gm.m01 * gm.m10;
+    gm.i00 = gm.m11 / det;
+    gm.i01 = -gm.m01 / det;
+    gm.i10 = -gm.m10 / det;
+    gm.i11 = gm.m00 / det;
+    gm.im00 = fabs(gm.m00) > 1e-12 ? 1.0 / gm.m00 : 0.0;
+    gm.im10 = fabs(gm.m10) > 1e-12 ? 1.0 / gm.m10 : 0.0;
+    const double xi = v20 / v22, eta = v21 / v22;
+    const double delta = (double)cell;
+    gm.sx = -xi / delta;
+    gm.sy = eta / delta;
+    gm.delta = delta;
+    gm.sin_on = (xi * xi + eta * eta != 0.0) ? 1 : 0;
+    // Singular values of the affine part, and the largest direction-cosine
+    // radius any source or target can reach.
+    const double h = (double)(I / 2);
+    const double tr = gm.m00 * gm.m00 + gm.m01 * gm.m01 + gm.m10 * gm.m10 + gm.m11 * gm.m11;
+    const double dd = fabs(det);
+    const double disc = sqrt(fmax(0.0, tr * tr - 4.0 * dd * dd));
+    const double smax = sqrt(0.5 * (tr + disc)), smin = sqrt(fmax(0.0, 0.5 * (tr - disc)));
+    const double rmax = delta * (smax * h * 1.4142135623730951 + 4.0 + h);
+    const double kap = sqrt(xi * xi + eta * eta) * rmax / sqrt(fmax(1e-300, 1.0 - rmax * rmax));
+    gm.kappa = kap;
+    if (!(rmax < 0.9) || !(kap < 0.5) || !isfinite(det) || det == 0.0) {
+        gm.curv = -1.0;   // no usable bound: the splat scans whole images
+    } else {
+        gm.curv = kap;
+    }
+    // A pixel receives splat weight from the sources mapped into the open
+    // 2 x 2 square around it.  The map expands by at least
+    // smin (1 - kappa), so they lie in a set of diameter
+    // 2 sqrt(2) / (smin (1 - kappa)), which holds at most (d + 1)^2
+    // integer points.  Without a usable bound every pixel of the image
+    // counts.
+    {
+        const double den = smin * (1.0 - kap);
+        double cap = (gm.curv >= 0.0 && den > 0.0) ? 2.8284271247461903 / den + 1.0 : 0.0;
+        cap = cap * cap;
+        const double all = (double)I * (double)I;
+        gm.ccap = (int)fmin(gm.curv >= 0.0 && den > 0.0 ? ceil(cap) : all, fmin(all, 1073741824.0));
+        gm.ccap = max(gm.ccap, 1);
+    }
+    // n' = 1 - sqrt(1 - r^2) = r^2 (1/2 + r^2/8 + r^4/16 + 5 r^6/128 + ...);
+    // for r^2 <= 0.01 the terms after r^8 are below 3e-12 of n'.
+    // The splat takes this series along each group of 8 consecutive
+    // sources of a row (k = 0..7) from its quadratic Taylor model in k.
+    // r^2 is quadratic in k with |dr^2/dk| <= 2 r d and d2r^2/dk2 = 2 d^2,
+    // d = cell |(m00, m10)|; for r <= 0.1 the series' third k-derivative
+    // is at most 0.31 d^3, so the model's remainder at k <= 7 is at most
+    // 17.6 d^3 in n', 17.6 d^3 max(|sx|, |sy|) in pixels.  The series
+    // form is taken only where that is at most 5e-8 px (a tenth of an FP32
+    // ulp of the splat's local positions); otherwise the closed form per
+    // source.
+    const double dcol = delta * sqrt(gm.m00 * gm.m00 + gm.m10 * gm.m10);
+    const double qerr = 18.0 * dcol * dcol * dcol * fmax(fabs(gm.sx), fabs(gm.sy));
+    gm.series = (rmax * rmax <= 0.01 && qerr <= 5e-8) ? 1 : 0;
+    gm.pad = 0;
+    return gm;
+}
+
+// Threads of a bin workgroup.  16 waves each keep the CUs busy although a
+// step has at most 64 workgroups per snapshot.
+constexpr int kBinThreads = 1024;
+
+// Column keys, in the order of the sorted records.  With the Hermitian fold
+// column c takes its own records and the mirrored ones of column -c, so beyond
+// the axis b2 = floor(p2) and -b2 share a key, and a column's records are one
+// run of keys.  Within eight columns of the axis the sign stays apart
+// (0..16 for b2 = -8..8): there a record can reach a column both ways, and a
+// column walks its direct and its mirrored run.
+__host__ __device__ constexpr int bin_keys(int G) { return G / 2 + 13; }
+// Ints of one row of key offsets (keys + 1, in 16-byte units).
+__host__ __device__ constexpr int boff_row(int G) { return (bin_keys(G) + 1 + 3) & ~3; }
+__device__ __forceinline__ int bin_key(int b2) { return 8 + (b2 < -8 ? -b2 : b2); }
+
+// Grid coordinates and weighted value of one visibility as a record, and its
+// column key; -1 where it has no tap.  rj = 1 / |V00 V11 - V01 V10|
+// (computeVisWeighted, FIPkernels.cu:188-195); positions in FP64, B * (cell g)
+// (FIPkernels.cu:211-212, 584).  r1, r2: largest |tap| on each axis.
+__device__ __forceinline__ int vis_record(float vr, float vi, float b1, float b2, double rj, double scale, int G,
+                                          VisRec& r, int& r1, int& r2)
+{
     const int M = G / 2;
-    for (int b = threadIdx.x; b < G; b += kBinThreads) lh[b] = 0;
-    __syncthreads();
-    int rmax = -1, r1max = -1, cnt = 0;
-    unsigned vmax = 0u;
-    int bk[kBinVpt], slot[kBinVpt];
+    const double p1 = (double)b1 * scale, p2 = (double)b2 * scale;
+    // Coordinates far outside the grid have no taps (and must not overflow int).
+    if (!(fabs(p1) < (double)G && fabs(p2) < (double)G)) return -1;
+    const double fb1 = floor(p1), fb2 = floor(p2);
+    const float f1 = (float)(p1 - fb1), f2 = (float)(p2 - fb2);
+    const int i1 = (int)fb1, i2 = (int)fb2;
+    // Taps: r in [ceil(p-4), floor(p+4)] (FIPkernels.cu:213-243), eight, or
+    // nine where the position is an integer.
+    const int nine1 = f1 > 0.0f ? 0 : 1, nine2 = f2 > 0.0f ? 0 : 1;
+    const int lo1 = i1 - 3 - nine1, hi1 = i1 + 4, lo2 = i2 - 3 - nine2, hi2 = i2 + 4;
+    const int clo1 = max(lo1, -M), chi1 = min(hi1, M - 1), clo2 = max(lo2, -M), chi2 = min(hi2, M - 1);
+    if (clo1 > chi1 || clo2 > chi2) return -1;
+    const int edge = (lo1 <= -M || hi1 >= M) ? 1 : 0;
+    r.row = (lo1 << 2) | (nine1 << 1) | edge;
+    r.f1 = nine1 ? 1.0f : f1;
+    r.col = (lo2 << 1) | nine2;
+    r.f2 = nine2 ? 1.0f : f2;
+    r.vr = (float)((double)vr * rj);
+    r.vi = (float)((double)vi * rj);
+    r1 = max(chi1, -clo1);
+    r2 = max(chi2, -clo2);
+    return bin_key(i2);
+}
+
+// Field k of a snapshot's gridded extent: largest |column tap|, |row tap| and
+// weighted magnitude (float bits).
+__device__ __forceinline__ void set_extent(SnapMeta& m, int k, int v)
+{
+    if (k == 0) m.rmax = v;
+    if (k == 1) m.r1max = v;
+    if (k == 2) m.maxv_bits = (unsigned)v;
+}
+
+// One segment of one snapshot's visibilities into column order: records and
+// keys, an LDS histogram whose atomics give each record its place within its
+// key, the exclusive scan of the counts, and the records to their places in
+// the segment's own stretch of the output, with the segment's key offsets.
+// Nothing is combined across workgroups here: no zeroed counters and no
+// global atomics.  A snapshot of one segment is done with that; k_merge puts
+// several into one order.
+//
+// VPT visibilities per thread held in registers between the two phases; 0:
+// any number, recomputed in the second phase.  Workgroup `nseg` of a snapshot
+// sets up what the later stages need: geometry, normalisation and cleared
+// maximum slots.
+//
+// Latency bound: at 2048^2 with 32640 visibilities 1.2 us of loads, 1.7 of
+// FP64 and LDS atomics, 1.5 of scan and 0.6 of stores; the rest of its 8 us is
+// launch and write-back.  With k_merge 7, 14, 15, 30 and 70 us (rocprofv3, three
+// snapshots) at 256^2, 1024^2, 2048^2, 4096^2 and 8192^2 with 2016, 8128, 32640,
+// 130816 and 523776 visibilities; clearing, histogram with global atomics, scan
+// and scatter as four launches took 16, 19.5, 22.6, 32 and 74.  (A column
+// kernel that took its records from the sorted segments themselves, with no
+// merge, lost more than the merge costs: 95 against 84 us at 4096^2.)
+template <class VT, int VPT>
+__global__ __launch_bounds__(kBinThreads) void k_bin(InputView in, BinView out, const int* __restrict__ norm_n,
+                                                     int norm_const, int G, int I, float cell, double scale)
+{
+    extern __shared__ int lh[];   // bin_keys(G) + 1 ints: counts, then starts
+    constexpr int NW = kBinThreads / 64;
+    constexpr int PER = (bin_keys(kMaxGrid) + kBinThreads - 1) / kBinThreads;   // keys per thread of the scan
+    __shared__ int sh_i[3][NW];
+    const int s = blockIdx.y, seg = blockIdx.x, t = threadIdx.x, lane = t & 63, wid = t >> 6;
     const float* V = in.vin + (size_t)s * 9;
-    // computeVisWeighted: v / |V00 V11 - V01 V10| (FIPkernels.cu:188-195)
-    const double J = fabs((double)V[0] * (double)V[4] - (double)V[1] * (double)V[3]);
+    if (seg == out.nseg) {
+        if (t < 2 * kMaxSlots) *max_slot(out.pmax, s, 0, t) = 0u;
+        if (t == 128) out.geom[s] = snap_geometry(V, I, cell);
+        if (t == 192) {
+            out.meta[s].maxp_bits = 0u;
+            out.meta[s].maxd_bits = 0u;
+            out.meta[s].norm_n = norm_n ? norm_n[s] : norm_const;
+        }
+        return;
+    }
+    const int ns = in.nvis ? in.nvis[s] : in.n_const;
+    const int K = bin_keys(G);
+    const int beg = seg * out.chunk, end = min(beg + out.chunk, ns);
+    const double rj = 1.0 / fabs((double)V[0] * (double)V[4] - (double)V[1] * (double)V[3]);
+    const size_t sbase = (size_t)s * in.stride;
+    int rmax = -1, r1max = -1;
+    unsigned vmax = 0u;
+    VisRec rec[VPT > 0 ? VPT : 1];
+    int key[VPT > 0 ? VPT : 1], slot[VPT > 0 ? VPT : 1];
+    auto note = [&](const VisRec& r, int r1, int r2) {
+        rmax = max(rmax, r2);
+        r1max = max(r1max, r1);
+        vmax = max(vmax, __float_as_uint(fmaxf(fabsf(r.vr), fabsf(r.vi))));
+    };
     // Every input of the thread's visibilities is loaded before any is used,
     // so the loads are in flight together: unconditionally, from an index
     // clamped into this snapshot's rows (entries past its count are loaded
     // but not used), since a load behind a per-lane test would wait in turn.
-    float lvr[kBinVpt], lvi[kBinVpt], lb1[kBinVpt], lb2[kBinVpt];
-    const int nlast = max(ns - 1, 0);
-#pragma unroll
-    for (int k = 0; k < kBinVpt; ++k) {
-        const int n = min(blockIdx.x * (kBinThreads * kBinVpt) + k * kBinThreads + threadIdx.x, nlast);
-        const size_t q = (size_t)s * in.stride + (size_t)n;
+    float lvr[VPT > 0 ? VPT : 1], lvi[VPT > 0 ? VPT : 1], lb1[VPT > 0 ? VPT : 1], lb2[VPT > 0 ? VPT : 1];
+    auto load = [&](int k, int n) {
+        const size_t q = sbase + (size_t)n;
         lvr[k] = vis_to_f<VT>(in.vis_re, q);
         lvi[k] = vis_to_f<VT>(in.vis_im, q);
         lb1[k] = in.bin[2 * q];
         lb2[k] = in.bin[2 * q + 1];
-    }
-    // Keeps the loads above the per-visibility tests (the compiler would
-    // otherwise sink each into the branch that uses it).
+    };
+    if constexpr (VPT > 0) {
+        if (beg < end) {
 #pragma unroll
-    for (int k = 0; k < kBinVpt; ++k) asm volatile("" ::"v"(lvr[k]), "v"(lvi[k]), "v"(lb1[k]), "v"(lb2[k]));
-#pragma unroll
-    for (int k = 0; k < kBinVpt; ++k) {
-        bk[k] = -1;
-        slot[k] = 0;
-        const int n = blockIdx.x * (kBinThreads * kBinVpt) + k * kBinThreads + threadIdx.x;
-        if (n >= ns) continue;
-        const size_t q = (size_t)s * in.stride + (size_t)n;
-        const float vr = (float)((double)lvr[k] / J);
-        const float vi = (float)((double)lvi[k] / J);
-        // grid coordinates in FP64: B * (cell * g) (FIPkernels.cu:211-212, 584)
-        const double p1 = (double)lb1[k] * scale;
-        const double p2 = (double)lb2[k] * scale;
-        // Coordinates far outside the grid have no taps (and must not overflow int).
-        if (!(fabs(p1) < (double)G && fabs(p2) < (double)G)) continue;
-        const double fb1 = floor(p1), fb2 = floor(p2);
-        VisRec r;
-        r.b1 = (int)fb1;
-        r.f1 = (float)(p1 - fb1);
-        r.b2 = (int)fb2;
-        r.f2 = (float)(p2 - fb2);
-        r.vr = vr;
-        r.vi = vi;
-        const int lo1 = max(r.b1 - 4 + (r.f1 > 0.0f ? 1 : 0), -M), hi1 = min(r.b1 + 4, M - 1);
-        const int lo2 = max(r.b2 - 4 + (r.f2 > 0.0f ? 1 : 0), -M), hi2 = min(r.b2 + 4, M - 1);
-        if (lo1 > hi1 || lo2 > hi2) continue;
-        bk[k] = min(max(r.b2 + M, 0), G - 1);
-        slot[k] = atomicAdd(&lh[bk[k]], 1);
-        rec[q] = r;
-        rmax = max(rmax, max(hi2, -lo2));
-        r1max = max(r1max, max(hi1, -lo1));
-        cnt += 1;
-        vmax = max(vmax, __float_as_uint(fmaxf(fabsf(vr), fabsf(vi))));
+            for (int k = 0; k < VPT; ++k) load(k, min(beg + k * kBinThreads + t, end - 1));
+        }
     }
+    for (int b = t; b <= K; b += kBinThreads) lh[b] = 0;
     __syncthreads();
-    // Flush: each thread's bucket counts are read, then all of its global
-    // atomics are issued before the first result is used.
-    {
-        constexpr int FL = (kMaxGrid + kBinThreads - 1) / kBinThreads;
-        int fc[FL];
+    if constexpr (VPT > 0) {
 #pragma unroll
-        for (int k = 0; k < FL; ++k) {
-            const int b = threadIdx.x + k * kBinThreads;
-            fc[k] = b < G ? lh[b] : 0;
+        for (int k = 0; k < VPT; ++k) {
+            int r1, r2;
+            key[k] = beg + k * kBinThreads + t < end
+                         ? vis_record(lvr[k], lvi[k], lb1[k], lb2[k], rj, scale, G, rec[k], r1, r2)
+                         : -1;
+            if (key[k] >= 0) {
+                slot[k] = atomicAdd(&lh[key[k]], 1);
+                note(rec[k], r1, r2);
+            }
         }
-#pragma unroll
-        for (int k = 0; k < FL; ++k) {
-            const int b = threadIdx.x + k * kBinThreads;
-            if (fc[k] > 0) fc[k] = atomicAdd(&hist[(size_t)s * G + b], fc[k]);
+    } else {
+        for (int n = beg + t; n < end; n += kBinThreads) {
+            int r1, r2;
+            load(0, n);
+            const int b = vis_record(lvr[0], lvi[0], lb1[0], lb2[0], rj, scale, G, rec[0], r1, r2);
+            if (b >= 0) {
+                atomicAdd(&lh[b], 1);
+                note(rec[0], r1, r2);
+            }
         }
-#pragma unroll
-        for (int k = 0; k < FL; ++k) {
-            const int b = threadIdx.x + k * kBinThreads;
-            if (b < G) lh[b] = fc[k];
-        }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < kBinVpt; ++k) {
-        const int n = blockIdx.x * (kBinThreads * kBinVpt) + k * kBinThreads + threadIdx.x;
-        if (n >= ns) continue;
-        const size_t q = (size_t)s * in.stride + (size_t)n;
-        bs[q] = bk[k] >= 0 ? make_int2(bk[k], lh[bk[k]] + slot[k]) : make_int2(-1, 0);
     }
     rmax = wave_max_i(rmax);
     r1max = wave_max_i(r1max);
-    cnt = wave_sum_i(cnt);
     vmax = wave_max_u(vmax);
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
     if (lane == 0) {
         sh_i[0][wid] = rmax;
         sh_i[1][wid] = r1max;
-        sh_i[2][wid] = cnt;
-        sh_u[wid] = vmax;
+        sh_i[2][wid] = (int)vmax;
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
-        for (int k = 1; k < NW; ++k) {
-            rmax = max(rmax, sh_i[0][k]);
-            r1max = max(r1max, sh_i[1][k]);
-            vmax = max(vmax, sh_u[k]);
-            cnt += sh_i[2][k];
-        }
-        if (cnt > 0) {
-            atomicMax(&meta[s].rmax, rmax);
-            atomicMax(&meta[s].r1max, r1max);
-            atomicMax(&meta[s].maxv_bits, vmax);
-            atomicAdd(&meta[s].ngrid, cnt);
-        }
+    if (t < 3) {   // the float bits of a non-negative maximum order as int
+        int v = sh_i[t][0];
+        for (int k = 1; k < NW; ++k) v = max(v, sh_i[t][k]);
+        if (out.nseg > 1)
+            out.seg[(size_t)s * out.seg_stride + t * kMaxSegs + seg] = v;
+        else
+            set_extent(out.meta[s], t, v);
     }
-}
-
-// ------------------------------------------------------------------ scan
-
-__global__ __launch_bounds__(1024) void k_scan(const int* __restrict__ hist, int* __restrict__ bstart, int G)
-{
-    // Exclusive prefix of the bucket counts: each thread loads a contiguous
-    // chunk into registers (one round of loads), waves scan their chunk sums
-    // with shuffles, one wave scans the 16 wave totals.
-    constexpr int PER = (kMaxGrid + 1023) / 1024;
-    __shared__ int wsum[16];
-    const int s = blockIdx.x;
-    const int t = threadIdx.x, lane = t & 63, wid = t >> 6;
-    const int per = (G + 1023) / 1024;
-    const int beg = min(t * per, G), end = min(beg + per, G);
-    const int* h = hist + (size_t)s * G;
-    int* o = bstart + (size_t)s * (G + 1);
-    int v[PER];
+    // Exclusive scan: each thread's run of keys in registers, shuffles within
+    // a wave, the wave totals summed by everyone.
+    const int per = (K + kBinThreads - 1) / kBinThreads;
+    int v[PER], local = 0;
 #pragma unroll
-    for (int k = 0; k < PER; ++k) v[k] = (beg + k < end) ? h[beg + k] : 0;
-    int local = 0;
-#pragma unroll
-    for (int k = 0; k < PER; ++k) local += v[k];
+    for (int k = 0; k < PER; ++k) {
+        const int b = t * per + k;
+        v[k] = (k < per && b < K) ? lh[b] : 0;
+        local += v[k];
+    }
     int x = local;
 #pragma unroll
     for (int d = 1; d < 64; d <<= 1) {
         const int y = __shfl_up(x, d);
         if (lane >= d) x += y;
     }
-    if (lane == 63) wsum[wid] = x;
+    __syncthreads();   // sh_i is read, the counts are in registers
+    if (lane == 63) sh_i[0][wid] = x;
     __syncthreads();
-    if (wid == 0) {
-        int w = lane < 16 ? wsum[lane] : 0;
+    int run = x - local;
 #pragma unroll
-        for (int d = 1; d < 16; d <<= 1) {
-            const int y = __shfl_up(w, d);
-            if (lane >= d) w += y;
-        }
-        if (lane < 16) wsum[lane] = w;   // inclusive totals
-    }
-    __syncthreads();
-    int run = x - local + (wid > 0 ? wsum[wid - 1] : 0);
+    for (int k = 0; k < NW; ++k) run += k < wid ? sh_i[0][k] : 0;
 #pragma unroll
     for (int k = 0; k < PER; ++k) {
-        if (beg + k < end) o[beg + k] = run;
+        const int b = t * per + k;
+        if (k < per && b < K) lh[b] = run;
         run += v[k];
     }
-    if (t == 1023) o[G] = wsum[15];
+    if (t == kBinThreads - 1) lh[K] = run;
+    __syncthreads();
+    int* o = out.nseg > 1 ? out.boff + (size_t)s * out.boff_stride + (size_t)seg * boff_row(G)
+                          : out.bstart + (size_t)s * boff_row(G);
+    for (int b = t; b <= K; b += kBinThreads) o[b] = lh[b];
+    VisRec* dst = (out.nseg > 1 ? out.rec : out.sorted) + sbase + (size_t)beg;
+    if constexpr (VPT > 0) {
+#pragma unroll
+        for (int k = 0; k < VPT; ++k)
+            if (key[k] >= 0) dst[lh[key[k]] + slot[k]] = rec[k];
+    } else {
+        __syncthreads();   // the offsets are stored; the starts become cursors
+        for (int n = beg + t; n < end; n += kBinThreads) {
+            int r1, r2;
+            load(0, n);
+            const int b = vis_record(lvr[0], lvi[0], lb1[0], lb2[0], rj, scale, G, rec[0], r1, r2);
+            if (b >= 0) dst[atomicAdd(&lh[b], 1)] = rec[0];
+        }
+    }
 }
 
-// --------------------------------------------------------------- scatter
-
-__global__ __launch_bounds__(256) void k_scatter(const VisRec* __restrict__ rec, const int2* __restrict__ bs,
-                                                 const int* __restrict__ bstart, VisRec* __restrict__ sorted,
-                                                 const SnapMeta* __restrict__ meta, size_t stride, int G)
+// Sum of rows [lo, hi) of four neighbouring keys' offsets, sixteen loads in
+// flight (rows past the end are read as the last one and masked off).
+__device__ __forceinline__ int4 sum_rows(const int* __restrict__ o, int row, int lo, int hi)
 {
-    const int s = blockIdx.y;
-    const int n = blockIdx.x * 256 + threadIdx.x;
-    // The last workgroup reaches past the largest count; n < stride keeps
-    // the loads inside this snapshot's rows, so they are issued before its
-    // count is known and all three are in flight together.
-    if ((size_t)n >= stride) return;
-    const size_t q = (size_t)s * stride + (size_t)n;
-    const int2 key = bs[q];
-    const VisRec r = rec[q];
-    if (n >= meta[s].nvis || key.x < 0) return;
-    sorted[(size_t)s * stride + (size_t)(bstart[(size_t)s * (G + 1) + key.x] + key.y)] = r;
+    int4 sum = make_int4(0, 0, 0, 0);
+    for (int g0 = lo; g0 < hi; g0 += 16) {
+        int4 x[16];
+#pragma unroll
+        for (int k = 0; k < 16; ++k) x[k] = *reinterpret_cast<const int4*>(o + (size_t)min(g0 + k, hi - 1) * row);
+#pragma unroll
+        for (int k = 0; k < 16; ++k) {
+            const int m = g0 + k < hi ? -1 : 0;
+            sum.x += x[k].x & m;
+            sum.y += x[k].y & m;
+            sum.z += x[k].z & m;
+            sum.w += x[k].w & m;
+        }
+    }
+    return sum;
+}
+
+// A snapshot's segments into one column order.  boff[g] is segment g's own
+// exclusive scan, so the scan of the whole snapshot is its sum over the
+// segments, and a record of segment `seg` and key k moves up by the later
+// segments' offsets of k (what they hold before k) and the earlier segments'
+// offsets of k + 1 (what they hold up to k).  Every workgroup adds the rows of
+// offsets up by itself (at most 64, four keys per load, from L2) rather than
+// wait for a launch that does; segment 0's also writes the snapshot's offsets
+// and extent.
+__global__ __launch_bounds__(kBinThreads) void k_merge(BinView v, int G)
+{
+    extern __shared__ int lds[];   // 2 boff_row(G) ints
+    const int s = blockIdx.y, seg = blockIdx.x, t = threadIdx.x;
+    const int K = bin_keys(G), row = boff_row(G);
+    int* before = lds;
+    int* after = lds + row;
+    const int* bo = v.boff + (size_t)s * v.boff_stride;
+    const int cnt = bo[(size_t)seg * row + K];
+    const VisRec* src = v.rec + (size_t)s * v.stride + (size_t)seg * v.chunk;
+    VisRec* dst = v.sorted + (size_t)s * v.stride;
+    auto put = [&](VisRec q, int i) {
+        const int key = bin_key((q.col >> 1) + 3 + (q.col & 1));
+        dst[i + after[key] + before[key + 1]] = q;
+    };
+    // The first records are loaded before their displacement is known (the
+    // segment has at least one place).
+    const int last = max(cnt - 1, 0);
+    const VisRec r0 = src[min(t, last)], r1 = src[min(t + kBinThreads, last)];
+    for (int b = 4 * t; b < row; b += 4 * kBinThreads) {
+        const int4 lo = sum_rows(bo + b, row, 0, seg), hi = sum_rows(bo + b, row, seg + 1, v.nseg);
+        *reinterpret_cast<int4*>(before + b) = lo;
+        *reinterpret_cast<int4*>(after + b) = hi;
+        if (seg == 0) {
+            const int4 own = *reinterpret_cast<const int4*>(bo + b);
+            *reinterpret_cast<int4*>(v.bstart + (size_t)s * row + b) =
+                make_int4(own.x + hi.x, own.y + hi.y, own.z + hi.z, own.w + hi.w);
+        }
+    }
+    if (seg == 0 && t < 64) {
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            const int* sm = v.seg + (size_t)s * v.seg_stride + k * kMaxSegs;
+            const int m = wave_max_i(t < v.nseg ? sm[t] : -1);
+            if (t == 0) set_extent(v.meta[s], k, m);
+        }
+    }
+    __syncthreads();
+    if (t < cnt) put(r0, t);
+    if (t + kBinThreads < cnt) put(r1, t + kBinThreads);
+    for (int i = t + 2 * kBinThreads; i < cnt; i += kBinThreads) put(src[i], i);
 }
 
 // ---------------------------------------------------------------- stage 1
@@ -470,29 +514,38 @@ __global__ __launch_bounds__(256) void k_scatter(const VisRec* __restrict__ rec,
 // whose taps reach the grid's edge is marked (edge): its taps are clipped and
 // a mirrored tap at -g/2 stays there, so each one is placed by itself.
 struct ColRec {
-    int b1, u0;
+    int lo1, u0;
     float f, vr, vi;
     int nine;
     bool mirror, edge, live;
 };
 
-// Taps follow FIPkernels.cu:213-243: r in [ceil(p-4), floor(p+4)] clipped to
-// [-g/2, g/2-1].
+// exp(beta*(sqrt(1-x^2)-1)) (FIPkernels.cu:67-71) of a tap distance X = 4x in
+// cells, |X| <= 4, as 2^(C s - C) with C = beta log2 e and s = sqrt(1 - x^2)
+// (1 - x^2 by one FMA, hardware sqrt and exp2, ~1 ulp each; the 1/16 of X^2
+// is moved into the constants, powers of two).  s <= 1 carries an absolute
+// error of ~1e-7, so the exponent's error stays below ~2e-6 (C = 22.2) and
+// the relative error of ES below ~1.5e-6 at every x.  The form without the
+// subtraction, exp(-beta x^2 / (1 + s)), is no more accurate at this precision
+// and costs a reciprocal and three more instructions per tap.
+__device__ __forceinline__ float es_tap(float X)
+{
+    constexpr float C = (float)(kBeta * 1.4426950408889634);
+    return __builtin_amdgcn_exp2f(fmaf(0.25f * C, __builtin_amdgcn_sqrtf(fmaf(-X, X, 16.0f)), -C));
+}
+
 __device__ __forceinline__ ColRec prep_rec(const VisRec& r, int col, bool mirror, int M)
 {
     ColRec c;
-    c.b1 = r.b1;
+    c.lo1 = r.row >> 2;
+    c.nine = (r.row >> 1) & 1;
+    c.edge = r.row & 1;
     c.mirror = mirror;
-    const bool frac = r.f1 > 0.0f;
-    c.nine = frac ? 0 : 1;
-    c.f = frac ? (mirror ? 1.0f - r.f1 : r.f1) : 1.0f;
-    const int lo1 = r.b1 - 4 + (frac ? 1 : 0), hi1 = r.b1 + 4;
-    c.u0 = M + (mirror ? -hi1 : lo1);
-    c.edge = lo1 <= -M || hi1 >= M;
-    const int lo2 = max(r.b2 - 4 + (r.f2 > 0.0f ? 1 : 0), -M);
-    const int hi2 = min(r.b2 + 4, M - 1);
-    c.live = col >= lo2 && col <= hi2 && lo1 < M && hi1 >= -M;
-    const float w2 = c.live ? es_f(((float)(col - r.b2) - r.f2) * 0.25f) * 0.5f : 0.0f;
+    c.f = mirror && !c.nine ? 1.0f - r.f1 : r.f1;
+    c.u0 = mirror ? M - (c.lo1 + 7 + c.nine) : M + c.lo1;
+    const int d = col - (r.col >> 1);   // the column's place among the record's taps
+    c.live = (unsigned)d <= (unsigned)(7 + (r.col & 1));
+    const float w2 = es_tap((float)(d - 3) - r.f2) * 0.5f;   // only of a live record
     c.vr = r.vr * w2;
     c.vi = (mirror ? -r.vi : r.vi) * w2;
     return c;
@@ -511,15 +564,6 @@ __device__ __forceinline__ int cvt_round_half_up_i32(float x)
     int r;
     asm("v_cvt_rpi_i32_f32 %0, %1" : "=v"(r) : "v"(x));
     return r;
-}
-
-// ES of a tap distance X in cells, |X| <= 4 (as es_f without the range test):
-// 2^(C sqrt(1 - X^2/16) - C) with the 1/16 moved into the constants (powers
-// of two, so the same roundings).
-__device__ __forceinline__ float es_tap(float X)
-{
-    constexpr float C = (float)(kBeta * 1.4426950408889634);
-    return __builtin_amdgcn_exp2f(fmaf(0.25f * C, __builtin_amdgcn_sqrtf(fmaf(-X, X, 16.0f)), -C));
 }
 
 // Shape of the column kernel.  Rows are grouped in blocks of RBS rows, each
@@ -590,7 +634,7 @@ __device__ __forceinline__ void grid_taps(const ColRec& c, const float* sc, int*
         return;
     }
     for (int j = 0; j < 8 + c.nine; ++j) {
-        const int t1 = c.mirror ? c.b1 + 4 - j : c.b1 - 3 - c.nine + j;   // the record's own row
+        const int t1 = c.mirror ? c.lo1 + 7 + c.nine - j : c.lo1 + j;   // the record's own row
         if (t1 < -M || t1 > M - 1) continue;
         const int u = (c.mirror ? (t1 == -M ? -M : -t1) : t1) + M;
         const float wk = es_tap((float)(j - 3) - c.f) * sc[u / Sh::RBS];
@@ -617,7 +661,7 @@ __device__ __forceinline__ void tap_mass(const ColRec& c, float qs, unsigned lon
         ba = c.u0 / Sh::RBS;
         bz = (c.u0 + 7 + c.nine) / Sh::RBS;
     } else {
-        const int lo1 = max(c.b1 - 3 - c.nine, -Sh::M), hi1 = min(c.b1 + 4, Sh::M - 1);
+        const int lo1 = max(c.lo1, -Sh::M), hi1 = min(c.lo1 + 7 + c.nine, Sh::M - 1);
         const int a = c.mirror ? (lo1 == -Sh::M ? -Sh::M : -lo1) : lo1;
         ba = (a + Sh::M) / Sh::RBS;
         bz = ((c.mirror ? (hi1 == -Sh::M ? -Sh::M : -hi1) : hi1) + Sh::M) / Sh::RBS;
@@ -631,19 +675,21 @@ __device__ __forceinline__ void tap_mass(const ColRec& c, float qs, unsigned lon
     if (bz != ba) atomicAdd(&mass[bz * Sh::MC + (threadIdx.x & (Sh::MC - 1))], q);
 }
 
-// Record ranges of column c: direct buckets cc-4..cc+4 and mirrored buckets
-// cm-4..cm+4 (x, y: direct [x, y); z, w: mirrored [z, w)).
+// Runs of the sorted records that can reach column c: [x, y) and [z, w).  The
+// first holds column c's own records, beyond eight columns from the axis with
+// the mirrored ones of column -c among them; nearer the axis those are the
+// second run.  Column g/2 is its own mirror and walks its records both ways.
 template <int G>
 __device__ __forceinline__ int4 column_ranges(const int* __restrict__ bst, int c)
 {
-    constexpr int M = G / 2;
-    const int cc = (c == M) ? -M : c;
-    const int cm = (c == 0) ? 0 : ((c == M) ? -M : -c);
+    constexpr int M = G / 2, K = bin_keys(G);
+    const int a0 = c + 4, a1 = min(c + 12, K - 1);
+    const int b0 = c <= 4 ? 4 - c : 0, b1 = 12 - c;
     int4 r;
-    r.x = bst[min(max(cc - 4 + M, 0), G - 1)];
-    r.y = bst[min(max(cc + 4 + M, 0), G - 1) + 1];
-    r.z = bst[min(max(cm - 4 + M, 0), G - 1)];
-    r.w = bst[min(max(cm + 4 + M, 0), G - 1) + 1];
+    r.x = bst[a0];
+    r.y = bst[a1 + 1];
+    r.z = c == M ? r.x : (c <= 12 ? bst[b0] : 0);
+    r.w = c == M ? r.y : (c <= 12 ? bst[b1 + 1] : 0);
     return r;
 }
 
@@ -672,6 +718,7 @@ __device__ __forceinline__ void stage1_column(int s, int c, int4 rg, const VisRe
     const int cm = (c == 0) ? 0 : ((c == M) ? -M : -c);      // mirrored column
     const int d0 = rg.x, d1 = rg.y, m0 = rg.z, m1 = rg.w;
     const int nd = d1 - d0, ntot = nd + (m1 - m0);
+    const bool by_run = c <= 4 || c == M;   // direct or mirrored by the run it is in, else by its side
     // Threads that grid (whole waves; every condition on them is uniform).
     const int na = min(max((ntot / KR + 63) & ~63, NT), Sh::NX);
     if (t >= na) return;
@@ -687,9 +734,9 @@ __device__ __forceinline__ void stage1_column(int s, int c, int4 rg, const VisRe
     const float amax = fmaxf(0.5f * maxv, 1e-30f);   // |v| ES / 2 <= amax
     const float qs = 4096.0f / amax;
 
-    // Direct records (buckets cc-4..cc+4) then mirrored ones (cm-4..cm+4) in
-    // one numbering.  A column whose records do not fit the registers walks
-    // them in passes, the next pass's records loaded under this one's work.
+    // The two runs in one numbering.  A column whose records do not fit the
+    // registers walks them in passes, the next pass's records loaded under
+    // this one's work.
     const int step = KR * na;
     VisRec rn[KR];
     ColRec cr[KR];
@@ -704,10 +751,12 @@ __device__ __forceinline__ void stage1_column(int s, int c, int4 rg, const VisRe
 #pragma unroll
         for (int k = 0; k < KR; ++k) {
             const int n = base + k * na + t;
-            if (n < ntot)
-                cr[k] = prep_rec(rn[k], n < nd ? cc : cm, n >= nd, M);
-            else
+            if (n < ntot) {
+                const bool mirror = by_run ? n >= nd : (rn[k].col >> 1) + (rn[k].col & 1) < -3;   // b2 < 0
+                cr[k] = prep_rec(rn[k], mirror ? cm : cc, mirror, M);
+            } else {
                 cr[k].live = false;
+            }
         }
     };
     const bool resident = ntot <= step;
@@ -793,6 +842,11 @@ __device__ __forceinline__ void stage1_column(int s, int c, int4 rg, const VisRe
                     }
                     const float k = NB0 % RBS == 0 ? isc[j / RBS + q0 / RBS] : isc[u / RBS];
                     v[r] = make_float2((float)re * k, (float)im * k);
+                    // A radix-32 butterfly fills the registers: its inputs
+                    // are scaled here (fused into the butterfly, the scales
+                    // stayed live and spilled; a kernel that needs scratch
+                    // memory can start 6 us late).
+                    if constexpr (R0 == 32) asm("" : "+v"(v[r].x), "+v"(v[r].y));
                 }
             },
             [&](int j, const float2* v) {
@@ -832,9 +886,9 @@ __global__ __launch_bounds__(ColShape<G>::NX, ColShape<G>::waves) void k_stage1(
     const int S = (int)(gridDim.x / (G / 2 + 1));
     const int s = (int)(blockIdx.x % S);
     const int c = (int)(blockIdx.x / S);
-    // The bucket ranges do not depend on the metadata: both loads are in
-    // flight together.
-    const int4 rg = column_ranges<G>(bstart + (size_t)s * (G + 1), c);
+    // The runs do not depend on the metadata: both loads are in flight
+    // together.
+    const int4 rg = column_ranges<G>(bstart + (size_t)s * boff_row(G), c);
     const SnapMeta m = meta[s];
     if (c > m.rmax) return;
     stage1_column<G, KR>(s, c, rg, sorted, m, tw, kt, stride, smem, sc, isc);
@@ -1858,51 +1912,66 @@ const char* stage_name(int st)
     return (st >= 0 && st < kStCount) ? names[st] : "?";
 }
 
-hipError_t launch_reset(const InputView& in, const WorkView& w, const PlanTables& p, int S, float cell,
-                        const int* norm_n_dev, int norm_n_const, hipStream_t st)
+// Segments of a snapshot of up to n visibilities and their length: 2 or 4
+// visibilities per thread while that is at most 32 segments, then 8 up to 64
+// segments (a workgroup sorts 2048 visibilities in 7 us, 4096 in 16 and 8192
+// in 17 to 33, its FP64 and LDS atomics; every merging workgroup adds all
+// segments' offsets up); beyond 64 * 8192 visibilities, 64 equal segments.
+struct SegShape {
+    int vpt, chunk, nseg;
+};
+static SegShape seg_shape(int n)
 {
-    const int total = max(S * p.G, S * 2 * kMaxSlots);
-    hipLaunchKernelGGL(k_reset, dim3((total + 255) / 256), dim3(256), 0, st, in.vin, in.nvis, in.n_const,
-                       norm_n_dev, norm_n_const, w.meta, w.geom, w.hist, w.work, w.pmax, S, p.G, p.I, cell);
-    return hipGetLastError();
+    constexpr int B = kBinThreads;
+    SegShape q;
+    q.vpt = n <= 64 * B ? 2 : (n <= 128 * B ? 4 : (n <= kMaxSegs * 8 * B ? 8 : 0));
+    const int each = (n + kMaxSegs - 1) / kMaxSegs;
+    q.chunk = q.vpt > 0 ? q.vpt * B : (each + B - 1) / B * B;
+    q.nseg = max(1, (n + q.chunk - 1) / q.chunk);
+    return q;
 }
 
-hipError_t launch_bin(const InputView& in, const WorkView& w, const PlanTables& p, int S, int nmax,
-                      double scale, hipStream_t st)
+size_t bstart_words(int G) { return (size_t)boff_row(G); }
+
+template <class VT>
+static void bin_dispatch(const InputView& in, const BinView& out, int vpt, const PlanTables& p, int S, float cell,
+                         double scale, const int* norm_n_dev, int norm_n_const, hipStream_t st)
 {
-    if (nmax <= 0) return hipSuccess;
-    dim3 grid((nmax + kBinThreads * kBinVpt - 1) / (kBinThreads * kBinVpt), S);
-    const size_t lds = (size_t)p.G * sizeof(int);
-    switch (in.vis_type) {
-    case kVisF32:
-        hipLaunchKernelGGL(k_bin<float>, grid, dim3(kBinThreads), lds, st, in, w.rec, w.bkslot, w.hist, w.meta, p.G, scale);
-        break;
-    case kVisBF16:
-        hipLaunchKernelGGL(k_bin<__hip_bfloat16>, grid, dim3(kBinThreads), lds, st, in, w.rec, w.bkslot, w.hist, w.meta,
-                           p.G, scale);
-        break;
-    case kVisF16:
-        hipLaunchKernelGGL(k_bin<__half>, grid, dim3(kBinThreads), lds, st, in, w.rec, w.bkslot, w.hist, w.meta, p.G,
+    const dim3 grid(out.nseg + 1, S);
+    const size_t lds = (size_t)(bin_keys(p.G) + 1) * sizeof(int);
+    auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, grid, dim3(kBinThreads), lds, st, in, out, norm_n_dev, norm_n_const, p.G, p.I, cell,
                            scale);
-        break;
-    default:
-        return hipErrorInvalidValue;
+    };
+    switch (vpt) {
+    case 2: go(k_bin<VT, 2>); break;
+    case 4: go(k_bin<VT, 4>); break;
+    case 8: go(k_bin<VT, 8>); break;
+    default: go(k_bin<VT, 0>); break;
     }
-    return hipGetLastError();
 }
 
-hipError_t launch_scan(const WorkView& w, const PlanTables& p, int S, hipStream_t st)
+hipError_t launch_bin(const InputView& in, const WorkView& w, const PlanTables& p, int S, int nmax, float cell,
+                      double scale, const int* norm_n_dev, int norm_n_const, hipStream_t st)
 {
-    if (p.G > kMaxGrid) return hipErrorInvalidValue;   // a scan thread holds at most 12 counts
-    hipLaunchKernelGGL(k_scan, dim3(S), dim3(1024), 0, st, w.hist, w.bstart, p.G);
-    return hipGetLastError();
-}
-
-hipError_t launch_scatter(const WorkView& w, const PlanTables& p, int S, int nmax, hipStream_t st)
-{
-    if (nmax <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_scatter, dim3((nmax + 255) / 256, S), dim3(256), 0, st, w.rec, w.bkslot, w.bstart,
-                       w.sorted, w.meta, w.stride, p.G);
+    if (p.G > kMaxGrid) return hipErrorInvalidValue;
+    const SegShape q = seg_shape(nmax);
+    // The segments' offsets and extents are only read by the merge: they lie
+    // in each snapshot's corrected image and K tiles, which later stages write
+    // (64 (g/2 + 14) ints in I^2 floats, 192 ints in I (g/2 + 1) pairs: I >= 64).
+    const size_t plane = (size_t)p.I * p.I, tiles = (size_t)p.I * (p.M + 1) * 2;
+    const BinView v{w.rec,  w.sorted, reinterpret_cast<int*>(w.pre), reinterpret_cast<int*>(w.kt), w.bstart, w.meta,
+                    w.geom, w.pmax,   w.stride,                      plane,                        tiles,    q.nseg,
+                    q.chunk};
+    switch (in.vis_type) {
+    case kVisF32: bin_dispatch<float>(in, v, q.vpt, p, S, cell, scale, norm_n_dev, norm_n_const, st); break;
+    case kVisBF16: bin_dispatch<__hip_bfloat16>(in, v, q.vpt, p, S, cell, scale, norm_n_dev, norm_n_const, st); break;
+    case kVisF16: bin_dispatch<__half>(in, v, q.vpt, p, S, cell, scale, norm_n_dev, norm_n_const, st); break;
+    default: return hipErrorInvalidValue;
+    }
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess || q.nseg == 1) return e;
+    hipLaunchKernelGGL(k_merge, dim3(q.nseg, S), dim3(kBinThreads), 2 * (size_t)boff_row(p.G) * sizeof(int), st, v, p.G);
     return hipGetLastError();
 }
 

@@ -8,11 +8,10 @@
 //   [tables]  stage twiddles, C2R split factors and grid-correction tables of
 //             every image size whose work can fit (64..1024), and the window
 //             {0, 1, 2}; written once per device when the device is set up;
-//   [work]    the work buffers of one call (rec, bkslot, sorted, hist,
-//             bstart, meta, geom, kt, pre, img, work, pmax), laid out per
-//             call for its shape.
-// Kernels clear what must start at zero (histograms, metadata, max slots)
-// in their first launch, so the contents left by the previous call do not
+//   [work]    the work buffers of one call (rec, sorted, bstart, meta, geom,
+//             kt, pre, img, pmax), laid out per call for its shape.
+// Kernels clear what must start at zero (metadata, max slots) in their
+// first launch, so the contents left by the previous call do not
 // matter.  Calls on one device share the array: calls that overlap in time
 // on one GPU (different streams, or different host threads) race.
 #include "fip.h"
@@ -22,6 +21,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstring>
 #include <mutex>
 #include <string>
@@ -29,8 +29,8 @@
 namespace fip {
 namespace {
 
-// 64 MiB (67.1 MB): the 1024^2 workload with 130816 baselines needs 66.1 MB
-// of work buffers (records 22 MB, K tiles 18.9 MB, two image sets 25.2 MB).
+// 64 MiB (67.1 MB): the 1024^2 workload with 130816 baselines is admitted at
+// 66.1 MB (see admitted_bytes).
 constexpr size_t kScratchBytes = size_t(64) << 20;
 constexpr size_t kAlign = 256;
 constexpr int kMaxDevices = 64;
@@ -82,6 +82,21 @@ TableLayout table_layout()
     o = align_up(o + 3 * sizeof(int));
     L.end = o;
     return L;
+}
+
+// What a call is admitted by: 168 bytes per baseline (three snapshots' records
+// in and out of column order and their keys), the grid's counters and the
+// images, each part aligned.  The work buffers themselves take less; the
+// limit is the documented one and does not move with them.
+size_t admitted_bytes(const TableLayout& L, size_t nbl, const PlanTables& p)
+{
+    const size_t S = 3, I = (size_t)p.I, G = (size_t)p.G;
+    const size_t parts[] = {S * nbl * 24,       S * nbl * 8,   S * nbl * 24,  S * G * 4,           S * (G + 1) * 4,
+                            S * sizeof(SnapMeta), S * sizeof(SnapGeom), S * I * (p.M + 1) * 8, S * I * I * 4, S * I * I * 4,
+                            256,                pmax_words((int)S) * 4};
+    size_t o = L.end;
+    for (size_t b : parts) o = align_up(o + b);
+    return o;
 }
 
 struct DeviceScratch {
@@ -163,6 +178,7 @@ extern "C" int fip_pipe_device_noalloc(const float* vis_re, const float* vis_im,
             off[i] = o;
             o = align_up(o + sz[i]);
         }
+        o = std::max(o, admitted_bytes(L, num_baselines, p));
         if (o > kScratchBytes)
             return set_error(FIP_ERR_SIZE, "fip_pipe_device_noalloc: " + std::to_string(num_baselines) +
                                                " baselines at " + std::to_string(image_size) + "^2 need " +
@@ -178,17 +194,14 @@ extern "C" int fip_pipe_device_noalloc(const float* vis_re, const float* vis_im,
         p.corr = reinterpret_cast<float*>(base + L.slot[k].corr);
         WorkView w{};
         w.rec = reinterpret_cast<VisRec*>(base + off[0]);
-        w.bkslot = reinterpret_cast<int2*>(base + off[1]);
-        w.sorted = reinterpret_cast<VisRec*>(base + off[2]);
-        w.hist = reinterpret_cast<int*>(base + off[3]);
-        w.bstart = reinterpret_cast<int*>(base + off[4]);
-        w.meta = reinterpret_cast<SnapMeta*>(base + off[5]);
-        w.geom = reinterpret_cast<SnapGeom*>(base + off[6]);
-        w.kt = reinterpret_cast<float2*>(base + off[7]);
-        w.pre = reinterpret_cast<float*>(base + off[8]);
-        w.img = reinterpret_cast<float*>(base + off[9]);
-        w.work = reinterpret_cast<unsigned*>(base + off[10]);
-        w.pmax = reinterpret_cast<unsigned*>(base + off[11]);
+        w.sorted = reinterpret_cast<VisRec*>(base + off[1]);
+        w.bstart = reinterpret_cast<int*>(base + off[2]);
+        w.meta = reinterpret_cast<SnapMeta*>(base + off[3]);
+        w.geom = reinterpret_cast<SnapGeom*>(base + off[4]);
+        w.kt = reinterpret_cast<float2*>(base + off[5]);
+        w.pre = reinterpret_cast<float*>(base + off[6]);
+        w.img = reinterpret_cast<float*>(base + off[7]);
+        w.pmax = reinterpret_cast<unsigned*>(base + off[8]);
         w.stride = num_baselines;
         hipStream_t st = static_cast<hipStream_t>(stream);
         InputView in{vis_re, vis_im, bin, vin, nullptr, num_baselines, (int)num_baselines, FIP_VIS_F32};

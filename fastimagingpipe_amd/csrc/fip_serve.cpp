@@ -100,9 +100,11 @@ BatchLayout batch_layout(const fip_stream_config& c)
     return L;
 }
 
-// Fixed device bytes of one stream: work buffers and gathered inputs for
-// kServeBatch snapshots, the ring of images with their metadata and max
-// slots, the window table and the tLISI of kServeBatch windows.
+// Fixed device bytes a stream is admitted with: work buffers and gathered
+// inputs for kServeBatch snapshots, the ring of images with their metadata and
+// max slots, the window table and the tLISI of kServeBatch windows.  The
+// visibilities count 56 bytes each and the grid 8 bytes per row; the front end
+// holds 48 of the one and 2 of the other.
 size_t stream_fixed_bytes(const fip_stream_config& c, int ring)
 {
     const size_t I = c.image_size, N = c.num_baselines, B = kServeBatch;
@@ -160,7 +162,7 @@ struct SubStream {
     Tuning tu{};
     hipStream_t hs = nullptr;   // launch sequences
     hipStream_t cs = nullptr;   // input copies, so they run under the sequences
-    DevBuf rec, bkslot, sorted, hist, bstart, kt, pre, work;   // kServeBatch snapshots
+    DevBuf rec, sorted, bstart, kt, pre;                       // kServeBatch snapshots
     DevBuf batch_in;                                           // gathered inputs (BatchLayout)
     DevBuf img, meta, geom, pmax;                              // ring
     DevBuf win, out;
@@ -329,16 +331,13 @@ int launch_queued(fip_server* srv, SubStream& ss)
     char* dbase = srv->pool.as<char>();
     WorkView w;
     w.rec = ss.rec.as<VisRec>();
-    w.bkslot = ss.bkslot.as<int2>();
     w.sorted = ss.sorted.as<VisRec>();
-    w.hist = ss.hist.as<int>();
     w.bstart = ss.bstart.as<int>();
     w.meta = ss.meta.as<SnapMeta>() + r0;
     w.geom = ss.geom.as<SnapGeom>() + r0;
     w.kt = ss.kt.as<float2>();
     w.pre = ss.pre.as<float>();
     w.img = ss.img.as<float>() + (size_t)r0 * plane;
-    w.work = ss.work.as<unsigned>();
     w.pmax = ss.pmax.as<unsigned>() + pmax_index(r0, 0, 0);
     w.stride = N;
     InputView in;
@@ -561,9 +560,8 @@ int fip_server_create(const fip_stream_config* streams, int nstreams, int ring, 
             const size_t G = ssp->G, M = ssp->M, B = kServeBatch;
             for (auto pr : {std::make_pair(&ssp->rec, B * N * sizeof(VisRec)),
                             std::make_pair(&ssp->sorted, B * N * sizeof(VisRec)),
-                            std::make_pair(&ssp->bkslot, B * N * sizeof(int2)), std::make_pair(&ssp->hist, B * G * 4),
-                            std::make_pair(&ssp->bstart, B * (G + 1) * 4), std::make_pair(&ssp->kt, B * I * (M + 1) * 8),
-                            std::make_pair(&ssp->pre, B * I * I * 4), std::make_pair(&ssp->work, (size_t)256),
+                            std::make_pair(&ssp->bstart, B * bstart_words((int)G) * sizeof(int)),
+                            std::make_pair(&ssp->kt, B * I * (M + 1) * 8), std::make_pair(&ssp->pre, B * I * I * 4),
                             std::make_pair(&ssp->batch_in, batch_layout(ssp->cfg).bytes),
                             std::make_pair(&ssp->img, (size_t)ring * I * I * 4),
                             std::make_pair(&ssp->meta, (size_t)ring * sizeof(SnapMeta)),
@@ -576,8 +574,8 @@ int fip_server_create(const fip_stream_config* streams, int nstreams, int ring, 
             }
             // Every buffer is written once here, so the first snapshots after
             // creation do not pay the first use of freshly allocated memory.
-            for (DevBuf* b : {&ssp->rec, &ssp->bkslot, &ssp->sorted, &ssp->hist, &ssp->bstart, &ssp->kt, &ssp->pre,
-                              &ssp->work, &ssp->batch_in, &ssp->img, &ssp->meta, &ssp->geom, &ssp->pmax, &ssp->out}) {
+            for (DevBuf* b : {&ssp->rec, &ssp->sorted, &ssp->bstart, &ssp->kt, &ssp->pre, &ssp->batch_in, &ssp->img,
+                              &ssp->meta, &ssp->geom, &ssp->pmax, &ssp->out}) {
                 e = hipMemsetAsync(b->p, 0, b->cap, ssp->hs);
                 if (e != hipSuccess) return fail(hip_error(e, "hipMemsetAsync (server)"));
             }
@@ -775,7 +773,7 @@ void fip_server_destroy(fip_server* srv)
     srv->pcv.notify_one();
     if (srv->poller.joinable()) srv->poller.join();
     for (auto& ss : srv->streams) {
-        for (DevBuf* b : {&ss->rec, &ss->bkslot, &ss->sorted, &ss->hist, &ss->bstart, &ss->kt, &ss->pre, &ss->work,
+        for (DevBuf* b : {&ss->rec, &ss->sorted, &ss->bstart, &ss->kt, &ss->pre,
                           &ss->batch_in, &ss->img, &ss->meta, &ss->geom, &ss->pmax, &ss->win, &ss->out})
             b->release();
         if (ss->hs) (void)hipStreamDestroy(ss->hs);

@@ -32,11 +32,10 @@ import sys
 from collections import defaultdict
 
 # Kernel name pattern -> pipeline stage (the names the library's per-stage
-# event timing reports).
+# event timing reports, where the merge counts to "bin").
 STAGES = [
-    (r"k_reset", "reset"), (r"k_bin", "bin"), (r"k_scan", "scan"), (r"k_scatter", "scatter"),
-    (r"k_stage1", "grid_colfft"), (r"k_stage2", "row_c2r"), (r"k_splat<\d+, true>", "splat_trigger"),
-    (r"k_splat", "splat"), (r"k_trigger", "trigger"),
+    (r"k_bin", "bin"), (r"k_merge", "merge"), (r"k_stage1", "grid_colfft"), (r"k_stage2", "row_c2r"),
+    (r"k_splat<\d+, true>", "splat_trigger"), (r"k_splat", "splat"), (r"k_trigger", "trigger"),
 ]
 COPY_PATTERN = r"copyBuffer|Copy"
 
