@@ -79,6 +79,10 @@ struct SnapGeom {
                                  // model of the series along a group is within 5e-8 px: n' by its series
     int ccap;                    // upper bound on the sources whose splat reaches one pixel
     int pad;
+    double kratio;               // kappa / (1 - kappa)
+    // FP32 copies for the source loop: affine step per column, SIN shift, and
+    // the steps of the direction cosines l, m along a row.
+    float fm00, fm10, fsx, fsy, fdelta, fdl, fdn, padf;
 };
 
 enum VisType { kVisF32 = 0, kVisBF16 = 1, kVisF16 = 2 };
@@ -171,8 +175,8 @@ hipError_t launch_splat(const WorkView& w, const PlanTables& p, int S, const Tun
 // window's first two images img_a, img_b (already splatted) and its own
 // values, and stores its own image only if store; then the finish pass turns
 // the terms into the tLISI.  The same bits as launch_splat of s3 followed by
-// launch_trigger.  Fusable when the splat uses 64-pixel tiles and the
-// trigger tile is 32.  The terms live in w.kt, which the row pass is done with.
+// launch_trigger.  Fusable from 4096^2 on when the splat uses 64-pixel tiles
+// and the trigger tile is 32.  The terms live in w.kt, which the row pass is done with.
 bool splat_trigger_fusable(const PlanTables& p, const Tuning& tu, int tile);
 hipError_t launch_splat_trigger(const WorkView& w, const PlanTables& p, int s3, const float* img_a,
                                 const float* img_b, bool store, hipStream_t st);

@@ -86,10 +86,16 @@ __device__ __forceinline__ unsigned wave_max_u(unsigned v)
     const unsigned d = (unsigned)__builtin_amdgcn_readlane((int)v, 63);
     return max(max(a, b), max(c, d));
 }
-__device__ __forceinline__ int wave_sum_i(int v)
+// Inclusive sum over the lanes (all active) by DPP: shifts within rows of 16,
+// then each row's and each half's total added to the later ones.
+__device__ __forceinline__ int wave_scan_i(int v)
 {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true);   // row_shr:1
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, true);   // row_shr:2
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, true);   // row_shr:4
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, true);   // row_shr:8
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // row_bcast:15 into rows 1, 3
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // row_bcast:31 into rows 2, 3
     return v;
 }
 __device__ __forceinline__ float wave_sum_f(float v)
@@ -208,6 +214,15 @@ __device__ SnapGeom snap_geometry(const float* __restrict__ vin, int I, float ce
     const double qerr = 18.0 * dcol * dcol * dcol * fmax(fabs(gm.sx), fabs(gm.sy));
     gm.series = (rmax * rmax <= 0.01 && qerr <= 5e-8) ? 1 : 0;
     gm.pad = 0;
+    gm.kratio = kap / (1.0 - kap);
+    gm.fm00 = (float)gm.m00;
+    gm.fm10 = (float)gm.m10;
+    gm.fsx = (float)gm.sx;
+    gm.fsy = (float)gm.sy;
+    gm.fdelta = (float)gm.delta;
+    gm.fdl = -gm.fdelta * gm.fm00;
+    gm.fdn = gm.fdelta * gm.fm10;
+    gm.padf = 0.0f;
     return gm;
 }
 
@@ -1243,25 +1258,6 @@ __device__ __forceinline__ int mad_i24(int a, int b, int c)
     return r;
 }
 
-// FP32 copy of the geometry the splat needs per source.
-struct GeomF {
-    float m00, m10;   // affine step per source column
-    float sx, sy, delta;
-    int sin_on, series;
-};
-__device__ __forceinline__ GeomF geom_f(const SnapGeom& g)
-{
-    GeomF f;
-    f.m00 = (float)g.m00;
-    f.m10 = (float)g.m10;
-    f.sx = (float)g.sx;
-    f.sy = (float)g.sy;
-    f.delta = (float)g.delta;
-    f.sin_on = g.sin_on;
-    f.series = g.series;
-    return f;
-}
-
 // Exact integer accumulation: contributions (non-negative) are scaled by a
 // power of two, rounded half up to integers and summed as int32; the scale
 // keeps every pixel sum below 2^29 (plus half a unit per contribution), so
@@ -1336,19 +1332,20 @@ __global__ __launch_bounds__(256, 8) void k_splat(const float* __restrict__ pre,
     constexpr int CHK = 512;              // runs of 64 numbered groups per window
     static_assert(GN % 4 == 0 && (GN & (GN - 1)) == 0, "groups of 16-byte loads");
     static_assert((A * A) % 4 == 0, "16-byte clears");
+    static_assert(NW == 4 && ROW_CAP < NT, "one row per thread");
     __shared__ __align__(16) int acc[A * A];
-    __shared__ int rlo[ROW_CAP], rcnt[ROW_CAP], rofs[ROW_CAP + 1];
+    __shared__ int rlo[ROW_CAP], rofs[ROW_CAP + 1];
     __shared__ unsigned char crow[CHK];   // row in which each run of 64 starts
     __shared__ double qb[6];
     __shared__ int bb[4];
+    __shared__ __align__(16) int wtot[NW];
     __shared__ unsigned shm[NT / 64];
-    __shared__ unsigned smaxp;
+    __shared__ float sscale[2];
     const int s = s0 + (int)blockIdx.y;
     const int ntx = I / TS;
     const int tile = xcd_remap(blockIdx.x, gridDim.x);
     const int R0 = (tile / ntx) * TS, C0 = (tile % ntx) * TS;
-    const SnapGeom g = geom[s];
-    const SnapMeta m = meta[s];
+    const SnapGeom& g = geom[s];
     const int h = I / 2;
     const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
     if (tid == 0) {
@@ -1379,25 +1376,23 @@ __global__ __launch_bounds__(256, 8) void k_splat(const float* __restrict__ pre,
             // of (q1, q2), so |d(q) - d| <= kappa times that.
             const double res = fabs(o1 - t1) + fabs(o2 - t2);
             const double halfdiag = 0.7071067811865476 * (TS + 1);
-            const double dv = g.kappa * (halfdiag + res) / (1.0 - g.kappa) + 0.02;
+            const double dv = g.kratio * (halfdiag + res) + 0.02;
             ql1 = (double)(C0 - 1) - h - d1 - dv;
             qh1 = (double)(C0 + TS) - h - d1 + dv;
             ql2 = (double)(R0 - 1) - h - d2 - dv;
             qh2 = (double)(R0 + TS) - h - d2 + dv;
-            double mini = 1e300, maxi = -1e300, minj = 1e300, maxj = -1e300;
-            for (int k = 0; k < 4; ++k) {
-                const double c1 = (k & 1) ? qh1 : ql1, c2 = (k & 2) ? qh2 : ql2;
-                const double a = g.i00 * c1 + g.i01 * c2 + h, b = g.i10 * c1 + g.i11 * c2 + h;
-                mini = fmin(mini, a);
-                maxi = fmax(maxi, a);
-                minj = fmin(minj, b);
-                maxj = fmax(maxj, b);
-            }
-            // clamp before converting (degenerate V can give huge values)
-            mini = fmin(fmax(mini, -4.0), (double)I + 4.0);
-            maxi = fmin(fmax(maxi, -4.0), (double)I + 4.0);
-            minj = fmin(fmax(minj, -4.0), (double)I + 4.0);
-            maxj = fmin(fmax(maxj, -4.0), (double)I + 4.0);
+            // Extent of the inverse map over the box: each term's own extremes.
+            auto extent = [&](double ca, double cb, double& lo, double& hi) {
+                const double a0 = ca * ql1, a1 = ca * qh1, b0 = cb * ql2, b1 = cb * qh2;
+                lo = fmin(a0, a1) + fmin(b0, b1) + h;
+                hi = fmax(a0, a1) + fmax(b0, b1) + h;
+                // clamp before converting (degenerate V can give huge values)
+                lo = fmin(fmax(lo, -4.0), (double)I + 4.0);
+                hi = fmin(fmax(hi, -4.0), (double)I + 4.0);
+            };
+            double mini, maxi, minj, maxj;
+            extent(g.i00, g.i01, mini, maxi);
+            extent(g.i10, g.i11, minj, maxj);
             i0 = max(0, (int)floor(mini) - 1);
             i1 = min(I - 1, (int)ceil(maxi) + 1);
             j0 = max(0, (int)floor(minj) - 1);
@@ -1419,10 +1414,19 @@ __global__ __launch_bounds__(256, 8) void k_splat(const float* __restrict__ pre,
         for (int q = tid; q < A * A / 4; q += NT) a4[q] = make_int4(0, 0, 0, 0);
     }
     if (wid == 1) {
-        // Max of the corrected image from its slots (one per lane), while
-        // thread 0 computes the box.
-        const unsigned v = wave_max_u(*max_slot(pmax, s, 0, lane));
-        if (lane == 0) smaxp = v;
+        // While thread 0 computes the box: the max of the corrected image
+        // from its slots (one per lane), and the scale.  A pixel sums at most
+        // ccap contributions of at most max(pre)/N each (1/N of
+        // FIPkernels.cu:391); 2^k * ccap * max(pre)/N < 2^29.
+        const float maxp = __uint_as_float(wave_max_u(*max_slot(pmax, s, 0, lane)));
+        const float nf = (float)meta[s].norm_n;
+        int e = 0;
+        frexpf(fmaxf((float)g.ccap * (maxp / nf), 1e-30f), &e);
+        const int ks = min(29 - e, 120);
+        if (lane == 0) {
+            sscale[0] = ldexpf(1.0f, ks) / nf;
+            sscale[1] = ldexpf(1.0f, -ks);
+        }
     }
     __syncthreads();
     const int i0 = bb[0], i1 = bb[1], j0 = bb[2], j1 = bb[3];
@@ -1435,21 +1439,17 @@ __global__ __launch_bounds__(256, 8) void k_splat(const float* __restrict__ pre,
     // Without a curvature bound positions are not bounded a priori.
     const bool unbounded = g.curv < 0.0;
     const int H = j1 - j0 + 1;
-    // A pixel sums at most ccap contributions of at most max(pre)/N each
-    // (1/N of FIPkernels.cu:391); 2^k * ccap * max(pre)/N < 2^29.
-    int e = 0;
-    const unsigned maxp_bits = smaxp;
-    frexpf(fmaxf((float)g.ccap * (__uint_as_float(maxp_bits) / (float)m.norm_n), 1e-30f), &e);
-    const int ks = min(29 - e, 120);
-    const float vscale = ldexpf(1.0f, ks) / (float)m.norm_n;
-    const float iscale = ldexpf(1.0f, -ks);
-    const GeomF gf = geom_f(g);
+    const float vscale = sscale[0], iscale = sscale[1];
     const float* ps = pre + (size_t)s * I * I;
     for (int rb = 0; rb < H; rb += ROW_CAP) {
         const int nrow = min(ROW_CAP, H - rb);
-        // Per source row: the i range whose affine position lies in the q box.
-        for (int r = tid; r < nrow; r += NT) {
-            const double b = (double)(j0 + rb + r - h);
+        // Per source row, one thread: the i range whose affine position lies
+        // in the q box, in groups of GN pixels aligned to i % GN == 0, and
+        // their running count over the rows (DPP within a wave, the waves'
+        // totals through LDS).
+        int first = 0, cnt = 0;
+        if (tid < nrow) {
+            const double b = (double)(j0 + rb + tid - h);
             double alo = -1e300, ahi = 1e300;
             const double mA[2] = {g.m00, g.m10}, mB[2] = {g.m01, g.m11}, iA[2] = {qb[4], qb[5]};
             // The q box is read from LDS here rather than held in registers
@@ -1460,14 +1460,9 @@ __global__ __launch_bounds__(256, 8) void k_splat(const float* __restrict__ pre,
                 if (fabs(mA[k]) > 1e-12) {
                     // The range is widened by one pixel below, so a rounded
                     // reciprocal is as good as a division here.
-                    double x = (lo[k] - cst) * iA[k], y = (hi[k] - cst) * iA[k];
-                    if (x > y) {
-                        const double t = x;
-                        x = y;
-                        y = t;
-                    }
-                    alo = fmax(alo, x);
-                    ahi = fmin(ahi, y);
+                    const double x = (lo[k] - cst) * iA[k], y = (hi[k] - cst) * iA[k];
+                    alo = fmax(alo, fmin(x, y));
+                    ahi = fmin(ahi, fmax(x, y));
                 } else if (cst < lo[k] || cst > hi[k]) {
                     alo = 1e300;
                     ahi = -1e300;
@@ -1475,41 +1470,33 @@ __global__ __launch_bounds__(256, 8) void k_splat(const float* __restrict__ pre,
             }
             alo = fmax(alo, (double)(i0 - h - 2));
             ahi = fmin(ahi, (double)(i1 - h + 2));
-            int ia = i0, n = 0;
             if (alo <= ahi) {
-                ia = max(i0, (int)floor(alo + h) - 1);
-                n = max(0, min(i1, (int)ceil(ahi + h) + 1) - ia + 1);
+                const int ia = max(i0, (int)floor(alo + h) - 1);
+                const int n = max(0, min(i1, (int)ceil(ahi + h) + 1) - ia + 1);
+                first = ia / GN;
+                cnt = n > 0 ? ((ia + n - 1) / GN) - first + 1 : 0;
             }
-            // Groups of GN pixels aligned to i % GN == 0 that cover [ia, ia + n).
-            rlo[r] = ia / GN;
-            rcnt[r] = n > 0 ? ((ia + n - 1) / GN) - (ia / GN) + 1 : 0;
         }
+        const int incl = wave_scan_i(cnt);
+        if (lane == 63) wtot[wid] = incl;
         __syncthreads();
-        // Exclusive prefix of the per-row counts (wave 0).
-        if (wid == 0) {
-            int run = 0;
-            for (int b0 = 0; b0 < nrow; b0 += 64) {
-                const int r = b0 + lane;
-                const int v = r < nrow ? rcnt[r] : 0;
-                int x = v;
-#pragma unroll
-                for (int d = 1; d < 64; d <<= 1) {
-                    const int y = __shfl_up(x, d);
-                    if (lane >= d) x += y;
-                }
-                if (r < nrow) rofs[r] = run + x - v;
-                run += __shfl(x, 63);
-            }
-            if (lane == 0) rofs[nrow] = run;
+        int ofs = incl - cnt, total = 0;
+        {
+            const int4 w = *reinterpret_cast<const int4*>(wtot);
+            ofs += (wid > 0 ? w.x : 0) + (wid > 1 ? w.y : 0) + (wid > 2 ? w.z : 0);
+            total = __builtin_amdgcn_readfirstlane(w.x + w.y + w.z + w.w);
         }
-        __syncthreads();
-        const int total = rofs[nrow];
+        if (tid < nrow) {
+            rlo[tid] = first;
+            rofs[tid] = ofs;
+        }
+        if (tid == nrow) rofs[nrow] = total;
         for (int f0 = 0; f0 < total; f0 += CHK * 64) {
             const int nf = min(CHK * 64, total - f0);
             // Row of the first number of every run of 64 in [f0, f0 + nf).
-            for (int r = tid; r < nrow; r += NT) {
-                const int a = max(rofs[r], f0), b = min(rofs[r] + rcnt[r], f0 + nf);
-                for (int k = (a - f0 + 63) >> 6; (k << 6) < b - f0; ++k) crow[k] = (unsigned char)r;
+            if (tid < nrow) {
+                const int a = max(ofs, f0), b = min(ofs + cnt, f0 + nf);
+                for (int k = (a - f0 + 63) >> 6; (k << 6) < b - f0; ++k) crow[k] = (unsigned char)tid;
             }
             __syncthreads();
             // The source loop, specialised on the tile: EDGE for tiles on the
@@ -1568,8 +1555,8 @@ __global__ __launch_bounds__(256, 8) void k_splat(const float* __restrict__ pre,
                     // SIN direction cosines along the group: l = -cell (P1 - c0),
                     // m = cell (P2 - c0), c0 = I/2 + 1 (FIPkernels.cu:315-316),
                     // rounded once from FP64.
-                    const float l0 = (float)fma(-g.delta, q1d, g.delta), dl = -gf.delta * gf.m00;
-                    const float n0 = (float)fma(g.delta, q2d, -g.delta), dn = gf.delta * gf.m10;
+                    const float l0 = (float)fma(-g.delta, q1d, g.delta), dl = g.fdl;
+                    const float n0 = (float)fma(g.delta, q2d, -g.delta), dn = g.fdn;
                     // Series form: source k of the group lands at
                     // (Q1 + B1 k + C1 k^2, Q2 + B2 k + C2 k^2) relative to the
                     // origin, the affine step plus the quadratic Taylor model in
@@ -1577,7 +1564,7 @@ __global__ __launch_bounds__(256, 8) void k_splat(const float* __restrict__ pre,
                     // bounded in k_reset).  With r^2(k) = R0 + R1 k + R2 k^2 and
                     // the series f(x) = x/2 + x^2/8 + x^3/16 + 5x^4/128,
                     // n'(k) ~ f(R0) + f'(R0) R1 k + (f'(R0) R2 + f''(R0) R1^2 / 2) k^2.
-                    float Q1 = r1, B1 = gf.m00, C1 = 0.0f, Q2 = r2, B2 = gf.m10, C2 = 0.0f;
+                    float Q1 = r1, B1 = g.fm00, C1 = 0.0f, Q2 = r2, B2 = g.fm10, C2 = 0.0f;
                     if constexpr (ser == 1) {
                         const float R0 = fmaf(l0, l0, n0 * n0);
                         const float R1 = fmaf(l0, 2.0f * dl, n0 * (2.0f * dn));
@@ -1586,12 +1573,12 @@ __global__ __launch_bounds__(256, 8) void k_splat(const float* __restrict__ pre,
                         const float f1 = fmaf(R0, fmaf(R0, fmaf(R0, 0.15625f, 0.1875f), 0.25f), 0.5f);
                         const float f2h = fmaf(R0, fmaf(R0, 0.234375f, 0.1875f), 0.125f);
                         const float b = f1 * R1, c = fmaf(f1, R2, f2h * R1 * R1);
-                        Q1 = fmaf(gf.sx, f0, r1);
-                        Q2 = fmaf(gf.sy, f0, r2);
-                        B1 = fmaf(gf.sx, b, gf.m00);
-                        B2 = fmaf(gf.sy, b, gf.m10);
-                        C1 = gf.sx * c;
-                        C2 = gf.sy * c;
+                        Q1 = fmaf(g.fsx, f0, r1);
+                        Q2 = fmaf(g.fsy, f0, r2);
+                        B1 = fmaf(g.fsx, b, g.fm00);
+                        B2 = fmaf(g.fsy, b, g.fm10);
+                        C1 = g.fsx * c;
+                        C2 = g.fsy * c;
                     }
 #pragma unroll
                     for (int k = 0; k < GN; ++k) {
@@ -1600,21 +1587,21 @@ __global__ __launch_bounds__(256, 8) void k_splat(const float* __restrict__ pre,
                             o1 = k == 0 ? Q1 : fmaf((float)(k * k), C1, fmaf((float)k, B1, Q1));
                             o2 = k == 0 ? Q2 : fmaf((float)(k * k), C2, fmaf((float)k, B2, Q2));
                         } else {
-                            o1 = fmaf((float)k, gf.m00, r1);
-                            o2 = fmaf((float)k, gf.m10, r2);
-                            if (ser == 0 || gf.sin_on) {
+                            o1 = fmaf((float)k, g.fm00, r1);
+                            o2 = fmaf((float)k, g.fm10, r2);
+                            if (ser == 0 || g.sin_on) {
                                 const float l = fmaf((float)k, dl, l0), mm = fmaf((float)k, dn, n0);
                                 const float rr = l * l + mm * mm;
                                 float np = 0.0f;
-                                if (ser < 0 && gf.series) {
+                                if (ser < 0 && g.series) {
                                     // every source of the image has r^2 <= 0.01 (checked in k_reset)
                                     np = rr * fmaf(rr, fmaf(rr, fmaf(rr, 0.0390625f, 0.0625f), 0.125f), 0.5f);
                                 } else if (rr <= 1.0f) {
                                     // 1 - sqrt(1 - r^2) = r^2 / (1 + sqrt(1 - r^2)); hardware sqrt/rcp
                                     np = rr * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_sqrtf(1.0f - rr));
                                 }
-                                o1 = fmaf(gf.sx, np, o1);
-                                o2 = fmaf(gf.sy, np, o2);
+                                o1 = fmaf(g.fsx, np, o1);
+                                o2 = fmaf(g.fsy, np, o2);
                             }
                         }
                         bool fin = true;
@@ -1662,22 +1649,22 @@ __global__ __launch_bounds__(256, 8) void k_splat(const float* __restrict__ pre,
             if (unbounded) {
                 sources(std::true_type{}, std::true_type{}, std::integral_constant<int, -1>{});
             } else if (cedge || redge) {
-                if (gf.series)
+                if (g.series)
                     sources(std::true_type{}, std::false_type{}, Series{});
                 else
                     sources(std::true_type{}, std::false_type{}, Closed{});
             } else {
-                if (gf.series)
+                if (g.series)
                     sources(std::false_type{}, std::false_type{}, Series{});
                 else
                     sources(std::false_type{}, std::false_type{}, Closed{});
             }
             __syncthreads();   // crow is rewritten by the next window
         }
-        __syncthreads();   // rlo/rcnt are rewritten by the next row batch
+        if (rb + ROW_CAP < H) __syncthreads();   // rlo/rofs/wtot are rewritten by the next row batch
     }
     float* out = img + (size_t)s * I * I;
-    float lmax = 0.0f;
+    int lmax = 0;   // the scale is positive: the largest sum is the largest value
     // Four consecutive pixels per thread per pass, one 16-byte store; each
     // pass covers NT / (TS / 4) rows, and the pointers step by that.
     {
@@ -1691,12 +1678,12 @@ __global__ __launch_bounds__(256, 8) void k_splat(const float* __restrict__ pre,
             const float4 v = make_float4((float)a[0] * iscale, (float)a[1] * iscale, (float)a[2] * iscale,
                                          (float)a[3] * iscale);
             if (!TRIG || store_img) *reinterpret_cast<float4*>(o) = v;
-            lmax = fmaxf(lmax, fmaxf(fmaxf(v.x, v.y), fmaxf(v.z, v.w)));
+            lmax = max(max(lmax, max(a[0], a[1])), max(a[2], a[3]));
             a += RSTEP * A;
             o += (size_t)RSTEP * I;
         }
     }
-    const unsigned bmx = block_max_u<NT>(__float_as_uint(lmax), shm);
+    const unsigned bmx = block_max_u<NT>(__float_as_uint((float)lmax * iscale), shm);
     if (tid == 0) atomicMax(max_slot(pmax, s, 1, (int)(blockIdx.x % kMaxSlots)), bmx);
     if constexpr (TRIG) {
         // The trigger tile of this wave; lanes take the pixels, and add them
@@ -2071,7 +2058,11 @@ hipError_t launch_splat(const WorkView& w, const PlanTables& p, int S, const Tun
 
 bool splat_trigger_fusable(const PlanTables& p, const Tuning& tu, int tile)
 {
-    return tu.splat_tile >= 64 && p.I % 64 == 0 && tile == 32;
+    // Below 4096^2 the images stay in the caches between the launches and one
+    // splat over all snapshots with the trigger after it is shorter: 59 against
+    // 70 us per call at 1024^2 (8128 visibilities), 105 against 108 at 2048^2
+    // (32640), but 311 against 302 at 4096^2 (130816).
+    return p.I >= 4096 && tu.splat_tile >= 64 && p.I % 64 == 0 && tile == 32;
 }
 
 // The reduced trigger terms go to the K tiles' buffer, which the column and

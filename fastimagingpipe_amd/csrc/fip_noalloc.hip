@@ -92,7 +92,7 @@ size_t admitted_bytes(const TableLayout& L, size_t nbl, const PlanTables& p)
 {
     const size_t S = 3, I = (size_t)p.I, G = (size_t)p.G;
     const size_t parts[] = {S * nbl * 24,       S * nbl * 8,   S * nbl * 24,  S * G * 4,           S * (G + 1) * 4,
-                            S * sizeof(SnapMeta), S * sizeof(SnapGeom), S * I * (p.M + 1) * 8, S * I * I * 4, S * I * I * 4,
+                            S * 32,             S * 136,       S * I * (p.M + 1) * 8, S * I * I * 4, S * I * I * 4,
                             256,                pmax_words((int)S) * 4};
     size_t o = L.end;
     for (size_t b : parts) o = align_up(o + b);

@@ -105,13 +105,15 @@ BatchLayout batch_layout(const fip_stream_config& c)
 // max slots, the window table and the tLISI of kServeBatch windows.  The
 // visibilities count 56 bytes each and the grid 8 bytes per row; the front end
 // holds 48 of the one and 2 of the other.
+constexpr size_t kAdmitGeom = 136;   // of a snapshot's geometry
+
 size_t stream_fixed_bytes(const fip_stream_config& c, int ring)
 {
     const size_t I = c.image_size, N = c.num_baselines, B = kServeBatch;
     const size_t G = grid_size_for(I), M = G / 2;
     const size_t un = I / c.unit_size;
     const size_t work = N * sizeof(VisRec) * 2 + N * sizeof(int2) + G * 4 + (G + 1) * 4 + I * (M + 1) * 8 + I * I * 4;
-    const size_t ringb = (size_t)ring * (I * I * 4 + sizeof(SnapMeta) + sizeof(SnapGeom)) +
+    const size_t ringb = (size_t)ring * (I * I * 4 + sizeof(SnapMeta) + kAdmitGeom) +
                          pmax_words(ring) * sizeof(unsigned) + 3 * sizeof(int) * (size_t)ring;
     return B * work + batch_layout(c).bytes + ringb + B * un * un * 4 + 256;
 }
