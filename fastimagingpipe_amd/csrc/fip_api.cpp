@@ -660,12 +660,12 @@ int fip_autotune(size_t image_size, size_t num_baselines, float cell_size, int r
             return FIP_OK;
         };
         Tuning best = C->tuning(image_size);
-        double best_s1 = 1e300, best_s2 = 1e300, best_sp = 1e300;
+        double best_s1 = 1e300, best_sp = 1e300;
         const int records[3] = {2, 4, 8};
-        const int rows[3] = {1, 2, 4};
         const int tiles[2] = {32, 64};
         double tm[kStCount];
         best.persistent = 0;
+        best.stage2_rows = default_tuning(image_size).stage2_rows;
         for (int r : records) {
             Tuning t = best;
             t.stage1_records = r;
@@ -673,15 +673,6 @@ int fip_autotune(size_t image_size, size_t num_baselines, float cell_size, int r
             if (tm[kStGridFft] < best_s1) {
                 best_s1 = tm[kStGridFft];
                 best.stage1_records = r;
-            }
-        }
-        for (int r : rows) {
-            Tuning t = best;
-            t.stage2_rows = r;
-            if (int rc = measure(t, tm)) return rc;
-            if (tm[kStRowC2R] < best_s2) {
-                best_s2 = tm[kStRowC2R];
-                best.stage2_rows = r;
             }
         }
         for (int ts : tiles) {

@@ -245,11 +245,8 @@ Tuning default_tuning(size_t image)
     // 4096^2 and 2048^2 on MI355X (each thread's records stay resident up
     // to 1024 per column; heavier columns take further passes).
     t.stage1_records = 2;
-    // Rows per C2R workgroup: four rows of up to 768 points, two of 1536 and
-    // 3072 (each pair of rows read with one 16-byte load per K entry: 6%
-    // faster than four rows at 2048), one of 6144 (two rows of it hold
-    // 100 KB of LDS, one workgroup per CU).
-    t.stage2_rows = image <= 1024 ? 4 : (image <= 4096 ? 2 : 1);
+    // What the row pass does: two rows per workgroup, at 8192^2 one.
+    t.stage2_rows = image <= 4096 ? 2 : 1;
     // Up to 512^2 a 64-pixel tile leaves most CUs without a workgroup (16 per
     // image at 256^2) and each one's chain of loads and LDS atomics is the
     // launch: 32-pixel tiles take a call from 37 to 33 us at 256^2 and from 47
@@ -345,7 +342,7 @@ int imaging_sequence(Context* C, const PlanTables& p, const WorkView& w, const I
     const double scale = (double)cell * (double)p.G;
     FIP_STAGE(C, kStBin, st, launch_bin(in, w, p, S, nmax, cell, scale, norm_dev, norm_const, st));
     FIP_STAGE(C, kStGridFft, st, launch_stage1(w, p, S, tu, st));
-    FIP_STAGE(C, kStRowC2R, st, launch_stage2(w, p, S, tu, st));
+    FIP_STAGE(C, kStRowC2R, st, launch_stage2(w, p, S, st));
     const int ns = S - ndefer;
     if (ns > 0) FIP_STAGE(C, kStSplat, st, launch_splat(w, p, ns, tu, st));
     return FIP_OK;

@@ -210,16 +210,28 @@ constexpr unsigned band_mask()
 // whose bit is clear in MASK are taken as zeros and not read.
 template <int A, int B>
 struct BflyAB {
-    template <unsigned MASK = 0xffffffffu>
-    static __device__ __forceinline__ void run(float2* v)
+    // Inputs from fetch(std::integral_constant<int, r>).  Radix 32 holds 64
+    // registers of data: its inputs are fetched and its DFTs formed a few at a
+    // time, or the schedule spills at 80 registers (and a kernel that needs
+    // scratch memory starts 6 us late).
+    template <unsigned MASK, class F>
+    static __device__ __forceinline__ void run_from(float2* v, const F& fetch)
     {
         constexpr int R = A * B;
+        static_assert(A == 4 || MASK == 0xffffffffu, "pruned inputs need 4-point DFTs first");
         float2 x[B][A];
+        auto get = [&](auto r2) {
+            static_for<A>([&](auto r1) {
+                constexpr int r = B * decltype(r1)::value + decltype(r2)::value;
+                if constexpr ((MASK >> r) & 1u) x[r2][r1] = fetch(std::integral_constant<int, r>{});
+            });
+        };
+        constexpr int AHEAD = R == 32 ? 4 : B;   // DFTs' inputs in flight
+        static_for<AHEAD>(get);
         static_for<B>([&](auto r2) {
-            static_for<A>([&](auto r1) { x[r2][r1] = v[B * r1 + r2]; });
-            static_assert(A == 4 || MASK == 0xffffffffu, "pruned inputs need 4-point DFTs first");
+            constexpr int q = decltype(r2)::value;
+            if constexpr (R == 32) __builtin_amdgcn_sched_barrier(0);
             if constexpr (A == 4 && MASK != 0xffffffffu) {
-                constexpr int q = decltype(r2)::value;
                 constexpr unsigned m = ((MASK >> q) & 1u) | (((MASK >> (B + q)) & 1u) << 1) |
                                        (((MASK >> (2 * B + q)) & 1u) << 2) | (((MASK >> (3 * B + q)) & 1u) << 3);
                 bfly4_masked<m>(x[r2]);
@@ -227,13 +239,20 @@ struct BflyAB {
                 Bfly<A>::run(x[r2]);
             }
             static_for<A>([&](auto s1) { x[r2][s1] = rot<R, decltype(r2)::value * decltype(s1)::value>(x[r2][s1]); });
+            if constexpr (q + AHEAD < B) get(std::integral_constant<int, q + AHEAD>{});
         });
         static_for<A>([&](auto s1) {
             float2 y[B];
             static_for<B>([&](auto r2) { y[r2] = x[r2][s1]; });
+            if constexpr (R == 32) __builtin_amdgcn_sched_barrier(0);
             Bfly<B>::run(y);
             static_for<B>([&](auto s2) { v[s1 + A * s2] = y[s2]; });
         });
+    }
+    template <unsigned MASK = 0xffffffffu>
+    static __device__ __forceinline__ void run(float2* v)
+    {
+        run_from<MASK>(v, [&](auto r) { return v[decltype(r)::value]; });
     }
 };
 template <> struct Bfly<6> : BflyAB<2, 3> {};
@@ -245,6 +264,7 @@ template <> struct Bfly<32> : BflyAB<4, 8> {};
 // Butterfly of radix R with zero inputs outside MASK, where the radix has a
 // pruned form (4-point DFTs first); the others read every input.
 constexpr bool bfly_prunes(int R) { return R == 12 || R == 16 || R == 32; }
+constexpr bool bfly_fetches(int R) { return R == 32; }
 template <int R, unsigned MASK>
 __device__ __forceinline__ void bfly_masked(float2* v)
 {
@@ -310,21 +330,32 @@ template <int Ns, int R> struct StoreOff {
     static constexpr __host__ __device__ int at(int r) { return small ? r * Ns : r * Ns + ((r * Ns) >> 5); }
 };
 
+// Input j + r N/R of a butterfly from the padded LDS array buf.
+template <int N, int R>
+__device__ __forceinline__ float2 lds_input(const float2* buf, int j, int r)
+{
+    constexpr int NB = N / R;
+    if constexpr (LoadOff<NB>::ok) return (buf + lds_pad(j))[LoadOff<NB>::at(r)];
+    return buf[lds_pad(j + r * NB)];
+}
+
 // One Stockham stage of radix R with Ns = product of earlier radices.
 // tw points at this stage's twiddles laid out [r-1][k], k < Ns.  Threads
 // t >= NT of a larger workgroup (whole waves, NT a multiple of 64) take no
 // butterfly but reach the barriers.
 //
-// The first stage's inputs come from load(j, v): v[r] = x[j + r N/R], and the
-// last stage's outputs go to store(j, v): X[j + r N/R] = v[r] (there Ns = N/R,
+// The first stage's inputs come from load(j, r) = x[j + r N/R], and the last
+// stage's outputs go to store(j, v): X[j + r N/R] = v[r] (there Ns = N/R,
 // so j is the output index's low part); every other exchange goes through buf.
 // LoadLds / StoreLds say whether load reads or store writes LDS that this
 // transform (or its caller's data in the same memory) uses, which needs a
 // barrier between the reads and the writes.  MASK: the first stage's inputs
-// that can be non-zero (load need not set the others).
+// that can be non-zero (the others are not loaded).  A store with a
+// prefetch(t) member has it called ahead of the last stage (one butterfly per
+// thread there).
 template <class P, int S, int Ns, int TwOff, bool LoadLds, bool StoreLds, unsigned MASK, class Load, class Store>
 __device__ __forceinline__ void fft_stage(float2* __restrict__ buf, const float2* __restrict__ tw, int t,
-                                          const Load& load, const Store& store)
+                                          Load& load, Store& store)
 {
     constexpr int N = P::n, NT = P::nt, R = P::radix[S];
     constexpr bool first = S == 0, last = S + 1 == P::nstages;
@@ -337,7 +368,8 @@ __device__ __forceinline__ void fft_stage(float2* __restrict__ buf, const float2
         float2 v[BPT][R];
         // Twiddles do not depend on the data: issue their (L1/L2-resident)
         // loads before the LDS loads and the barrier so their latency is
-        // hidden.
+        // hidden; likewise what store needs.
+        if constexpr (last && requires { store.prefetch(t); }) store.prefetch(t);
         float2 w[BPT][R > 1 ? R - 1 : 1];
         if (Ns > 1) {
 #pragma unroll
@@ -352,15 +384,16 @@ __device__ __forceinline__ void fft_stage(float2* __restrict__ buf, const float2
         for (int b = 0; b < BPT; ++b) {
             const int j = t + b * NT;
             if (all || (t < NT && j < NB)) {
-                if constexpr (first) {
-                    load(j, v[b]);
-                } else if constexpr (LoadOff<NB>::ok) {
-                    const float2* p = buf + lds_pad(j);
+                if constexpr (first && bfly_fetches(R)) {
+                    Bfly<R>::template run_from<MASK>(
+                        v[b], [&](auto r) { return load(j, decltype(r)::value); });
+                } else if constexpr (first) {
 #pragma unroll
-                    for (int r = 0; r < R; ++r) v[b][r] = p[LoadOff<NB>::at(r)];
+                    for (int r = 0; r < R; ++r)
+                        if ((MASK >> r) & 1u) v[b][r] = load(j, r);
                 } else {
 #pragma unroll
-                    for (int r = 0; r < R; ++r) v[b][r] = buf[lds_pad(j + r * NB)];
+                    for (int r = 0; r < R; ++r) v[b][r] = lds_input<N, R>(buf, j, r);
                 }
             }
         }
@@ -374,7 +407,7 @@ __device__ __forceinline__ void fft_stage(float2* __restrict__ buf, const float2
 #pragma unroll
                     for (int r = 1; r < R; ++r) v[b][r] = cmul(v[b][r], w[b][r - 1]);
                 }
-                bfly_masked<R, first ? MASK : 0xffffffffu>(v[b]);
+                if constexpr (!(first && bfly_fetches(R))) bfly_masked<R, first ? MASK : 0xffffffffu>(v[b]);
                 if constexpr (last) {
                     store(j, v[b]);
                 } else {
@@ -421,8 +454,8 @@ __device__ __forceinline__ void fft_stage(float2* __restrict__ buf, const float2
 // Inverse FFT of length N between load and store (see fft_stage) with buf
 // (lds_len(N) entries) for the exchanges.
 template <int N, bool LoadLds, bool StoreLds, unsigned MASK = 0xffffffffu, class Load, class Store>
-__device__ __forceinline__ void fft_inverse_io(float2* buf, const float2* __restrict__ tw, int t, const Load& load,
-                                               const Store& store)
+__device__ __forceinline__ void fft_inverse_io(float2* buf, const float2* __restrict__ tw, int t, Load&& load,
+                                               Store&& store)
 {
     fft_stage<FftPlan<N>, 0, 1, 0, LoadLds, StoreLds, MASK>(buf, tw, t, load, store);
 }
@@ -437,10 +470,7 @@ __device__ __forceinline__ void fft_inverse(float2* buf, const float2* __restric
     constexpr int R0 = P::radix[0], R1 = P::radix[P::nstages - 1];
     fft_inverse_io<N, true, true>(
         buf, tw, t,
-        [&](int j, float2* v) {
-#pragma unroll
-            for (int r = 0; r < R0; ++r) v[r] = buf[lds_pad(j + r * (N / R0))];
-        },
+        [&](int j, int r) { return lds_input<N, R0>(buf, j, r); },
         [&](int j, const float2* v) {
 #pragma unroll
             for (int r = 0; r < R1; ++r) buf[lds_pad(j + r * (N / R1))] = v[r];

@@ -137,7 +137,7 @@ struct BinView {
 // Tunable launch parameters (the autotuner picks among these).
 struct Tuning {
     int stage1_records;   // gridding records per thread held in registers (2, 4, 8)
-    int stage2_rows;    // image rows per stage-2 workgroup (1, 2, 4)
+    int stage2_rows;    // accepted and kept; the row pass has one launch form
     int splat_tile;     // target tile edge of the splat (32 or 64)
     int persistent;     // accepted and kept; the column kernel has one launch form
 };
@@ -164,8 +164,7 @@ hipError_t launch_bin(const InputView& in, const WorkView& w, const PlanTables& 
                       double scale, const int* norm_n_dev, int norm_n_const, hipStream_t st);
 hipError_t launch_stage1(const WorkView& w, const PlanTables& p, int S, const Tuning& tu,
                          hipStream_t st);
-hipError_t launch_stage2(const WorkView& w, const PlanTables& p, int S, const Tuning& tu,
-                         hipStream_t st);
+hipError_t launch_stage2(const WorkView& w, const PlanTables& p, int S, hipStream_t st);
 // Splat of snapshots 0..S-1 of the view.
 hipError_t launch_splat(const WorkView& w, const PlanTables& p, int S, const Tuning& tu,
                         hipStream_t st);

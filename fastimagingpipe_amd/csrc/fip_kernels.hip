@@ -9,10 +9,10 @@
 //   stage1   per uv column c >= 0: deterministic integer LDS gridding of the
 //            Hermitian-folded grid column (FIPkernels.cu:197-245) and its
 //            length-g inverse FFT along the row axis, cropped to I rows
-//   stage2   per image row: complex-to-real length-g inverse FFT along the
-//            column axis via a length-g/2 complex FFT, cropped, |.| and the
-//            separable grid correction -> corrected image
-//            (FIPkernels.cu:256-287), plus its maximum (spread slots)
+//   stage2   per two image rows: complex-to-real length-g inverse FFT along the
+//            column axis, cropped, |.| and the separable grid correction ->
+//            corrected image (FIPkernels.cu:256-287), plus its maximum (spread
+//            slots)
 //   splat    per target tile: affine + SIN re-projection (FP64 per group of
 //            sources, FP32 within it) and the bilinear forward splat
 //            accumulated exactly in int32 LDS, plus the image maximum
@@ -844,25 +844,20 @@ __device__ __forceinline__ void stage1_column(int s, int c, int4 rg, const VisRe
         constexpr unsigned mask = band_mask<R0, nz, nz>();
         fft_inverse_io<G, true, false, mask>(
             fb, tw, t,
-            [&](int j, float2* v) {
+            [&](int j, int r) {
+                const int q0 = NB0 * ((r + R0 / 2) % R0), u = j + q0;
+                int re = 0, im = 0;
 #pragma unroll
-                for (int r = 0; r < R0; ++r) {
-                    if (!((mask >> r) & 1u)) continue;
-                    const int q0 = NB0 * ((r + R0 / 2) % R0), u = j + q0;
-                    int re = 0, im = 0;
-#pragma unroll
-                    for (int q = 0; q < NC; ++q) {
-                        re += col[u * NC + q];
-                        im += col[(G + u) * NC + q];
-                    }
-                    const float k = NB0 % RBS == 0 ? isc[j / RBS + q0 / RBS] : isc[u / RBS];
-                    v[r] = make_float2((float)re * k, (float)im * k);
-                    // A radix-32 butterfly fills the registers: its inputs
-                    // are scaled here (fused into the butterfly, the scales
-                    // stayed live and spilled; a kernel that needs scratch
-                    // memory can start 6 us late).
-                    if constexpr (R0 == 32) asm("" : "+v"(v[r].x), "+v"(v[r].y));
+                for (int q = 0; q < NC; ++q) {
+                    re += col[u * NC + q];
+                    im += col[(G + u) * NC + q];
                 }
+                const float k = NB0 % RBS == 0 ? isc[j / RBS + q0 / RBS] : isc[u / RBS];
+                float2 x = make_float2((float)re * k, (float)im * k);
+                // Scaled here, not in the radix-32 butterfly's own multiply-adds:
+                // those kept the scales in registers and spilled.
+                if constexpr (R0 == 32) asm("" : "+v"(x.x), "+v"(x.y));
+                return x;
             },
             [&](int j, const float2* v) {
                 float2* o = ks + (size_t)(j / kKTile) * (M + 1) * kKTile + (j % kKTile);
@@ -911,154 +906,6 @@ __global__ __launch_bounds__(ColShape<G>::NX, ColShape<G>::waves) void k_stage1(
 
 // ---------------------------------------------------------------- stage 2
 
-// Gather and C2R split of ROWS image rows in one pass: Z[k] = E[k] + i O[k],
-// E = K[k] + K~[k+M], O = (K[k] - K~[k+M]) e^{2 pi i k/G},
-// K~[k+M] = conj(K[M-k]) (k > 0), K[M] (k = 0).  A thread takes the pairs
-// (p, M-p) of every row, reads K[p] and K[M-p] straight from the K tiles
-// (zero beyond cmax) and writes Z[p], Z[M-p]; the pairs cover every index
-// 0..M-1.  wpost[M - p] = -conj(wpost[p]).  The loads of all the thread's
-// pairs are issued together (load), then paired into LDS (store).
-template <int M, int ROWS>
-struct C2RGather {
-    static constexpr int NT = FftPlan<M>::nt * ROWS;          // threads of the workgroup
-    static constexpr int PB = (M / 2 + NT) / NT;               // pairs per thread: ceil((M/2+1)/NT)
-    float2 a[PB][ROWS], b[PB][ROWS], wv[PB];
-
-    // kt0: K tile run of the first row of the group (row y0 of its snapshot).
-    __device__ __forceinline__ void load(const float2* __restrict__ kt0, const float2* __restrict__ wpost,
-                                         int cmax, int tid)
-    {
-#pragma unroll
-        for (int u = 0; u < PB; ++u) {
-            const int p = tid + u * NT;
-            const bool ok = p <= M / 2;
-            wv[u] = ok ? wpost[p] : make_float2(0.0f, 0.0f);
-            if constexpr (ROWS % 2 == 0) {
-                // Two rows per 16-byte load: y0 is a multiple of ROWS, so the
-                // pair is 16-byte aligned inside its 64-byte tile run.
-#pragma unroll
-                for (int r = 0; r < ROWS; r += 2) {
-                    const float4 va = (ok && p <= cmax)
-                                          ? *reinterpret_cast<const float4*>(kt0 + (size_t)p * kKTile + r)
-                                          : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-                    const float4 vb = (ok && M - p <= cmax)
-                                          ? *reinterpret_cast<const float4*>(kt0 + (size_t)(M - p) * kKTile + r)
-                                          : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-                    a[u][r] = make_float2(va.x, va.y);
-                    a[u][r + 1] = make_float2(va.z, va.w);
-                    b[u][r] = make_float2(vb.x, vb.y);
-                    b[u][r + 1] = make_float2(vb.z, vb.w);
-                }
-            } else {
-#pragma unroll
-                for (int r = 0; r < ROWS; ++r) {
-                    a[u][r] = (ok && p <= cmax) ? kt0[(size_t)p * kKTile + r] : make_float2(0.0f, 0.0f);
-                    b[u][r] = (ok && M - p <= cmax) ? kt0[(size_t)(M - p) * kKTile + r] : make_float2(0.0f, 0.0f);
-                }
-            }
-        }
-    }
-
-    __device__ __forceinline__ void store(float2* zb, int tid) const
-    {
-        constexpr int L = lds_len(M + 1);
-#pragma unroll
-        for (int u = 0; u < PB; ++u) {
-            const int p = tid + u * NT;
-            if (p > M / 2) break;
-#pragma unroll
-            for (int r = 0; r < ROWS; ++r) {
-                float2* zr = zb + r * L;
-                const float2 av = a[u][r], bv = b[u][r];
-                if (p == 0) {
-                    zr[lds_pad(0)] = cadd(cadd(av, bv), cmul_i(csub(av, bv)));
-                } else {
-                    const float2 kp = cconj(bv);   // K~[p+M]
-                    zr[lds_pad(p)] = cadd(cadd(av, kp), cmul_i(cmul(csub(av, kp), wv[u])));
-                    if (p != M - p) {
-                        const float2 km = cconj(av);   // K~[M-p+M]
-                        const float2 wm = make_float2(-wv[u].x, wv[u].y);
-                        zr[lds_pad(M - p)] = cadd(cadd(bv, km), cmul_i(cmul(csub(bv, km), wm)));
-                    }
-                }
-            }
-        }
-    }
-};
-
-// The same gather for a K band narrower than half the row (cmax < M/2), the
-// usual case (the uv coverage spans under half the Nyquist band): every
-// K[M-p] of a pair is then zero, so only K[p] is read and the pairing keeps
-// the operations on the non-zero terms, Z[p] = K[p] + i K[p] w_p and
-// Z[M-p] = conj(K[p]) + i (-conj(K[p])) w_{M-p}.  Pair blocks that start
-// beyond cmax only write zeros.
-template <int M, int ROWS>
-struct C2RGatherLow {
-    static constexpr int NT = FftPlan<M>::nt * ROWS;
-    static constexpr int PB = (M / 2 + NT) / NT;
-    float2 a[PB][ROWS], wv[PB];
-
-    __device__ __forceinline__ void load(const float2* __restrict__ kt0, const float2* __restrict__ wpost,
-                                         int cmax, int tid)
-    {
-#pragma unroll
-        for (int u = 0; u < PB; ++u) {
-            if (u * NT > cmax) break;
-            const int p = tid + u * NT;
-            const bool ok = p <= cmax;
-            wv[u] = ok ? wpost[p] : make_float2(0.0f, 0.0f);
-            if constexpr (ROWS % 2 == 0) {
-#pragma unroll
-                for (int r = 0; r < ROWS; r += 2) {
-                    const float4 va = ok ? *reinterpret_cast<const float4*>(kt0 + (size_t)p * kKTile + r)
-                                         : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-                    a[u][r] = make_float2(va.x, va.y);
-                    a[u][r + 1] = make_float2(va.z, va.w);
-                }
-            } else {
-#pragma unroll
-                for (int r = 0; r < ROWS; ++r)
-                    a[u][r] = ok ? kt0[(size_t)p * kKTile + r] : make_float2(0.0f, 0.0f);
-            }
-        }
-    }
-
-    __device__ __forceinline__ void store(float2* zb, int cmax, int tid) const
-    {
-        constexpr int L = lds_len(M + 1);
-#pragma unroll
-        for (int u = 0; u < PB; ++u) {
-            const int p = tid + u * NT;
-            if (p > M / 2) break;
-            if (u * NT > cmax) {
-#pragma unroll
-                for (int r = 0; r < ROWS; ++r) {
-                    float2* zr = zb + r * L;
-                    zr[lds_pad(p)] = make_float2(0.0f, 0.0f);
-                    zr[lds_pad(M - p)] = make_float2(0.0f, 0.0f);
-                }
-                continue;
-            }
-#pragma unroll
-            for (int r = 0; r < ROWS; ++r) {
-                float2* zr = zb + r * L;
-                const float2 av = a[u][r];
-                if (p == 0) {
-                    zr[lds_pad(0)] = cadd(av, cmul_i(av));
-                } else {
-                    zr[lds_pad(p)] = cadd(av, cmul_i(cmul(av, wv[u])));
-                    if (p != M - p) {
-                        const float2 km = cconj(av);
-                        const float2 nk = make_float2(-av.x, av.y);   // -conj(K[p])
-                        const float2 wm = make_float2(-wv[u].x, wv[u].y);
-                        zr[lds_pad(M - p)] = cadd(km, cmul_i(cmul(nk, wm)));
-                    }
-                }
-            }
-        }
-    }
-};
-
 // First K tile run of image row y0 of snapshot s.
 template <int M>
 __device__ __forceinline__ const float2* c2r_rows(const float2* __restrict__ kt, int s, int y0, int I)
@@ -1067,153 +914,212 @@ __device__ __forceinline__ const float2* c2r_rows(const float2* __restrict__ kt,
     return ks + (size_t)(y0 / kKTile) * (M + 1) * kKTile + (y0 % kKTile);
 }
 
-// d[2n] = Re z[n], d[2n+1] = Im z[n]; crop x in [-h, h), |.| and the grid
-// correction 1/(c(|x|) c(|y|) norm^2) (FIPkernels.cu:256-287) for all ROWS
-// rows of a workgroup at once:
-// each thread takes whole columns, so a column's correction factor is loaded
-// once for all the rows; returns the thread's max.  out0: output row of the
-// workgroup's first row.
-template <int M, int ROWS, int NTB>
-__device__ __forceinline__ float c2r_output_rows(const float2* zb, const float* __restrict__ corr, float* out0,
-                                                 int y0, int I, int tid)
-{
-    constexpr int G = 2 * M;
-    constexpr int L = lds_len(M + 1);
-    const int h = I / 2;
-    float lmax = 0.0f;
-    // Row correction of each row (the grid correction is separable).
-    float cy[ROWS];
+// Grid correction and output of two image rows from the transform's registers:
+// real part the first row, imaginary part the second.  Element n of the
+// transform is image column x = n (n < h) or n - g (n >= g - h), offset by h;
+// with h = g/3 and the last radix a multiple of 3 the crop drops whole outputs
+// of each butterfly.  |.| and 1/(c(|x|) c(|y|) norm^2) (FIPkernels.cu:256-287).
+template <int G>
+struct RowStore {
+    static constexpr int I = 2 * G / 3, h = I / 2;
+    static constexpr int R = FftPlan<G>::radix[FftPlan<G>::nstages - 1], NS = G / R, KEEP = R / 3;
+    static_assert(R % 3 == 0 && 3 * h == G, "whole outputs are cropped");
+    const float* __restrict__ corr;
+    float* out;      // first row
+    float cy0, cy1;
+    float lmax;      // of this thread's butterfly
+    float cv[2 * KEEP];
+
+    __device__ __forceinline__ void prefetch(int j)
+    {
+        lmax = 0.0f;
+        if (j >= NS) return;
 #pragma unroll
-    for (int r = 0; r < ROWS; ++r) {
-        const int y = y0 + r - h;
-        cy[r] = corr[y < 0 ? -y : y];
-    }
-    for (int c0 = tid; c0 < I; c0 += 4 * NTB) {
-        float cv[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int x = c0 + u * NTB - h;
-            cv[u] = (c0 + u * NTB < I) ? corr[x < 0 ? -x : x] : 0.0f;
+        for (int k = 0; k < KEEP; ++k) {
+            cv[k] = corr[NS * k + j];                                  // x = n
+            cv[KEEP + k] = corr[(G - NS * (2 * KEEP + k)) - j];        // x = n - g
         }
+    }
+    __device__ __forceinline__ void operator()(int j, const float2* v)
+    {
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int col = c0 + u * NTB;
-            if (col < I) {
-                const int x = col - h;
-                const int mm = x < 0 ? x + G : x;
+        for (int k = 0; k < 2 * KEEP; ++k) {
+            const float2 z = v[k < KEEP ? k : k + KEEP];
+            float* o = out + (k < KEEP ? h + NS * k : h + NS * (k + KEEP) - G) + j;
+            const float a = fabsf(z.x) * (cv[k] * cy0), b = fabsf(z.y) * (cv[k] * cy1);
+            // Non-temporal stores: 122-127 -> 108-109 us at 4096^2 for the row
+            // pass, and the splat that reads these images next is not slower.
+            __builtin_nontemporal_store(a, o);
+            __builtin_nontemporal_store(b, o + I);
+            lmax = fmaxf(lmax, fmaxf(a, b));
+        }
+    }
+};
+
+// Two image rows in one complex transform of length g: with Z[n] = K1[n] + i K2[n]
+// over the whole Hermitian band (K[-n] = conj(K[n])), its real and imaginary
+// parts are the two rows.  Each K entry of the pair is one 16-byte load, there
+// is no split factor, the band (|n| <= cmax) leaves first-stage inputs out, and
+// the crop leaves from the registers: one LDS pass in, two exchanges.  (A
+// real transform per row as a complex one of half the length took its pairing
+// factors, a full-length gather and two more LDS passes.)  K[0] and K[g/2] are
+// real for exact data; their real parts are taken, so no row leaks into the
+// other.
+//
+// Three images, before and after: 103.8 -> 94.7 us at 4096^2 (339 MB, 3.6 TB/s),
+// 26 -> 24 at 2048^2.  Arithmetic and LDS turns of the waves (52 us of vector
+// instructions) and the start of each workgroup on cold loads bound it now.
+// Next rows' K loads held across the transform (a persistent loop) took 112
+// registers instead of 70, with fewer waves and no gain.
+//
+// Workgroup: one row pair.  (Two pairs per workgroup: 3.7 -> 4.3 us at 128^2,
+// 4.1 -> 4.3 at 256^2, within 6% either way from 512^2 to 2048^2, and the
+// compiler contracts the two bodies differently, so the bits differ.)
+template <int G>
+__global__ __launch_bounds__(FftPlan<G>::nt, G >= 6144 ? 6 : 2) void k_stage2(
+    const float2* __restrict__ kt, const SnapMeta* __restrict__ meta, unsigned* __restrict__ pmax,
+    const float2* __restrict__ tw, const float* __restrict__ corr, float* __restrict__ pre)
+{
+    constexpr int M = G / 2, I = 2 * G / 3, h = I / 2, NT = FftPlan<G>::nt;
+    constexpr int R0 = FftPlan<G>::radix[0], NB0 = G / R0;
+    __shared__ float2 z[lds_len(G)];
+    __shared__ unsigned shm[NT / 64];
+    const int s = blockIdx.y, t = threadIdx.x;
+    const int y0 = xcd_remap(blockIdx.x, gridDim.x) * 2;
+    const int cmax = min(meta[s].rmax, M);
+    const float2* k0 = c2r_rows<M>(kt, s, y0, I);
+    RowStore<G> rows;
+    rows.corr = corr;
+    rows.out = pre + (size_t)s * I * I + (size_t)y0 * I;
+    rows.cy0 = corr[y0 < h ? h - y0 : y0 - h];
+    rows.cy1 = corr[y0 + 1 < h ? h - y0 - 1 : y0 + 1 - h];
+    if (RowStore<G>::NS < NT) rows.lmax = 0.0f;   // threads without a last butterfly
+    // NZ: first-stage inputs 0..NZ-1 and R0-NZ..R0-1, |n| <= NZ NB0.
+    auto run = [&](auto NZ) {
+        constexpr int nz = decltype(NZ)::value, L = nz * NB0, NIT = (L + NT - 1) / NT;
+        auto pair = [&](int p) {
+            return p <= cmax ? *reinterpret_cast<const float4*>(k0 + (size_t)p * kKTile)
+                             : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        };
+        float4 k[NIT];
 #pragma unroll
-                for (int r = 0; r < ROWS; ++r) {
-                    const float2 v = zb[r * L + lds_pad(mm >> 1)];
-                    const float val = fabsf((mm & 1) ? v.y : v.x) * (cv[u] * cy[r]);
-                    // Non-temporal store: 122-127 -> 108-109 us at 4096^2, and
-                    // the splat that reads these images next is not slower.
-                    __builtin_nontemporal_store(val, out0 + (size_t)r * I + col);
-                    lmax = fmaxf(lmax, val);
+        for (int u = 0; u < NIT; ++u)
+            if (L % NT == 0 || t + u * NT < L) k[u] = pair(t + u * NT);
+#pragma unroll
+        for (int u = 0; u < NIT; ++u) {
+            const int p = t + u * NT;
+            if (L % NT == 0 || p < L) {
+                if (p == 0) {
+                    z[lds_pad(0)] = make_float2(k[u].x, k[u].z);
+                    const float4 e = pair(L);   // g/2, or the band's first empty place
+                    z[lds_pad(G - L)] = make_float2(e.x, e.z);
+                } else {
+                    z[lds_pad(p)] = make_float2(k[u].x - k[u].w, k[u].y + k[u].z);
+                    z[lds_pad(G - p)] = make_float2(k[u].x + k[u].w, k[u].z - k[u].y);
                 }
             }
         }
-    }
-    return lmax;
+        __syncthreads();
+        constexpr unsigned mask = band_mask<R0, nz, nz>();
+        fft_inverse_io<G, true, false, mask>(
+            z, tw, t, [&](int j, int r) { return lds_input<G, R0>(z, j, r); }, rows);
+    };
+    // The same band limit as the column pass: 9/32 of the grid on either side.
+    constexpr int NZ = bfly_prunes(R0) ? (9 * R0 + 31) / 32 : R0 / 2;
+    if (NZ < R0 / 2 && cmax < NZ * NB0)
+        run(std::integral_constant<int, NZ>{});
+    else
+        run(std::integral_constant<int, R0 / 2>{});
+    const unsigned bm = block_max_u<NT>(__float_as_uint(rows.lmax), shm);
+    if (t == 0) atomicMax(max_slot(pmax, s, 0, (int)(blockIdx.x % kMaxSlots)), bm);
 }
 
-// The image size of a plan: G = 2M = 1.5 I.
+// Gather and C2R split of one image row in one pass: Z[k] = E[k] + i O[k],
+// E = K[k] + K~[k+M], O = (K[k] - K~[k+M]) e^{2 pi i k/G},
+// K~[k+M] = conj(K[M-k]) (k > 0), K[M] (k = 0).  A thread takes the pairs
+// (p, M-p), reads K[p] and K[M-p] straight from the K tiles (zero beyond cmax)
+// and writes Z[p], Z[M-p]; the pairs cover every index 0..M-1.
+// wpost[M - p] = -conj(wpost[p]).  The loads of all the thread's pairs are
+// issued together, then paired into LDS.
 template <int M>
-constexpr int c2r_image() { return 4 * M / 3; }
-
-// Whether c2r_output_fixed applies: each of a thread's columns lies wholly on
-// one side of the crop's wrap point h, and every column's offset from the
-// thread's first one is a multiple of 64.
-template <int M, int NTB>
-constexpr bool c2r_fixed_ok()
+__device__ __forceinline__ void c2r_gather(float2* zr, const float2* __restrict__ kt0,
+                                           const float2* __restrict__ wpost, int cmax, int tid)
 {
-    constexpr int G = 2 * M, I = c2r_image<M>(), h = I / 2;
-    return 3 * I == 2 * G && NTB % 64 == 0 && h % 64 == 0 && (G - h) % 64 == 0 && NTB <= h && h % NTB == 0;
-}
-
-// c2r_output_rows for the plan's own image size, with the column walk resolved
-// at compile time: thread t takes columns t + j*NTB.  Column col maps to the
-// real sample mm = col + G - h (col < h) or col - h (col >= h), i.e. t plus a
-// constant C_j that is a multiple of 64, so its float in the LDS row,
-// 2*lds_pad(mm >> 1) + (mm & 1), is t + 2*(t >> 6) + C_j + C_j/32: one 4-byte
-// LDS read at an immediate offset from a per-thread base, in place of an
-// index computation, an 8-byte read and a select.  The same values, products
-// and maxima as c2r_output_rows.
-template <int M, int ROWS, int NTB>
-__device__ __forceinline__ float c2r_output_fixed(const float2* zb, const float* __restrict__ corr, float* out0,
-                                                  int y0, int tid)
-{
-    constexpr int G = 2 * M, I = c2r_image<M>(), h = I / 2;
-    constexpr int L2 = 2 * lds_len(M + 1);   // floats per LDS row
-    constexpr int NC = I / NTB;              // columns per thread
-    float lmax = 0.0f;
-    float cy[ROWS];
+    constexpr int NT = FftPlan<M>::nt;
+    constexpr int PB = (M / 2 + NT) / NT;               // pairs per thread: ceil((M/2+1)/NT)
+    float2 a[PB], b[PB], wv[PB];
 #pragma unroll
-    for (int r = 0; r < ROWS; ++r) {
-        const int y = y0 + r - h;
-        cy[r] = corr[y < 0 ? -y : y];
+    for (int u = 0; u < PB; ++u) {
+        const int p = tid + u * NT;
+        const bool ok = p <= M / 2;
+        wv[u] = ok ? wpost[p] : make_float2(0.0f, 0.0f);
+        a[u] = (ok && p <= cmax) ? kt0[(size_t)p * kKTile] : make_float2(0.0f, 0.0f);
+        b[u] = (ok && M - p <= cmax) ? kt0[(size_t)(M - p) * kKTile] : make_float2(0.0f, 0.0f);
     }
-    const float* zf = reinterpret_cast<const float*>(zb) + tid + 2 * (tid >> 6);
-    float cv[NC];
-    static_for<NC>([&](auto jc) {
-        constexpr int j = decltype(jc)::value;
-        if constexpr ((j + 1) * NTB <= h)
-            cv[j] = corr[(h - j * NTB) - tid];   // |x| = h - col
-        else
-            cv[j] = corr[tid + (j * NTB - h)];   // |x| = col - h
-    });
-    static_for<NC>([&](auto jc) {
-        constexpr int j = decltype(jc)::value;
-        constexpr int C = ((j + 1) * NTB <= h) ? j * NTB + (G - h) : j * NTB - h;
-        constexpr int off = C + C / 32;
 #pragma unroll
-        for (int r = 0; r < ROWS; ++r) {
-            const float val = fabsf(zf[r * L2 + off]) * (cv[j] * cy[r]);
-            __builtin_nontemporal_store(val, out0 + (size_t)r * I + tid + j * NTB);
-            lmax = fmaxf(lmax, val);
+    for (int u = 0; u < PB; ++u) {
+        const int p = tid + u * NT;
+        if (p > M / 2) break;
+        const float2 av = a[u], bv = b[u];
+        if (p == 0) {
+            zr[lds_pad(0)] = cadd(cadd(av, bv), cmul_i(csub(av, bv)));
+        } else {
+            const float2 kp = cconj(bv);   // K~[p+M]
+            zr[lds_pad(p)] = cadd(cadd(av, kp), cmul_i(cmul(csub(av, kp), wv[u])));
+            if (p != M - p) {
+                const float2 km = cconj(av);   // K~[M-p+M]
+                const float2 wm = make_float2(-wv[u].x, wv[u].y);
+                zr[lds_pad(M - p)] = cadd(cadd(bv, km), cmul_i(cmul(csub(bv, km), wm)));
+            }
         }
-    });
-    return lmax;
+    }
 }
 
-template <int M, int ROWS>
-__global__ __launch_bounds__(FftPlan<M>::nt * ROWS) void k_stage2(const float2* __restrict__ kt,
+// One image row per workgroup as a real transform (a complex one of length
+// M = g/2): for 8192^2, where two rows in one transform of length 12288 would
+// hold 101 KB of LDS, one workgroup per CU.  Element n of the transform is
+// columns 2n and 2n + 1 of the row, cropped and stored as in RowStore.
+// 588 -> 565 us for three images: 8-byte loads of 64-byte runs bound it.
+template <int M>
+__global__ __launch_bounds__(FftPlan<M>::nt, 6) void k_stage2_row(const float2* __restrict__ kt,
                                                                    const SnapMeta* __restrict__ meta,
                                                                    unsigned* __restrict__ pmax,
                                                                    const float2* __restrict__ tw,
                                                                    const float2* __restrict__ wpost,
                                                                    const float* __restrict__ corr,
-                                                                   float* __restrict__ pre, int I)
+                                                                   float* __restrict__ pre)
 {
-    constexpr int NT = FftPlan<M>::nt;
-    constexpr int L = lds_len(M + 1);
-    __shared__ float2 zb[ROWS * L];
-    __shared__ unsigned shm[NT * ROWS / 64];
-    const int s = blockIdx.y;
-    const int y0 = xcd_remap(blockIdx.x, gridDim.x) * ROWS;
-    const int grp = threadIdx.x / NT, t = threadIdx.x % NT;
-    const int cmax = min(meta[s].rmax, M);
-    if (cmax < M / 2) {
-        C2RGatherLow<M, ROWS> gth;
-        gth.load(c2r_rows<M>(kt, s, y0, I), wpost, cmax, threadIdx.x);
-        gth.store(zb, cmax, threadIdx.x);
-    } else {
-        C2RGather<M, ROWS> gth;
-        gth.load(c2r_rows<M>(kt, s, y0, I), wpost, cmax, threadIdx.x);
-        gth.store(zb, threadIdx.x);
-    }
+    constexpr int G = 2 * M, I = 2 * G / 3, h = I / 2, NT = FftPlan<M>::nt;
+    constexpr int R = FftPlan<M>::radix[FftPlan<M>::nstages - 1], NS = M / R, KEEP = R / 3;
+    static_assert(R % 3 == 0 && 3 * h == G, "whole outputs are cropped");
+    __shared__ float2 z[lds_len(M)];
+    __shared__ unsigned shm[NT / 64];
+    const int s = blockIdx.y, t = threadIdx.x;
+    const int y = xcd_remap(blockIdx.x, gridDim.x);
+    c2r_gather<M>(z, c2r_rows<M>(kt, s, y, I), wpost, min(meta[s].rmax, M), t);
     __syncthreads();
-    float2* z = zb + grp * L;
-    fft_inverse<M>(z, tw, t);
-    float* const out0 = pre + (size_t)s * I * I + (size_t)y0 * I;
-    float lmax;
-    if constexpr (c2r_fixed_ok<M, NT * ROWS>()) {
-        lmax = I == c2r_image<M>() ? c2r_output_fixed<M, ROWS, NT * ROWS>(zb, corr, out0, y0, threadIdx.x)
-                                   : c2r_output_rows<M, ROWS, NT * ROWS>(zb, corr, out0, y0, I, threadIdx.x);
-    } else {
-        lmax = c2r_output_rows<M, ROWS, NT * ROWS>(zb, corr, out0, y0, I, threadIdx.x);
-    }
-    const unsigned bm = block_max_u<NT * ROWS>(__float_as_uint(lmax), shm);
-    if (threadIdx.x == 0) atomicMax(max_slot(pmax, s, 0, (int)(blockIdx.x % kMaxSlots)), bm);
+    const float cy = corr[y < h ? h - y : y - h];
+    float* const row = pre + (size_t)s * I * I + (size_t)y * I;
+    float lmax = 0.0f;
+    constexpr int R0 = FftPlan<M>::radix[0];
+    fft_inverse_io<M, true, false>(
+        z, tw, t,
+        [&](int j, int r) { return lds_input<M, R0>(z, j, r); },
+        [&](int j, const float2* v) {
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                if (r >= KEEP && r < 2 * KEEP) continue;
+                const int x = 2 * (j + NS * r) - (r < KEEP ? 0 : G);
+                const float a = fabsf(v[r].x) * (corr[x < 0 ? -x : x] * cy);
+                const float b = fabsf(v[r].y) * (corr[x < 0 ? -x - 1 : x + 1] * cy);
+                typedef float fip_f2 __attribute__((ext_vector_type(2)));
+                const fip_f2 ab = {a, b};
+                __builtin_nontemporal_store(ab, reinterpret_cast<fip_f2*>(row + (x + h)));
+                lmax = fmaxf(lmax, fmaxf(a, b));
+            }
+        });
+    const unsigned bm = block_max_u<NT>(__float_as_uint(lmax), shm);
+    if (t == 0) atomicMax(max_slot(pmax, s, 0, (int)(blockIdx.x % kMaxSlots)), bm);
 }
 
 // ----------------------------------------------------------------- splat
@@ -1997,45 +1903,27 @@ hipError_t launch_stage1(const WorkView& w, const PlanTables& p, int S, const Tu
     return hipGetLastError();
 }
 
-template <int M, int ROWS>
+template <int G>
 static void stage2_dispatch(const WorkView& w, const PlanTables& p, int S, hipStream_t st)
 {
-    constexpr int NT = FftPlan<M>::nt * ROWS;
-    hipLaunchKernelGGL((k_stage2<M, ROWS>), dim3(p.I / ROWS, S), dim3(NT), 0, st, w.kt, w.meta, w.pmax, p.tw_m,
-                       p.wpost, p.corr, w.pre, p.I);
+    hipLaunchKernelGGL(k_stage2<G>, dim3(p.I / 2, S), dim3(FftPlan<G>::nt), 0, st, w.kt, w.meta, w.pmax, p.tw_g,
+                       p.corr, w.pre);
 }
 
-template <int M>
-static void stage2_pick(const WorkView& w, const PlanTables& p, int S, const Tuning& tu, hipStream_t st)
+hipError_t launch_stage2(const WorkView& w, const PlanTables& p, int S, hipStream_t st)
 {
-    // LDS per row is (M + M/32 + 2) * 8 bytes; keep a workgroup under 128 KiB.
-    constexpr int row_bytes = lds_len(M + 1) * 8;
-    if constexpr (4 * row_bytes <= 128 * 1024 && kKTile % 4 == 0) {
-        if (tu.stage2_rows >= 4) {
-            stage2_dispatch<M, 4>(w, p, S, st);
-            return;
-        }
-    }
-    if constexpr (2 * row_bytes <= 128 * 1024 && kKTile % 2 == 0) {
-        if (tu.stage2_rows >= 2) {
-            stage2_dispatch<M, 2>(w, p, S, st);
-            return;
-        }
-    }
-    stage2_dispatch<M, 1>(w, p, S, st);
-}
-
-hipError_t launch_stage2(const WorkView& w, const PlanTables& p, int S, const Tuning& tu, hipStream_t st)
-{
-    switch (p.M) {
-    case 48: stage2_pick<48>(w, p, S, tu, st); break;
-    case 96: stage2_pick<96>(w, p, S, tu, st); break;
-    case 192: stage2_pick<192>(w, p, S, tu, st); break;
-    case 384: stage2_pick<384>(w, p, S, tu, st); break;
-    case 768: stage2_pick<768>(w, p, S, tu, st); break;
-    case 1536: stage2_pick<1536>(w, p, S, tu, st); break;
-    case 3072: stage2_pick<3072>(w, p, S, tu, st); break;
-    case 6144: stage2_pick<6144>(w, p, S, tu, st); break;
+    switch (p.G) {
+    case 96: stage2_dispatch<96>(w, p, S, st); break;
+    case 192: stage2_dispatch<192>(w, p, S, st); break;
+    case 384: stage2_dispatch<384>(w, p, S, st); break;
+    case 768: stage2_dispatch<768>(w, p, S, st); break;
+    case 1536: stage2_dispatch<1536>(w, p, S, st); break;
+    case 3072: stage2_dispatch<3072>(w, p, S, st); break;
+    case 6144: stage2_dispatch<6144>(w, p, S, st); break;
+    case 12288:
+        hipLaunchKernelGGL(k_stage2_row<6144>, dim3(p.I, S), dim3(FftPlan<6144>::nt), 0, st, w.kt, w.meta, w.pmax,
+                           p.tw_m, p.wpost, p.corr, w.pre);
+        break;
     default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
