@@ -103,11 +103,9 @@ public:
     hipStream_t copy_stream = nullptr;
     hipEvent_t in_ready[3] = {};
     // Preprocessing (projection, collapse and the raw-input chain): device
-    // inputs of the host-array entry points, per-block moment partials,
-    // per-snapshot projection parameters, and pinned memory for the partials
-    // read back and the parameters sent.
+    // inputs of the host-array entry points, per-block moment partials and
+    // per-snapshot projection parameters.
     DevBuf pp_uvw, pp_freq, pp_in, pp_part, pp_par;
-    PinnedBuf pp_host;
 
     // Every entry point that enqueues work on `work` from some stream calls
     // order_work(st) before and mark_work(st) after, so uses of the shared

@@ -3,19 +3,33 @@
 // SVDPreprocessKernels.cu:167-206).
 #pragma once
 
+#include <hip/hip_runtime.h>
+
 #include <cmath>
 
 namespace fip {
 
+// Both functions run on the host and on the GPU.  Without contraction, and with
+// IEEE division and square root on both sides, their results are the same bits,
+// so the sign rule's ties fall the same way too.  Indices are compile-time
+// constants once unrolled: on the GPU the matrices stay in registers.
+
 // Cyclic Jacobi on a symmetric 3x3 matrix a (destroyed).  evec columns are
-// the eigenvectors of eval.
-inline void jacobi3(double a[3][3], double evec[3][3], double eval[3])
+// the eigenvectors of eval.  It ends once the off-diagonal is below 1e-25 of the
+// diagonal: a further rotation's sine is then far below an ulp of the vectors
+// (unless two eigenvalues agree to 1e-9, where they are not determined by
+// the data).
+__host__ __device__ inline void jacobi3(double a[3][3], double evec[3][3], double eval[3])
 {
+#pragma clang fp contract(off)
     double v[3][3] = {{1, 0, 0}, {0, 1, 0}, {0, 0, 1}};
+#pragma unroll 1
     for (int sweep = 0; sweep < 64; ++sweep) {
         const double off = std::fabs(a[0][1]) + std::fabs(a[0][2]) + std::fabs(a[1][2]);
-        if (off == 0.0) break;
+        if (off <= 1e-25 * (std::fabs(a[0][0]) + std::fabs(a[1][1]) + std::fabs(a[2][2]))) break;
+#pragma unroll
         for (int p = 0; p < 2; ++p) {
+#pragma unroll
             for (int q = p + 1; q < 3; ++q) {
                 if (a[p][q] == 0.0) continue;
                 const double theta = (a[q][q] - a[p][p]) / (2.0 * a[p][q]);
@@ -48,27 +62,35 @@ inline void jacobi3(double a[3][3], double evec[3][3], double eval[3])
 // From a covariance matrix: V0, V1 = eigenvectors of the two largest
 // eigenvalues, each with its largest-magnitude entry made positive (first
 // index on ties), and V2 = V0 x V1.  V is row-major [3][3].
-inline void pca_basis(const double cov_in[3][3], double V[3][3])
+__host__ __device__ inline void pca_basis(const double cov_in[3][3], double V[3][3])
 {
+#pragma clang fp contract(off)
     double a[3][3], evec[3][3], eval[3];
     for (int i = 0; i < 3; ++i)
         for (int j = 0; j < 3; ++j) a[i][j] = cov_in[i][j];
     jacobi3(a, evec, eval);
-    int order[3] = {0, 1, 2};
+    // Columns in descending order of their eigenvalues.
+#pragma unroll
     for (int i = 0; i < 3; ++i)
+#pragma unroll
         for (int j = i + 1; j < 3; ++j)
-            if (eval[order[j]] > eval[order[i]]) {
-                const int t = order[i];
-                order[i] = order[j];
-                order[j] = t;
+            if (eval[j] > eval[i]) {
+                const double t = eval[i];
+                eval[i] = eval[j];
+                eval[j] = t;
+                for (int k = 0; k < 3; ++k) {
+                    const double u = evec[k][i];
+                    evec[k][i] = evec[k][j];
+                    evec[k][j] = u;
+                }
             }
+#pragma unroll
     for (int c = 0; c < 2; ++c) {
-        for (int k = 0; k < 3; ++k) V[c][k] = evec[k][order[c]];
-        int am = 0;
+        double top = evec[0][c];
+#pragma unroll
         for (int k = 1; k < 3; ++k)
-            if (std::fabs(V[c][k]) > std::fabs(V[c][am])) am = k;
-        if (V[c][am] < 0)
-            for (int k = 0; k < 3; ++k) V[c][k] = -V[c][k];
+            if (std::fabs(evec[k][c]) > std::fabs(top)) top = evec[k][c];
+        for (int k = 0; k < 3; ++k) V[c][k] = top < 0 ? -evec[k][c] : evec[k][c];
     }
     V[2][0] = V[0][1] * V[1][2] - V[0][2] * V[1][1];
     V[2][1] = V[0][2] * V[1][0] - V[0][0] * V[1][2];

@@ -2,12 +2,15 @@
 // (SVD_MFS.py:38-110; SVDPreprocessKernels.cu:41-237).
 //
 // The projection reduces the baseline mean and covariance in FP64 in one
-// pass with fixed per-block partial sums (summed on the host in block order,
-// so the result is deterministic), diagonalises the 3x3 covariance on the
-// host in FP64 after one small read-back, and applies B = D.[V0 V1] as one
-// coalesced streaming kernel.  fip_pipe_raw_device chains collapse,
-// projection, imaging and trigger on the device.  Buffers are the context's
-// grow-only ones: no call allocates once sizes are warm.
+// pass with fixed per-block partial sums, adds those up in a fixed order (so
+// the result is deterministic) and diagonalises the 3x3 covariance in FP64 in
+// one workgroup per snapshot, and applies B = D.[V0 V1] as one coalesced
+// streaming kernel.  fip_pipe_raw_device chains collapse, projection, imaging
+// and trigger on the device without waiting for any of it: the workgroups of
+// the eigen-solve go out with those of the collapse.  (With the solve on the
+// host, a read-back and two uploads left the GPU idle for 70 us of a call of
+// 135 at 1024^2 with 4 x 8128 samples.)  Buffers are the context's grow-only
+// ones: no call allocates once sizes are warm.
 #include "fip.h"
 
 #include "fip_context.hpp"
@@ -16,41 +19,49 @@
 #include <hip/hip_runtime.h>
 
 #include <cmath>
-#include <vector>
 
 namespace fip {
 namespace {
 
 constexpr double kLight = 299792458.0;   // SVD_MFS.py:7
 constexpr int kPT = 256;                 // threads per block
-constexpr int kPerThread = 16;           // samples per thread per moment block
+// Samples per thread of a moment block: four, for enough workgroups at the
+// usual counts (32512 samples in 32 rather than 8 workgroups: 11.2 us before).
+constexpr int kPerThread = 4;
 constexpr int kPerBlock = kPT * kPerThread;
 constexpr int kMom = 9;                  // 3 first + 6 second moments
 constexpr int kPar = 12;                 // per-snapshot projection parameters (mean, V0, V1, pad)
 
 // Sample n = row + chan*nrows (channel-major flattening, SVD_MFS.py:48-52).
+// The counts' division is a 32-bit one where they allow it.
 __device__ __forceinline__ void sample(const double* __restrict__ uvw, const double* __restrict__ freqs,
-                                       size_t nrows, size_t n, double d[3])
+                                       size_t nrows, size_t n, bool small, double d[3])
 {
-    const size_t row = n % nrows, chan = n / nrows;
+    const size_t chan = small ? (size_t)((unsigned)n / (unsigned)nrows) : n / nrows;
+    const size_t row = n - chan * nrows;
     const double sc = freqs[chan] / kLight;
     d[0] = uvw[3 * row] * sc;
     d[1] = uvw[3 * row + 1] * sc;
     d[2] = uvw[3 * row + 2] * sc;
 }
+__device__ __forceinline__ bool small_counts(size_t ns) { return ns <= 0xffffffffull; }
 
+// Sums of NV values over the workgroup in a fixed order: a wave's by
+// shuffles, the four waves' through LDS.  Valid in thread 0.
 template <int NV>
-__device__ __forceinline__ void block_sum(double (&v)[NV], double* sh, double* out)
+__device__ __forceinline__ void block_sum(double (&v)[NV], double (*sh)[NV])
 {
-    for (int k = 0; k < NV; ++k) sh[k * kPT + threadIdx.x] = v[k];
+#pragma unroll
+    for (int k = 0; k < NV; ++k)
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) v[k] += __shfl_down(v[k], o, 64);
+    if ((threadIdx.x & 63) == 0)
+#pragma unroll
+        for (int k = 0; k < NV; ++k) sh[threadIdx.x >> 6][k] = v[k];
     __syncthreads();
-    for (int st = kPT / 2; st > 0; st >>= 1) {
-        if ((int)threadIdx.x < st)
-            for (int k = 0; k < NV; ++k) sh[k * kPT + threadIdx.x] += sh[k * kPT + threadIdx.x + st];
-        __syncthreads();
-    }
     if (threadIdx.x == 0)
-        for (int k = 0; k < NV; ++k) out[k] = sh[k * kPT];
+#pragma unroll
+        for (int k = 0; k < NV; ++k) v[k] = (sh[0][k] + sh[1][k]) + (sh[2][k] + sh[3][k]);
 }
 
 // One pass of moments for snapshot blockIdx.y: per block of kPerBlock
@@ -61,19 +72,24 @@ __device__ __forceinline__ void block_sum(double (&v)[NV], double* sh, double* o
 __global__ __launch_bounds__(kPT) void k_moments(const double* __restrict__ uvw, const double* __restrict__ freqs,
                                                  size_t nrows, size_t ns, int nb, double* __restrict__ part)
 {
-    __shared__ double sh[kMom * kPT];
+    __shared__ double sh[kPT / 64][kMom];
     const int s = blockIdx.y;
     const double* u = uvw + (size_t)s * nrows * 3;
-    double d0[3];
-    sample(u, freqs, nrows, 0, d0);
-    double v[kMom] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
-    const size_t base = (size_t)blockIdx.x * kPerBlock;
+    const bool small = small_counts(ns);
+    double d0[3], d[kPerThread][3];
+    const size_t base = (size_t)blockIdx.x * kPerBlock + threadIdx.x;
+    // every load before its use (samples past the end: the last one, not added)
+#pragma unroll
     for (int k = 0; k < kPerThread; ++k) {
-        const size_t n = base + (size_t)k * kPT + threadIdx.x;
-        if (n < ns) {
-            double d[3];
-            sample(u, freqs, nrows, n, d);
-            const double a = d[0] - d0[0], b = d[1] - d0[1], c = d[2] - d0[2];
+        const size_t n = base + (size_t)k * kPT;
+        sample(u, freqs, nrows, n < ns ? n : ns - 1, small, d[k]);
+    }
+    sample(u, freqs, nrows, 0, small, d0);
+    double v[kMom] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+    for (int k = 0; k < kPerThread; ++k) {
+        if (base + (size_t)k * kPT < ns) {
+            const double a = d[k][0] - d0[0], b = d[k][1] - d0[1], c = d[k][2] - d0[2];
             v[0] += a;
             v[1] += b;
             v[2] += c;
@@ -85,10 +101,52 @@ __global__ __launch_bounds__(kPT) void k_moments(const double* __restrict__ uvw,
             v[8] += c * c;
         }
     }
+    block_sum<kMom>(v, sh);
     double* ps = part + (size_t)s * (nb + 1) * kMom;
-    block_sum<kMom>(v, sh, ps + (size_t)blockIdx.x * kMom);
-    if (blockIdx.x == 0 && threadIdx.x == 0)
-        for (int k = 0; k < 3; ++k) ps[(size_t)nb * kMom + k] = d0[k];
+    if (threadIdx.x == 0) {
+        for (int k = 0; k < kMom; ++k) ps[(size_t)blockIdx.x * kMom + k] = v[k];
+        if (blockIdx.x == 0)
+            for (int k = 0; k < 3; ++k) ps[(size_t)nb * kMom + k] = d0[k];
+    }
+}
+
+// Projection of one snapshot from its nb moment partials, by one workgroup:
+// mean and covariance, their principal axes (SVD_MFS.py:64-75, 98-103), and
+// par (mean, V0, V1) and vin (V, float).  The partials are added up in a
+// fixed order; the eigen-solve is one thread's FP64 chain.
+__device__ void snapshot_basis(const double* __restrict__ ps, int nb, size_t ns, double* __restrict__ par,
+                               float* __restrict__ vin)
+{
+    __shared__ double sh[kPT / 64][kMom];
+    double m[kMom] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
+    for (int b = threadIdx.x; b < nb; b += kPT)
+#pragma unroll
+        for (int k = 0; k < kMom; ++k) m[k] += ps[(size_t)b * kMom + k];
+    block_sum<kMom>(m, sh);
+    if (threadIdx.x != 0) return;
+    const double* d0 = ps + (size_t)nb * kMom;
+    const double dn = (double)ns;
+    // mean = D_0 + sum(a)/n; centred sums = sum(a a^T) - n (mean-D_0)(mean-D_0)^T
+    const double e[3] = {m[0] / dn, m[1] / dn, m[2] / dn};
+    const double mu[3] = {d0[0] + e[0], d0[1] + e[1], d0[2] + e[2]};
+    const double c00 = m[3] - dn * e[0] * e[0], c01 = m[4] - dn * e[0] * e[1], c02 = m[5] - dn * e[0] * e[2];
+    const double c11 = m[6] - dn * e[1] * e[1], c12 = m[7] - dn * e[1] * e[2], c22 = m[8] - dn * e[2] * e[2];
+    const double den = (double)(ns - 1);
+    const double cov[3][3] = {{c00 / den, c01 / den, c02 / den},
+                              {c01 / den, c11 / den, c12 / den},
+                              {c02 / den, c12 / den, c22 / den}};
+    double V[3][3];
+    pca_basis(cov, V);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        par[k] = mu[k];
+        par[3 + k] = V[0][k];
+        par[6 + k] = V[1][k];
+        par[9 + k] = 0.0;
+        vin[k] = (float)V[0][k];
+        vin[3 + k] = (float)V[1][k];
+        vin[6 + k] = (float)V[2][k];
+    }
 }
 
 // B[n] = (D_n - mean).Vj + mean.Vj (SVD_MFS.py:68, 105-110), streaming, for
@@ -104,7 +162,7 @@ __global__ __launch_bounds__(kPT) void k_proj_apply(const double* __restrict__ u
     const double m0 = q[0], m1 = q[1], m2 = q[2];
     const double v00 = q[3], v01 = q[4], v02 = q[5], v10 = q[6], v11 = q[7], v12 = q[8];
     double d[3];
-    sample(uvw + (size_t)s * nrows * 3, freqs, nrows, n, d);
+    sample(uvw + (size_t)s * nrows * 3, freqs, nrows, n, small_counts(ns), d);
     const double a = d[0] - m0, b = d[1] - m1, c = d[2] - m2;
     const double mv0 = m0 * v00 + m1 * v01 + m2 * v02, mv1 = m0 * v10 + m1 * v11 + m2 * v12;
     bin[(size_t)s * stride + n] =
@@ -113,16 +171,34 @@ __global__ __launch_bounds__(kPT) void k_proj_apply(const double* __restrict__ u
 
 // (w0 XX + w3 YY)/(w0 + w3), w = weight * !flag, 0 where the sum is not
 // positive (SVDPreprocessKernels.cu:208-237), for snapshot blockIdx.y:
-// inputs at s*n, outputs at s*ostride.
+// inputs at s*n, outputs at s*ostride.  proj.part set: workgroup 0 of each
+// snapshot computes its projection instead, under the others' streaming.
+struct Projection {
+    const double* part;   // [S][nb + 1][kMom]
+    int nb;
+    size_t ns;
+    double* par;          // [S][kPar]
+    float* vin;           // [S][9]
+};
 __global__ __launch_bounds__(kPT) void k_collapse(const float* __restrict__ xr, const float* __restrict__ xi,
                                                   const float* __restrict__ yr, const float* __restrict__ yi,
                                                   const unsigned char* __restrict__ f0,
                                                   const unsigned char* __restrict__ f3,
                                                   const float* __restrict__ w0, const float* __restrict__ w3,
                                                   size_t n, float* __restrict__ ore, float* __restrict__ oim,
-                                                  size_t ostride)
+                                                  size_t ostride, Projection proj)
 {
-    const size_t i = (size_t)blockIdx.x * kPT + threadIdx.x;
+    const int s0 = blockIdx.y;
+    unsigned blk = blockIdx.x;
+    if (proj.part) {
+        if (blk == 0) {
+            snapshot_basis(proj.part + (size_t)s0 * (proj.nb + 1) * kMom, proj.nb, proj.ns, proj.par + s0 * kPar,
+                           proj.vin + s0 * 9);
+            return;
+        }
+        --blk;
+    }
+    const size_t i = (size_t)blk * kPT + threadIdx.x;
     if (i >= n) return;
     const size_t q = (size_t)blockIdx.y * n + i, o = (size_t)blockIdx.y * ostride + i;
     const float a = f0[q] ? 0.0f : w0[q];
@@ -139,78 +215,36 @@ __global__ __launch_bounds__(kPT) void k_collapse(const float* __restrict__ xr, 
 
 size_t moment_blocks(size_t ns) { return (ns + kPerBlock - 1) / kPerBlock; }
 
-// Pinned layout of pp_host for S snapshots: partials read back, then the
-// projection parameters and the float V matrices sent.
-struct PpHostLayout {
-    size_t part, par, vin, bytes;
-};
-PpHostLayout pp_host_layout(int S, size_t nb)
+__global__ __launch_bounds__(kPT) void k_basis(Projection proj)
 {
-    PpHostLayout L;
-    L.part = 0;
-    L.par = L.part + (size_t)S * (nb + 1) * kMom * sizeof(double);
-    L.vin = L.par + (size_t)S * kPar * sizeof(double);
-    L.bytes = L.vin + (size_t)S * 9 * sizeof(float);
-    return L;
+    const int s = blockIdx.x;
+    snapshot_basis(proj.part + (size_t)s * (proj.nb + 1) * kMom, proj.nb, proj.ns, proj.par + s * kPar,
+                   proj.vin + s * 9);
 }
 
-// Projection of S snapshots whose uvw ([S][nrows][3]) and frequencies are in
-// device memory: one moment pass, one read-back of the partials, the 3x3
-// eigen-solve per snapshot on the host in FP64 (partials summed in block
-// order, so the result is deterministic), then B into bin + s*stride
-// (float2) and, when vin_dev is set, V as float into vin_dev + 9 s.
-// Synchronises `st` once (after the moments); the rest stays enqueued.
-int project_device(Context& C, const double* uvw, const double* freqs, size_t nrows, size_t nchan, int S,
-                   float2* bin, size_t stride, float* vin_dev, double (*V)[3][3], hipStream_t st)
+// Moments of S snapshots whose uvw ([S][nrows][3]) and frequencies are in
+// device memory, enqueued on `st`; `proj` then describes their eigen-solve
+// (k_basis, or workgroups of the collapse), which writes V as float into
+// vin_dev + 9 s.
+int enqueue_moments(Context& C, const double* uvw, const double* freqs, size_t nrows, size_t nchan, int S,
+                    float* vin_dev, Projection& proj, hipStream_t st)
 {
     const size_t ns = nrows * nchan;
     const size_t nb = moment_blocks(ns);
-    const PpHostLayout L = pp_host_layout(S, nb);
     FIP_HIP(C.pp_part.ensure((size_t)S * (nb + 1) * kMom * sizeof(double)));
     FIP_HIP(C.pp_par.ensure((size_t)S * kPar * sizeof(double)));
-    FIP_HIP(C.pp_host.ensure(L.bytes));
-    char* h = static_cast<char*>(C.pp_host.p);
     hipLaunchKernelGGL(k_moments, dim3((unsigned)nb, (unsigned)S), dim3(kPT), 0, st, uvw, freqs, nrows, ns, (int)nb,
                        C.pp_part.as<double>());
     FIP_HIP(hipGetLastError());
-    FIP_HIP(hipMemcpyAsync(h + L.part, C.pp_part.p, (size_t)S * (nb + 1) * kMom * sizeof(double),
-                           hipMemcpyDeviceToHost, st));
-    FIP_HIP(hipStreamSynchronize(st));
-    const double* part = reinterpret_cast<const double*>(h + L.part);
-    double* par = reinterpret_cast<double*>(h + L.par);
-    float* vf = reinterpret_cast<float*>(h + L.vin);
-    for (int s = 0; s < S; ++s) {
-        const double* ps = part + (size_t)s * (nb + 1) * kMom;
-        double m[kMom] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
-        for (size_t b = 0; b < nb; ++b)
-            for (int k = 0; k < kMom; ++k) m[k] += ps[b * kMom + k];
-        const double* d0 = ps + nb * kMom;
-        const double dn = (double)ns;
-        // mean = D_0 + sum(a)/n; centred sums = sum(a a^T) - n (mean-D_0)(mean-D_0)^T
-        const double e[3] = {m[0] / dn, m[1] / dn, m[2] / dn};
-        const double mu[3] = {d0[0] + e[0], d0[1] + e[1], d0[2] + e[2]};
-        const double c00 = m[3] - dn * e[0] * e[0], c01 = m[4] - dn * e[0] * e[1], c02 = m[5] - dn * e[0] * e[2];
-        const double c11 = m[6] - dn * e[1] * e[1], c12 = m[7] - dn * e[1] * e[2], c22 = m[8] - dn * e[2] * e[2];
-        const double den = (double)(ns - 1);
-        const double cov[3][3] = {{c00 / den, c01 / den, c02 / den},
-                                  {c01 / den, c11 / den, c12 / den},
-                                  {c02 / den, c12 / den, c22 / den}};
-        pca_basis(cov, V[s]);
-        double* q = par + (size_t)s * kPar;
-        q[0] = mu[0];
-        q[1] = mu[1];
-        q[2] = mu[2];
-        for (int k = 0; k < 3; ++k) {
-            q[3 + k] = V[s][0][k];
-            q[6 + k] = V[s][1][k];
-        }
-        q[9] = q[10] = q[11] = 0.0;
-        for (int a = 0; a < 3; ++a)
-            for (int b = 0; b < 3; ++b) vf[9 * s + 3 * a + b] = (float)V[s][a][b];
-    }
-    FIP_HIP(hipMemcpyAsync(C.pp_par.p, h + L.par, (size_t)S * kPar * sizeof(double), hipMemcpyHostToDevice, st));
-    if (vin_dev)
-        FIP_HIP(hipMemcpyAsync(vin_dev, h + L.vin, (size_t)S * 9 * sizeof(float), hipMemcpyHostToDevice, st));
+    proj = Projection{C.pp_part.as<double>(), (int)nb, ns, C.pp_par.as<double>(), vin_dev};
+    return FIP_OK;
+}
+
+// B of S snapshots from their projections into bin + s*stride (float2).
+int enqueue_apply(Context& C, const double* uvw, const double* freqs, size_t nrows, size_t nchan, int S, float2* bin,
+                  size_t stride, hipStream_t st)
+{
+    const size_t ns = nrows * nchan;
     hipLaunchKernelGGL(k_proj_apply, dim3((unsigned)((ns + kPT - 1) / kPT), (unsigned)S), dim3(kPT), 0, st, uvw,
                        freqs, nrows, ns, C.pp_par.as<double>(), bin, stride);
     FIP_HIP(hipGetLastError());
@@ -235,9 +269,9 @@ extern "C" int fip_project(const double* uvw, size_t nrows, const double* freqs,
         if (int rc = Context::get(&C)) return rc;
         std::lock_guard<std::recursive_mutex> lk(C->mu);
         hipStream_t st = C->stream;
-        // The pinned and device preprocessing buffers are shared with
-        // fip_pipe_raw_device, whose last copies may still be in flight on a
-        // caller's stream: wait for them first.
+        // The preprocessing buffers are shared with fip_pipe_raw_device, whose
+        // last launches may still be in flight on a caller's stream: wait for
+        // them first.
         if (int rc = C->order_work(st)) return rc;
         FIP_HIP(hipStreamSynchronize(st));
         FIP_HIP(C->pp_uvw.ensure(nrows * 3 * sizeof(double)));
@@ -245,15 +279,17 @@ extern "C" int fip_project(const double* uvw, size_t nrows, const double* freqs,
         FIP_HIP(C->pp_in.ensure(ns * sizeof(float2)));
         FIP_HIP(hipMemcpy(C->pp_uvw.p, uvw, nrows * 3 * sizeof(double), hipMemcpyHostToDevice));
         FIP_HIP(hipMemcpy(C->pp_freq.p, freqs, nchan * sizeof(double), hipMemcpyHostToDevice));
-        double V[1][3][3];
-        if (int rc = project_device(*C, C->pp_uvw.as<double>(), C->pp_freq.as<double>(), nrows, nchan, 1,
-                                    C->pp_in.as<float2>(), ns, nullptr, V, st))
-            return rc;
+        FIP_HIP(C->in_v.ensure(9 * sizeof(float)));
+        const double *u = C->pp_uvw.as<double>(), *f = C->pp_freq.as<double>();
+        Projection proj{};
+        if (int rc = enqueue_moments(*C, u, f, nrows, nchan, 1, C->in_v.as<float>(), proj, st)) return rc;
+        hipLaunchKernelGGL(k_basis, dim3(1), dim3(kPT), 0, st, proj);
+        FIP_HIP(hipGetLastError());
+        if (int rc = enqueue_apply(*C, u, f, nrows, nchan, 1, C->pp_in.as<float2>(), ns, st)) return rc;
         FIP_HIP(hipMemcpyAsync(bin, C->pp_in.p, ns * sizeof(float2), hipMemcpyDeviceToHost, st));
+        FIP_HIP(hipMemcpyAsync(vin, C->in_v.p, 9 * sizeof(float), hipMemcpyDeviceToHost, st));
         if (int rc = C->mark_work(st)) return rc;
         FIP_HIP(hipStreamSynchronize(st));
-        for (int a = 0; a < 3; ++a)
-            for (int b = 0; b < 3; ++b) vin[3 * a + b] = (float)V[0][a][b];
         return FIP_OK;
     } catch (...) {
         return set_error(FIP_ERR_ALLOC, "host allocation failed");
@@ -296,7 +332,7 @@ extern "C" int fip_collapse(const float* xx_re, const float* xx_im, const float*
         FIP_HIP(hipMemcpy(f0, flag0, n, hipMemcpyHostToDevice));
         FIP_HIP(hipMemcpy(f3, flag3, n, hipMemcpyHostToDevice));
         hipLaunchKernelGGL(k_collapse, dim3((unsigned)((n + kPT - 1) / kPT), 1), dim3(kPT), 0, st, xr, xi, yr, yi, f0,
-                           f3, a, b, n, ore, oim, n);
+                           f3, a, b, n, ore, oim, n, Projection{});
         FIP_HIP(hipGetLastError());
         FIP_HIP(hipStreamSynchronize(st));
         FIP_HIP(hipMemcpy(out_re, ore, fb, hipMemcpyDeviceToHost));
@@ -336,14 +372,13 @@ extern "C" int fip_pipe_raw_device(const fip_raw_view* raw, size_t image_size, f
         FIP_HIP(C->in_b.ensure(S * ns * sizeof(float2)));
         FIP_HIP(C->in_v.ensure(S * 9 * sizeof(float)));
         if (int rc = C->order_work(st)) return rc;
-        hipLaunchKernelGGL(k_collapse, dim3((unsigned)((ns + kPT - 1) / kPT), (unsigned)S), dim3(kPT), 0, st, r.xx_re,
-                           r.xx_im, r.yy_re, r.yy_im, r.flag0, r.flag3, r.w0, r.w3, ns, C->in_vr.as<float>(),
-                           C->in_vi.as<float>(), ns);
+        Projection proj{};
+        if (int rc = enqueue_moments(*C, r.uvw, r.freqs, r.nrows, r.nchan, S, C->in_v.as<float>(), proj, st)) return rc;
+        hipLaunchKernelGGL(k_collapse, dim3((unsigned)((ns + kPT - 1) / kPT) + 1, (unsigned)S), dim3(kPT), 0, st,
+                           r.xx_re, r.xx_im, r.yy_re, r.yy_im, r.flag0, r.flag3, r.w0, r.w3, ns, C->in_vr.as<float>(),
+                           C->in_vi.as<float>(), ns, proj);
         FIP_HIP(hipGetLastError());
-        double V[S][3][3];
-        if (int rc = project_device(*C, r.uvw, r.freqs, r.nrows, r.nchan, S, C->in_b.as<float2>(), ns,
-                                    C->in_v.as<float>(), V, st))
-            return rc;
+        if (int rc = enqueue_apply(*C, r.uvw, r.freqs, r.nrows, r.nchan, S, C->in_b.as<float2>(), ns, st)) return rc;
         InputView in{C->in_vr.p, C->in_vi.p, C->in_b.as<float>(), C->in_v.as<float>(), nullptr, ns, (int)ns,
                      FIP_VIS_F32};
         if (int rc = pipe_sequence(C, P->t, C->work.view(ns), in, (int)ns, cell_size, C->tuning(image_size),

@@ -185,13 +185,13 @@ typedef struct fip_raw_view {
  * The whole chain on the device, from raw visibilities to trigger: the
  * weighted XX/YY collapse (SVDPreprocessKernels.cu:208-237), the SVD-plane
  * projection B = D.[V0 V1] (SVD_MFS.py:38-75, 98-110;
- * SVDPreprocessKernels.cu:255-424; FP64 moments in one pass, the 3x3
- * eigen-solve on the host after one small read-back), then FIpipe's imaging
+ * SVDPreprocessKernels.cu:255-424; FP64 moments in one pass and the 3x3
+ * eigen-solve), then FIpipe's imaging
  * and trigger (FIPkernels.cu:554-862) of snapshots 0..2 with N = nchan*nrows
  * samples each.  result: device (image/unit)^2 floats.  bin_out ([3][N][2])
  * and vin_out ([3][9]) receive B and V when not NULL (device).  Returns once
- * the work after the eigen-solve is enqueued on `stream` (NULL: the
- * library's stream); the result is ready when the stream is.
+ * the work is enqueued on `stream` (NULL: the library's stream); the result
+ * is ready when the stream is.
  */
 int fip_pipe_raw_device(const fip_raw_view *raw, size_t image_size,
                         float cell_size, size_t unit_size, float *result,

@@ -82,3 +82,19 @@ def test_project_and_collapse_reuse_context_buffers(fip, oracle):
         got = fip.collapse(xx, yy, f0, f3, w0, w3)
         ref = oracle.collapse(xx, yy, f0, f3, w0, w3)
         assert np.abs(got - ref).max() < 1e-5 * np.abs(ref).max()
+
+
+@pytest.mark.parametrize("nrows,nchan", [(3, 1), (64, 4), (255, 1), (341, 3), (1024, 1), (1025, 1), (1500, 9),
+                                         (70001, 4)])
+def test_project_at_block_edges(fip, oracle, nrows, nchan):
+    """Sample counts below, at and above one moment workgroup, and more
+    partials than the workgroup that adds them up has threads.  Tolerance: two
+    roundings to float (the interchange type), 2 * 6e-8."""
+    rng = np.random.default_rng(1000 * nchan + nrows)
+    uvw = rng.normal(size=(nrows, 3)) * np.array([2e4, 1e4, 1e3])
+    freqs = 140e6 + 1e6 * np.arange(nchan)
+    print(f"project {nrows} x {nchan}", flush=True)
+    B, V = fip.project(uvw, freqs)
+    ob, ov = oracle.project(uvw, freqs)
+    assert np.abs(V - ov).max() <= 1.2e-7
+    assert np.abs(B - ob).max() <= 1.2e-7 * np.abs(ob).max()
