@@ -190,9 +190,9 @@ def image(vis_re, vis_im, bin_, vin, num_baselines: int, image_size: int, num_sn
     """Imaging half: returns (pre [S,I,I], img [S,I,I], max [S])."""
     vr, vi, b, v = _c(vis_re), _c(vis_im), _c(bin_), _c(vin)
     S, I = num_snapshots, image_size
-    pre = np.zeros((S, I, I), dtype=np.float32)
-    img = np.zeros((S, I, I), dtype=np.float32)
-    mx = np.zeros(S, dtype=np.float32)
+    pre = np.empty((S, I, I), dtype=np.float32)
+    img = np.empty((S, I, I), dtype=np.float32)
+    mx = np.empty(S, dtype=np.float32)
     _check(lib.fip_image(_ptr(vr), _ptr(vi), _ptr(b), _ptr(v), num_baselines, I, S, cell_size,
                          _ptr(pre), _ptr(img), _ptr(mx)))
     return pre, img, mx

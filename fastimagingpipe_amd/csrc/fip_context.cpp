@@ -270,6 +270,13 @@ int Context::order_work(hipStream_t st)
     return FIP_OK;
 }
 
+int Context::ensure_copy_events()
+{
+    for (hipEvent_t& e : copy_events)
+        if (!e) FIP_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    return FIP_OK;
+}
+
 int Context::ensure_win012()
 {
     if (win012_ && win.p) return FIP_OK;

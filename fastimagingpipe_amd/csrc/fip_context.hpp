@@ -102,6 +102,11 @@ public:
     DevBuf in_snap;
     hipStream_t copy_stream = nullptr;
     hipEvent_t in_ready[3] = {};
+    // Slots of the image read-back's ring (in `staging`) and their events,
+    // created on first use.
+    static constexpr int kCopySlots = 16;
+    hipEvent_t copy_events[kCopySlots] = {};
+    int ensure_copy_events();
     // Preprocessing (projection, collapse and the raw-input chain): device
     // inputs of the host-array entry points, per-block moment partials and
     // per-snapshot projection parameters.
