@@ -160,13 +160,12 @@ int pipe_host(const void* vis_re, const void* vis_im, int vt, const float* bin, 
     const size_t region = o_v + al(9 * sizeof(float));
     const size_t un = image / tile;
     const size_t rbytes = un * un * sizeof(float);
-    FIP_HIP(C->staging.ensure(S * region + rbytes + S * sizeof(SnapMeta)));
+    FIP_HIP(C->staging.ensure(S * region + rbytes));
     char* hs = static_cast<char*>(C->staging.p);
     FIP_HIP(C->in_snap.ensure(S * region));
     char* ds = C->in_snap.as<char>();
     if (int rc = C->work.ensure(S, nbl, P->t)) return rc;
     if (int rc = C->ensure_win012()) return rc;
-    FIP_HIP(C->out.ensure(rbytes));
     hipStream_t st = C->stream, cs = C->copy_stream;
     if (int rc = C->order_work(st)) return rc;
     // Snapshot s+1 is copied (host -> pinned staging -> device, on the copy
@@ -180,7 +179,52 @@ int pipe_host(const void* vis_re, const void* vis_im, int vt, const float* bin, 
     const WorkView wall = C->work.view(nbl);
     // the third snapshot's splat carries the trigger where it can
     const bool fuse = splat_trigger_fusable(P->t, tu, (int)tile);
+    // Small inputs go up first, in few copies, and through one launch sequence
+    // of three snapshots: three sequences of one take longer on the GPU (346
+    // against 309 us at 4096^2, far more at smaller sizes) and cost the host 35
+    // calls.  Pipelining wins where it hides enough of the copies.  Together
+    // against pipelined: 70 and 199 us at 256^2 with 96 KB, 106 and 214 at 1024^2
+    // with 292 KB, 200 and 280 at 2048^2 with 1.6 MB, 644 and 661 with 14 MB; 367
+    // and 443 at 4096^2 with 1 MB, 527 and 525 with 4.7 MB; at 8192^2 one
+    // snapshot fills the GPU and pipelining is always ahead.
+    const size_t m_vi = al(S * nbl * esz), m_b = m_vi + m_vi, m_v = m_b + al(S * nbl * 2 * sizeof(float));
+    const size_t most = image <= 2048 ? (size_t)16 << 20 : (image <= 4096 ? (size_t)4 << 20 : 0);
+    const bool together = m_v <= most;
+    // A small tLISI is stored by the trigger straight into the pinned memory: a
+    // copy engine's start after the last kernel cost 10 us at 256^2 (1 KB)
+    // and 25 at 4096^2 (64 KB).
+    const bool direct = rbytes <= ((size_t)64 << 10);
+    if (!direct) FIP_HIP(C->out.ensure(rbytes));
+    float* const out = direct ? reinterpret_cast<float*>(hr) : C->out.as<float>();
+    auto finish = [&]() -> int {
+        if (!direct) FIP_HIP(hipMemcpyAsync(hr, out, rbytes, hipMemcpyDeviceToHost, st));
+        return C->mark_work(st);
+    };
     auto enqueue = [&]() -> int {
+        if (together) {
+            const struct {
+                const void* src;
+                size_t off, bytes;
+            } parts[4] = {{vis_re, 0, S * nbl * esz},
+                          {vis_im, m_vi, S * nbl * esz},
+                          {bin, m_b, S * nbl * 2 * sizeof(float)},
+                          {vin, m_v, S * 9 * sizeof(float)}};
+            // The DMA of one piece runs under the host copy of the next.
+            size_t sent = 0;
+            for (const auto& pt : parts)
+                for (size_t o = 0; o < pt.bytes; o += kChunk) {
+                    const size_t n = std::min(kChunk, pt.bytes - o), filled = pt.off + o + n;
+                    std::memcpy(hs + pt.off + o, static_cast<const char*>(pt.src) + o, n);
+                    if (filled - sent < kChunk && &pt != &parts[3]) continue;
+                    FIP_HIP(hipMemcpyAsync(ds + sent, hs + sent, filled - sent, hipMemcpyHostToDevice, st));
+                    sent = filled;
+                }
+            const InputView in{ds, ds + m_vi, reinterpret_cast<const float*>(ds + m_b),
+                               reinterpret_cast<const float*>(ds + m_v), nullptr, nbl, (int)nbl, vt};
+            if (int rc = pipe_sequence(C, P->t, wall, in, (int)nbl, cell, tu, C->win.as<int>(), (int)tile, out, st))
+                return rc;
+            return finish();
+        }
         for (int s = 0; s < S; ++s) {
             const size_t sv = (size_t)s * nbl;
             const struct {
@@ -205,14 +249,11 @@ int pipe_host(const void* vis_re, const void* vis_im, int vt, const float* bin, 
                 return rc;
         }
         if (fuse) {
-            if (int rc = fused_trigger_sequence(C, P->t, wall, (int)tile, C->out.as<float>(), st)) return rc;
-        } else if (int rc = run_trigger(*C, *P, C->work, nbl, C->win.as<int>(), 1, (int)tile, C->out.as<float>(),
-                                        st)) {
+            if (int rc = fused_trigger_sequence(C, P->t, wall, (int)tile, out, st)) return rc;
+        } else if (int rc = run_trigger(*C, *P, C->work, nbl, C->win.as<int>(), 1, (int)tile, out, st)) {
             return rc;
         }
-        FIP_HIP(hipMemcpyAsync(hr, C->out.p, rbytes, hipMemcpyDeviceToHost, st));
-        FIP_HIP(hipMemcpyAsync(hr + rbytes, C->work.meta.p, S * sizeof(SnapMeta), hipMemcpyDeviceToHost, st));
-        return C->mark_work(st);
+        return finish();
     };
     const int erc = enqueue();
     // Also on an error: copies out of the staging buffer may be in flight.
@@ -223,10 +264,14 @@ int pipe_host(const void* vis_re, const void* vis_im, int vt, const float* bin, 
     if (se != hipSuccess) return hip_error(se, "hipStreamSynchronize");
     if (int rc = C->collect_stages()) return rc;
     std::memcpy(result, hr, rbytes);
-    SnapMeta meta[3];
-    std::memcpy(meta, hr + rbytes, sizeof(meta));
-    if (!(max3_from_meta(meta) > 0.0f))
-        return set_error(FIP_ERR_DEGENERATE, "all three images are zero: tLISI divides by maxall^2 = 0");
+    // With all maxima zero every tLISI is 0/0: only then are the maxima
+    // themselves fetched.
+    if (std::isnan(result[0])) {
+        SnapMeta meta[3];
+        FIP_HIP(hipMemcpy(meta, C->work.meta.p, sizeof(meta), hipMemcpyDeviceToHost));
+        if (!(max3_from_meta(meta) > 0.0f))
+            return set_error(FIP_ERR_DEGENERATE, "all three images are zero: tLISI divides by maxall^2 = 0");
+    }
     return FIP_OK;
 }
 

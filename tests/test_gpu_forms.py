@@ -671,3 +671,19 @@ def test_serving_subarrays_full_workload(fip, oracle):
             _check_trigger_sets(tl, ref, err)
     finally:
         srv.close()
+
+
+@pytest.mark.parametrize("image,nbl,tile", [(256, 1, 16), (1024, 8128, 8), (1024, 22000, 7), (512, 349000, 32),
+                                            (512, 350000, 32), (4096, 87000, 32), (4096, 88000, 31),
+                                            (8192, 3000, 32)])
+def test_host_pipe_on_both_sides_of_its_copy_rules(fip, image, nbl, tile):
+    """The host drop-in's two ways with its inputs (together, in pieces; or
+    one snapshot under the other) and with its result (stored by the trigger
+    or copied) give the bits of the images and the trigger taken separately."""
+    cell = 1.45e-5 * 1024 / image
+    print(f"host pipe {image} {nbl} {tile}", flush=True)
+    vr, vi, B, V = snapshots(11 + image, 3, nbl, image, cell)
+    got = fip.fipipe(vr, vi, B, V, nbl, image, 3, cell, tile)
+    _, img, mx = fip.image(vr, vi, B, V, nbl, image, 3, cell)
+    ref = fip.trigger(img[0], img[1], img[2], mx, tile)
+    assert np.array_equal(got.view(np.uint32), ref.view(np.uint32))
