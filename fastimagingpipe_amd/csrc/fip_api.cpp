@@ -193,7 +193,7 @@ int pipe_host(const void* vis_re, const void* vis_im, int vt, const float* bin, 
     // A small tLISI is stored by the trigger straight into the pinned memory: a
     // copy engine's start after the last kernel cost 10 us at 256^2 (1 KB)
     // and 25 at 4096^2 (64 KB).
-    const bool direct = rbytes <= ((size_t)64 << 10);
+    const bool direct = rbytes <= kDirectBytes;
     if (!direct) FIP_HIP(C->out.ensure(rbytes));
     float* const out = direct ? reinterpret_cast<float*>(hr) : C->out.as<float>();
     auto finish = [&]() -> int {

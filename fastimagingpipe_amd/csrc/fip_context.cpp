@@ -358,7 +358,10 @@ int imaging_sequence(Context* C, const PlanTables& p, const WorkView& w, const I
 int trigger_sequence(Context* C, const PlanTables& p, const WorkView& w, const int* win_dev, int nwin, int tile,
                      float* out_dev, hipStream_t st)
 {
-    FIP_STAGE(C, kStTrigger, st, launch_trigger(w, p, win_dev, nwin, tile, out_dev, st));
+    const size_t un = (size_t)(p.I / tile);
+    TriggerOut to{};
+    for (int k = 0; k < kMaxWindows; ++k) to.w[k] = out_dev + (size_t)k * un * un;
+    FIP_STAGE(C, kStTrigger, st, launch_trigger(w, p, win_dev, nwin, tile, to, st));
     return FIP_OK;
 }
 

@@ -183,8 +183,16 @@ hipError_t launch_trigger_finish(const WorkView& w, const PlanTables& p, int s1,
                                  hipStream_t st);
 
 // Trigger over nwin windows; win: device int[3*nwin] of snapshot slots in img.
+// Where each window's tLISI goes (device memory, or pinned host memory).
+constexpr int kMaxWindows = 3;
+struct TriggerOut {
+    float* w[kMaxWindows];
+};
 hipError_t launch_trigger(const WorkView& w, const PlanTables& p, const int* win, int nwin,
-                          int tile, float* out, hipStream_t st);
+                          int tile, const TriggerOut& out, hipStream_t st);
+// tLISI of up to this many bytes are stored by the trigger straight into pinned
+// memory instead of copied there after it.
+constexpr size_t kDirectBytes = (size_t)64 << 10;
 
 // Trigger over the consecutive windows (s0+k, s0+k+1, s0+k+2), k < nwin,
 // reading each image once per group of windows.

@@ -1660,7 +1660,7 @@ __global__ __launch_bounds__(256) void k_trigger_finish(const float* __restrict_
 // 16-byte loads, then wave reductions only (FIPkernels.cu:499-552).
 __global__ __launch_bounds__(256) void k_trigger(const float* __restrict__ img, SnapMeta* __restrict__ meta,
                                                  unsigned* __restrict__ pmax, const int* __restrict__ win, int I,
-                                                 int T, float* __restrict__ out)
+                                                 int T, TriggerOut out)
 {
     const int w = blockIdx.y;
     const int un = I / T;
@@ -1721,7 +1721,7 @@ __global__ __launch_bounds__(256) void k_trigger(const float* __restrict__ img, 
     }
     if (lane == 0) {
         const float m3 = fmaxf(__uint_as_float(m1b), fmaxf(__uint_as_float(m2b), __uint_as_float(m3b)));
-        out[(size_t)w * un * un + tile] = tlisi_value(sum, mx, sr, m3, T);
+        out.w[w][tile] = tlisi_value(sum, mx, sr, m3, T);
     }
 }
 
@@ -1976,11 +1976,12 @@ hipError_t launch_trigger_finish(const WorkView& w, const PlanTables& p, int s1,
     return hipGetLastError();
 }
 
-hipError_t launch_trigger(const WorkView& w, const PlanTables& p, const int* win, int nwin, int tile, float* out,
-                          hipStream_t st)
+hipError_t launch_trigger(const WorkView& w, const PlanTables& p, const int* win, int nwin, int tile,
+                          const TriggerOut& out, hipStream_t st)
 {
     const int un = p.I / tile;
     if (un <= 0 || nwin <= 0) return hipSuccess;
+    if (nwin > kMaxWindows) return hipErrorInvalidValue;
     hipLaunchKernelGGL(k_trigger, dim3((un * un + 3) / 4, nwin), dim3(256), 0, st, w.img, w.meta, w.pmax, win, p.I,
                        tile, out);
     return hipGetLastError();

@@ -387,21 +387,27 @@ int launch_queued(fip_server* srv, SubStream& ss)
     wr.meta = ss.meta.as<SnapMeta>();
     wr.pmax = ss.pmax.as<unsigned>();
     wr.img = ss.img.as<float>();
-    float* dout = ss.out.as<float>();
+    // A small tLISI goes from the trigger into the reservation's pinned mirror.
+    const bool direct = un * un * 4 <= kDirectBytes;
+    auto window_out = [&](int j) {
+        return direct ? reinterpret_cast<float*>(hbase + b[j]->off + L.res) : ss.out.as<float>() + (size_t)(j - j0) * un * un;
+    };
     if (fuse) {
         for (int j = j0; j < k; ++j) {
             const int sa = (int)((b[j]->index - 2) % ring), sb = (int)((b[j]->index - 1) % ring);
             SRV_HIP(launch_splat_trigger(w, p, j, wr.img + (size_t)sa * plane, wr.img + (size_t)sb * plane, true,
                                          st));
-            SRV_HIP(launch_trigger_finish(wr, p, sa, sb, r0 + j, T, dout + (size_t)(j - j0) * un * un, st));
+            SRV_HIP(launch_trigger_finish(wr, p, sa, sb, r0 + j, T, window_out(j), st));
         }
     } else if (j0 < k) {
         // windows (r-2, r-1, r) of ring slots r0+j0 .. r0+k-1, one table row each
-        SRV_HIP(launch_trigger(wr, p, ss.win.as<int>() + 3 * (r0 + j0), k - j0, T, dout, st));
+        static_assert(kServeBatch <= kMaxWindows, "one output per window");
+        TriggerOut to{};
+        for (int j = j0; j < k; ++j) to.w[j - j0] = window_out(j);
+        SRV_HIP(launch_trigger(wr, p, ss.win.as<int>() + 3 * (r0 + j0), k - j0, T, to, st));
     }
-    for (int j = j0; j < k; ++j)
-        SRV_HIP(hipMemcpyAsync(hbase + b[j]->off + L.res, dout + (size_t)(j - j0) * un * un, un * un * 4,
-                               hipMemcpyDeviceToHost, st));
+    for (int j = j0; j < k && !direct; ++j)
+        SRV_HIP(hipMemcpyAsync(hbase + b[j]->off + L.res, window_out(j), un * un * 4, hipMemcpyDeviceToHost, st));
     for (int j = 0; j < k; ++j) {
         b[j]->last = j == k - 1;
         SRV_HIP(hipEventRecord(b[j]->done, st));
@@ -708,15 +714,24 @@ int fip_server_drain(fip_server* srv)
     // sequence ahead of them completes, so the streams are synchronised
     // again until the completion thread has recorded every snapshot.
     const double deadline = now_s() + 120.0;
+    double idle = now_s();   // since when the streams have had nothing to wait for
     for (;;) {
+        const double t0 = now_s();
         for (auto& ss : srv->streams) FIP_HIP(hipStreamSynchronize(ss->hs));
+        const double t = now_s();
+        if (t - t0 > 50e-6) idle = t;
         {
             std::lock_guard<std::mutex> lk(srv->mu);
             if (srv->inflight <= 0) return srv->launch_error ? set_error(srv->launch_error, "a queued launch failed")
                                                              : FIP_OK;
         }
-        if (now_s() > deadline) return set_error(FIP_ERR_HIP, "completions did not arrive");
-        std::this_thread::sleep_for(std::chrono::microseconds(10));
+        if (t > deadline) return set_error(FIP_ERR_HIP, "completions did not arrive");
+        // The completion thread sees an event within microseconds; a sleep
+        // would last the 50 us of this thread's timer slack.
+        if (t - idle < 200e-6)
+            std::this_thread::yield();
+        else
+            std::this_thread::sleep_for(std::chrono::microseconds(10));
     }
 }
 
