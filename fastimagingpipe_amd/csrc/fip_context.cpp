@@ -245,7 +245,7 @@ Tuning default_tuning(size_t image)
     // 4096^2 and 2048^2 on MI355X (each thread's records stay resident up
     // to 1024 per column; heavier columns take further passes).
     t.stage1_records = 2;
-    // What the row pass does: two rows per workgroup, at 8192^2 one.
+    // Without effect (the row pass takes two rows per workgroup everywhere).
     t.stage2_rows = image <= 4096 ? 2 : 1;
     // Up to 512^2 a 64-pixel tile leaves most CUs without a workgroup (16 per
     // image at 256^2) and each one's chain of loads and LDS atomics is the

@@ -104,7 +104,7 @@ struct PlanTables {
     int I, G, M;
     float2* tw_g;      // stage twiddles for the length-G transform
     float2* tw_m;      // stage twiddles for the length-M transform
-    float2* wpost;     // exp(+2 pi i k / G), k < M (C2R split)
+    float2* wpost;     // exp(+2 pi i k / G), k < M (split row pass of 8192^2)
     float* corr;       // 1 / (c(t) * norm), t = 0..I/2
 };
 

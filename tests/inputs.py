@@ -146,3 +146,27 @@ def raw_snapshots(seed: int, nant: int, radius_m: float, nsnap: int, freqs, imag
     w0 = rng.uniform(0.5, 2.0, (nsnap, ns)).astype(np.float32)
     w3 = rng.uniform(0.5, 2.0, (nsnap, ns)).astype(np.float32)
     return uvw, freqs, xx, yy, flag0, flag3, w0, w3
+
+
+def direct_pre_rows(oracle, vr, vi, B, V, image: int, cell: float, rows) -> np.ndarray:
+    """Rows of the corrected image by the sum over each visibility's taps, FP64:
+    the taps are separable, so a row is a sum of n outer products."""
+    g, h = oracle.grid_size(image), image // 2
+    J = abs(float(V[0, 0]) * float(V[1, 1]) - float(V[0, 1]) * float(V[1, 0]))
+
+    def axis(p, at):   # [n, len(at)]: sum over the taps r of ES((r - p)/4) e^{2 pi i r at/g}
+        r = np.ceil(p - 4)[:, None] + np.arange(9)
+        x = (r - p[:, None]) / 4
+        w = np.where(np.abs(x) <= 1, np.exp(15.3704324328 * (np.sqrt(np.maximum(0, 1 - x * x)) - 1)), 0)
+        w = np.where((r >= -(g // 2)) & (r <= g // 2 - 1), w, 0)
+        return (w[:, :, None] * np.exp(2j * np.pi * ((r[:, :, None] * at) % g) / g)).sum(1)
+
+    p = B.astype(np.float64) * (cell * g)
+    y, x = np.asarray(rows) - h, np.arange(image) - h
+    v = (vr.astype(np.float64) + 1j * vi) / J
+    d = np.abs(((v[:, None] * axis(p[:, 0], y)).T @ axis(p[:, 1], x)).real)
+    # conv_corr is of the kernel divided by its integral, 4 int ES(x) dx with x = sin(t)
+    t, wt = np.polynomial.legendre.leggauss(200)
+    t, wt = t * np.pi / 2, wt * np.pi / 2
+    c = oracle.conv_corr(image) * 4.0 * np.sum(np.exp(15.3704324328 * (np.cos(t) - 1)) * np.cos(t) * wt)
+    return d / (c[np.abs(y)][:, None] * c[np.abs(x)][None, :])

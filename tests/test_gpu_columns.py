@@ -6,7 +6,7 @@ than its threads hold.
 import numpy as np
 import pytest
 
-from tests.inputs import rel_rms, rotation
+from tests.inputs import direct_pre_rows, rel_rms, rotation
 
 pytestmark = pytest.mark.gpu
 
@@ -93,3 +93,28 @@ def test_front_end_keeps_every_visibility(fip, oracle, n):
     # cell (rms value 20) round to 5e-4 together, 2.5e-5 of it; the grid
     # correction amplifies that by at most 40 at the image's edge.
     assert err < 1e-3
+
+
+@pytest.mark.parametrize("cmax", [0.0, 3067.6, 3068.6, 3069.6, 4700.2, 6139.9, 6143.5])
+def test_row_pass_of_the_largest_image(fip, oracle, cmax):
+    """8192^2: two rows in two transforms of half the grid.  Columns up to each
+    side of g/4 (where the two halves of the band begin to overlap), to g/2 and
+    clipped there, against the sum over the taps at sixteen rows."""
+    image, n = 8192, 60
+    rng = np.random.default_rng(int(10 * cmax))
+    g = fip.grid_size(image)
+    cell = 2.0 ** -14 * 64 / image
+    p = np.stack([rng.uniform(-0.45, 0.45, n) * g, rng.uniform(-1, 1, n) * cmax], -1)
+    p[:2, 1] = cmax, -cmax
+    p[2:4] = 0.0
+    B = (p / (cell * g)).astype(np.float32)
+    vr, vi = rng.standard_normal((2, n)).astype(np.float32)
+    V = rotation(0.1, 0.3, 0.2).astype(np.float32)
+    pre, _, _ = fip.image(vr, vi, B, V, n, image, 1, cell)
+    rows = np.unique(np.concatenate([[0, 1, 2, 3, 4095, 4096, 8190, 8191], rng.integers(0, image, 8)]))
+    ref = direct_pre_rows(oracle, vr, vi, B, V, image, cell, rows)
+    err = rel_rms(pre[0][rows], ref)
+    print(f"cmax {cmax}: pre rel-rms {err:.2e}")
+    # Twice the bound of the sizes up to 1024 above: a longer transform and the
+    # sum that splits it.
+    assert err < 1e-5
