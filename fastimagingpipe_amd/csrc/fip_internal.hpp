@@ -125,7 +125,9 @@ struct WorkView {
 // The front end's part of the work buffers, with its segments.
 struct BinView {
     VisRec *rec, *sorted;
-    int *boff, *seg;   // per snapshot: key offsets [segment][keys + 1]; extents [3][kMaxSegs]
+    // Per snapshot: key offsets [segment][keys + 1], extents [3][kMaxSegs],
+    // displacements [segment][keys] (of the snapshots' seg_stride too).
+    int *boff, *seg, *disp;
     int* bstart;
     SnapMeta* meta;
     SnapGeom* geom;

@@ -297,9 +297,9 @@ __device__ __forceinline__ void set_extent(SnapMeta& m, int k, int v)
 //
 // Latency bound: at 2048^2 with 32640 visibilities 1.2 us of loads, 1.7 of
 // FP64 and LDS atomics, 1.5 of scan and 0.6 of stores; the rest of its 8 us is
-// launch and write-back.  With k_merge 7, 14, 15, 30 and 70 us (rocprofv3, three
+// launch and write-back.  With k_merge 7, 14, 14, 26 and 58 us (rocprofv3, three
 // snapshots) at 256^2, 1024^2, 2048^2, 4096^2 and 8192^2 with 2016, 8128, 32640,
-// 130816 and 523776 visibilities; clearing, histogram with global atomics, scan
+// 130816 and 523776 visibilities (the last two with k_offsets); clearing, histogram with global atomics, scan
 // and scatter as four launches took 16, 19.5, 22.6, 32 and 74.  (A column
 // kernel that took its records from the sorted segments themselves, with no
 // merge, lost more than the merge costs: 95 against 84 us at 4096^2.)
@@ -467,17 +467,64 @@ __device__ __forceinline__ int4 sum_rows(const int* __restrict__ o, int row, int
     return sum;
 }
 
+// Where many segments' records go: workgroups of 64 keys by 16 groups of
+// segments add boff up once and store the displacement of every segment's
+// records of a key (see k_merge), and the snapshot's offsets.
+__global__ __launch_bounds__(1024) void k_offsets(BinView v, int G)
+{
+    constexpr int GR = 16, PER = kMaxSegs / GR;
+    static_assert(kMaxSegs % GR == 0, "whole groups");
+    __shared__ int part[GR][2][64];
+    const int s = blockIdx.y, lane = threadIdx.x & 63, grp = threadIdx.x >> 6;
+    const int K = bin_keys(G), row = boff_row(G);
+    const int k = blockIdx.x * 64 + lane, ka = min(k, K), kb = min(k + 1, K);
+    const int* bo = v.boff + (size_t)s * v.boff_stride;
+    int a[PER], b[PER], sa = 0, sb = 0;
+#pragma unroll
+    for (int q = 0; q < PER; ++q) {   // segments past the end are read as the last one and masked off
+        const int g = grp * PER + q, m = g < v.nseg ? -1 : 0;
+        const int* o = bo + (size_t)min(g, v.nseg - 1) * row;
+        a[q] = o[ka] & m;
+        b[q] = o[kb] & m;
+    }
+#pragma unroll
+    for (int q = 0; q < PER; ++q) {
+        sa += a[q];
+        sb += b[q];
+    }
+    part[grp][0][lane] = sa;
+    part[grp][1][lane] = sb;
+    __syncthreads();
+    int after = 0, before = 0, total = 0;   // of this key in this group's and later, of the next in earlier segments
+#pragma unroll
+    for (int e = 0; e < GR; ++e) {
+        const int x = part[e][0][lane];
+        total += x;
+        after += e < grp ? 0 : x;
+        before += e < grp ? part[e][1][lane] : 0;
+    }
+    if (grp == 0 && k <= K) v.bstart[(size_t)s * row + k] = total;
+#pragma unroll
+    for (int q = 0; q < PER; ++q) {
+        const int g = grp * PER + q;
+        after -= a[q];
+        if (g < v.nseg && k < K) v.disp[(size_t)s * v.seg_stride + (size_t)g * row + k] = after + before;
+        before += b[q];
+    }
+}
+
 // A snapshot's segments into one column order.  boff[g] is segment g's own
 // exclusive scan, so the scan of the whole snapshot is its sum over the
 // segments, and a record of segment `seg` and key k moves up by the later
 // segments' offsets of k (what they hold before k) and the earlier segments'
-// offsets of k + 1 (what they hold up to k).  Every workgroup adds the rows of
-// offsets up by itself (at most 64, four keys per load, from L2) rather than
-// wait for a launch that does; segment 0's also writes the snapshot's offsets
-// and extent.
+// offsets of k + 1 (what they hold up to k).  Of few segments every workgroup
+// adds the rows of offsets up by itself (four keys per load, from L2) rather
+// than wait for a launch that does, and segment 0's also writes the snapshot's
+// offsets; SUMMED: k_offsets has.  Segment 0 writes the snapshot's extent.
+template <bool SUMMED>
 __global__ __launch_bounds__(kBinThreads) void k_merge(BinView v, int G)
 {
-    extern __shared__ int lds[];   // 2 boff_row(G) ints
+    extern __shared__ int lds[];   // boff_row(G) ints, twice unless SUMMED
     const int s = blockIdx.y, seg = blockIdx.x, t = threadIdx.x;
     const int K = bin_keys(G), row = boff_row(G);
     int* before = lds;
@@ -488,13 +535,18 @@ __global__ __launch_bounds__(kBinThreads) void k_merge(BinView v, int G)
     VisRec* dst = v.sorted + (size_t)s * v.stride;
     auto put = [&](VisRec q, int i) {
         const int key = bin_key((q.col >> 1) + 3 + (q.col & 1));
-        dst[i + after[key] + before[key + 1]] = q;
+        dst[i + (SUMMED ? before[key] : after[key] + before[key + 1])] = q;
     };
     // The first records are loaded before their displacement is known (the
     // segment has at least one place).
     const int last = max(cnt - 1, 0);
     const VisRec r0 = src[min(t, last)], r1 = src[min(t + kBinThreads, last)];
     for (int b = 4 * t; b < row; b += 4 * kBinThreads) {
+        if constexpr (SUMMED) {
+            *reinterpret_cast<int4*>(before + b) = *reinterpret_cast<const int4*>(
+                v.disp + (size_t)s * v.seg_stride + (size_t)seg * row + b);
+            continue;
+        }
         const int4 lo = sum_rows(bo + b, row, 0, seg), hi = sum_rows(bo + b, row, seg + 1, v.nseg);
         *reinterpret_cast<int4*>(before + b) = lo;
         *reinterpret_cast<int4*>(after + b) = hi;
@@ -1824,11 +1876,17 @@ const char* stage_name(int st)
     return (st >= 0 && st < kStCount) ? names[st] : "?";
 }
 
-// Segments of a snapshot of up to n visibilities and their length: 2 or 4
-// visibilities per thread while that is at most 32 segments, then 8 up to 64
-// segments (a workgroup sorts 2048 visibilities in 7 us, 4096 in 16 and 8192
-// in 17 to 33, its FP64 and LDS atomics; every merging workgroup adds all
-// segments' offsets up); beyond 64 * 8192 visibilities, 64 equal segments.
+// Segments of a snapshot of up to n visibilities and their length: the fewest
+// visibilities per thread (2, 4 or 8) that need at most 64 segments (a
+// workgroup sorts 2048 visibilities in 8 to 12 us, 4096 in 16 and 8192 in 17 to
+// 33, its FP64 and LDS atomics); beyond 64 * 8192 visibilities, 64 equal
+// segments.
+//
+// Up to kOwnSums segments the merging workgroups add the offsets up themselves:
+// bin and merge of three snapshots take 18.2 us with 38 segments (77777
+// visibilities at 2048^2), with k_offsets between them 19.5; with 49 (100000
+// at 4096^2) 27.9 and 24.3, with 64 (523776 at 8192^2) 69.8 and 58.4.
+constexpr int kOwnSums = 40;
 struct SegShape {
     int vpt, chunk, nseg;
 };
@@ -1836,7 +1894,7 @@ static SegShape seg_shape(int n)
 {
     constexpr int B = kBinThreads;
     SegShape q;
-    q.vpt = n <= 64 * B ? 2 : (n <= 128 * B ? 4 : (n <= kMaxSegs * 8 * B ? 8 : 0));
+    q.vpt = n <= 2 * kMaxSegs * B ? 2 : (n <= 4 * kMaxSegs * B ? 4 : (n <= 8 * kMaxSegs * B ? 8 : 0));
     const int each = (n + kMaxSegs - 1) / kMaxSegs;
     q.chunk = q.vpt > 0 ? q.vpt * B : (each + B - 1) / B * B;
     q.nseg = max(1, (n + q.chunk - 1) / q.chunk);
@@ -1868,13 +1926,14 @@ hipError_t launch_bin(const InputView& in, const WorkView& w, const PlanTables& 
 {
     if (p.G > kMaxGrid) return hipErrorInvalidValue;
     const SegShape q = seg_shape(nmax);
-    // The segments' offsets and extents are only read by the merge: they lie
-    // in each snapshot's corrected image and K tiles, which later stages write
-    // (64 (g/2 + 14) ints in I^2 floats, 192 ints in I (g/2 + 1) pairs: I >= 64).
+    // The segments' offsets, extents and displacements are only read by the
+    // merge: they lie in each snapshot's corrected image and K tiles, which later
+    // stages write (64 (g/2 + 16) ints in I^2 floats, 256 more in I (g/2 + 1)
+    // pairs: I >= 64).
     const size_t plane = (size_t)p.I * p.I, tiles = (size_t)p.I * (p.M + 1) * 2;
-    const BinView v{w.rec,  w.sorted, reinterpret_cast<int*>(w.pre), reinterpret_cast<int*>(w.kt), w.bstart, w.meta,
-                    w.geom, w.pmax,   w.stride,                      plane,                        tiles,    q.nseg,
-                    q.chunk};
+    int* const kt = reinterpret_cast<int*>(w.kt);
+    const BinView v{w.rec,  w.sorted, reinterpret_cast<int*>(w.pre), kt, kt + 256, w.bstart, w.meta, w.geom, w.pmax,
+                    w.stride, plane, tiles, q.nseg, q.chunk};
     switch (in.vis_type) {
     case kVisF32: bin_dispatch<float>(in, v, q.vpt, p, S, cell, scale, norm_n_dev, norm_n_const, st); break;
     case kVisBF16: bin_dispatch<__hip_bfloat16>(in, v, q.vpt, p, S, cell, scale, norm_n_dev, norm_n_const, st); break;
@@ -1883,7 +1942,15 @@ hipError_t launch_bin(const InputView& in, const WorkView& w, const PlanTables& 
     }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || q.nseg == 1) return e;
-    hipLaunchKernelGGL(k_merge, dim3(q.nseg, S), dim3(kBinThreads), 2 * (size_t)boff_row(p.G) * sizeof(int), st, v, p.G);
+    const size_t row = (size_t)boff_row(p.G) * sizeof(int);
+    if (q.nseg <= kOwnSums) {
+        hipLaunchKernelGGL(k_merge<false>, dim3(q.nseg, S), dim3(kBinThreads), 2 * row, st, v, p.G);
+        return hipGetLastError();
+    }
+    hipLaunchKernelGGL(k_offsets, dim3((bin_keys(p.G) + 1 + 63) / 64, S), dim3(1024), 0, st, v, p.G);
+    e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(k_merge<true>, dim3(q.nseg, S), dim3(kBinThreads), row, st, v, p.G);
     return hipGetLastError();
 }
 

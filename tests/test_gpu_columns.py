@@ -68,7 +68,7 @@ def test_crowded_columns_do_not_depend_on_the_order(fip, image, n):
     assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
 
 
-@pytest.mark.parametrize("n", [1, 2047, 2048, 2049, 65537, 131073, 524289])
+@pytest.mark.parametrize("n", [1, 2047, 2048, 2049, 65537, 81920, 81921, 131073, 262145, 524289])
 def test_front_end_keeps_every_visibility(fip, oracle, n):
     """Counts around a sorting workgroup's 2048 visibilities and around each
     change of its visibilities per thread.  A visibility lost or taken twice by
