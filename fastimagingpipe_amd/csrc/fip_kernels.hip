@@ -1728,7 +1728,13 @@ __global__ __launch_bounds__(256) void k_trigger_finish(const float* __restrict_
 // --------------------------------------------------------------- trigger
 
 // One wave per tile (four tiles per workgroup): per-lane partial sums over
-// 16-byte loads, then wave reductions only (FIPkernels.cu:499-552).
+// 16-byte loads, then wave reductions only (FIPkernels.cu:499-552).  A tile
+// whose edge is no multiple of four pixels takes 4-byte loads, of eight turns
+// together where a lane has more than two pixels: at tile 50 (40 pixels a lane)
+// 20 -> 9 us at 1024^2, 19 -> 12 at 2048^2 and 43 -> 40 at 4096^2 (201 MB, 5
+// TB/s); with one or two, the set-up would cost 2 to 5% (tile 3 to 9).
+enum TriggerMode { kTrigWide, kTrigDeep, kTrigSmall };
+template <TriggerMode MODE>
 __global__ __launch_bounds__(256) void k_trigger(const float* __restrict__ img, SnapMeta* __restrict__ meta,
                                                  unsigned* __restrict__ pmax, const int* __restrict__ win, int I,
                                                  int T, TriggerOut out)
@@ -1748,7 +1754,7 @@ __global__ __launch_bounds__(256) void k_trigger(const float* __restrict__ img, 
     const float* d3 = img + (size_t)s3 * I * I;
     float sum = 0.0f, mx = 0.0f, sr = 0.0f;
     auto px = [&](float a, float b, float c) { tlisi_px(a, b, c, sum, mx, sr); };
-    if ((T & 3) == 0) {
+    if constexpr (MODE == kTrigWide) {
         // 16-byte loads: rows of a tile start at multiples of 4 floats; the
         // loads of four passes are issued together.
         const int T4 = T >> 2, n4 = T * T4;
@@ -1773,6 +1779,32 @@ __global__ __launch_bounds__(256) void k_trigger(const float* __restrict__ img, 
                     px(a[u].w, b[u].w, c[u].w);
                 }
             }
+        }
+    } else if constexpr (MODE == kTrigDeep) {
+        // eight turns' loads together, the places stepped instead of divided
+        constexpr int U = 8;
+        const int drow = 64 / T, dcol = 64 % T;
+        int row = lane / T, col = lane % T;
+        for (int p0 = lane; p0 < T * T; p0 += U * 64) {
+            float a[U], b[U], c[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                if (p0 + u * 64 < T * T) {
+                    const size_t q = (size_t)(ti * T + row) * I + (size_t)(tj * T + col);
+                    a[u] = d1[q];
+                    b[u] = d2[q];
+                    c[u] = d3[q];
+                }
+                row += drow;
+                col += dcol;
+                if (col >= T) {
+                    col -= T;
+                    ++row;
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                if (p0 + u * 64 < T * T) px(a[u], b[u], c[u]);
         }
     } else {
         for (int p = lane; p < T * T; p += 64) {
@@ -2068,8 +2100,16 @@ hipError_t launch_trigger(const WorkView& w, const PlanTables& p, const int* win
     const int un = p.I / tile;
     if (un <= 0 || nwin <= 0) return hipSuccess;
     if (nwin > kMaxWindows) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_trigger, dim3((un * un + 3) / 4, nwin), dim3(256), 0, st, w.img, w.meta, w.pmax, win, p.I,
-                       tile, out);
+    auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3((un * un + 3) / 4, nwin), dim3(256), 0, st, w.img, w.meta, w.pmax, win, p.I,
+                           tile, out);
+    };
+    if (tile % 4 == 0)
+        go(k_trigger<kTrigWide>);
+    else if (tile * tile > 128)
+        go(k_trigger<kTrigDeep>);
+    else
+        go(k_trigger<kTrigSmall>);
     return hipGetLastError();
 }
 
