@@ -1205,7 +1205,7 @@ __device__ __forceinline__ void sin_shift(const SnapGeom& g, double q1, double q
     const float mm = (float)(g.delta * (q2 - 1.0));
     const float r2 = l * l + mm * mm;
     if (g.series) {
-        // every source of the image has r^2 <= 0.01 (checked in k_reset)
+        // every source of the image has r^2 <= 0.01 (checked in snap_geometry)
         const float np = r2 * fmaf(r2, fmaf(r2, fmaf(r2, 0.0390625f, 0.0625f), 0.125f), 0.5f);
         o1 = q1 + g.sx * (double)np;
         o2 = q2 + g.sy * (double)np;
@@ -1538,7 +1538,7 @@ __global__ __launch_bounds__(256, 8) void k_splat(const float* __restrict__ pre,
                     // (Q1 + B1 k + C1 k^2, Q2 + B2 k + C2 k^2) relative to the
                     // origin, the affine step plus the quadratic Taylor model in
                     // k of the SIN shift (sx, sy) n'(k) (its remainder is
-                    // bounded in k_reset).  With r^2(k) = R0 + R1 k + R2 k^2 and
+                    // bounded in snap_geometry).  With r^2(k) = R0 + R1 k + R2 k^2 and
                     // the series f(x) = x/2 + x^2/8 + x^3/16 + 5x^4/128,
                     // n'(k) ~ f(R0) + f'(R0) R1 k + (f'(R0) R2 + f''(R0) R1^2 / 2) k^2.
                     float Q1 = r1, B1 = g.fm00, C1 = 0.0f, Q2 = r2, B2 = g.fm10, C2 = 0.0f;
@@ -1571,7 +1571,7 @@ __global__ __launch_bounds__(256, 8) void k_splat(const float* __restrict__ pre,
                                 const float rr = l * l + mm * mm;
                                 float np = 0.0f;
                                 if (ser < 0 && g.series) {
-                                    // every source of the image has r^2 <= 0.01 (checked in k_reset)
+                                    // every source of the image has r^2 <= 0.01 (checked in snap_geometry)
                                     np = rr * fmaf(rr, fmaf(rr, fmaf(rr, 0.0390625f, 0.0625f), 0.125f), 0.5f);
                                 } else if (rr <= 1.0f) {
                                     // 1 - sqrt(1 - r^2) = r^2 / (1 + sqrt(1 - r^2)); hardware sqrt/rcp

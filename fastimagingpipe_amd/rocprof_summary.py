@@ -32,9 +32,10 @@ import sys
 from collections import defaultdict
 
 # Kernel name pattern -> pipeline stage (the names the library's per-stage
-# event timing reports, where the merge counts to "bin").
+# event timing reports, where offsets and merge count to "bin").
 STAGES = [
-    (r"k_bin", "bin"), (r"k_merge", "merge"), (r"k_stage1", "grid_colfft"), (r"k_stage2", "row_c2r"),
+    (r"k_bin", "bin"), (r"k_offsets", "offsets"), (r"k_merge", "merge"), (r"k_stage1", "grid_colfft"),
+    (r"k_stage2", "row_c2r"),
     (r"k_splat<\d+, true>", "splat_trigger"), (r"k_splat", "splat"), (r"k_trigger", "trigger"),
 ]
 COPY_PATTERN = r"copyBuffer|Copy"
