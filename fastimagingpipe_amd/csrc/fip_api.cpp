@@ -61,18 +61,25 @@ struct ReadBack {
 // DMA fills a ring of pinned chunks and up to kCopyThreads threads, which live for
 // this call only, move them out.  Chunk k goes through slot k % kSlots and
 // belongs to thread k % T; the DMA of a chunk is enqueued once the slot's
-// previous chunk has left.  Below two chunks per thread the plain copy is as
-// fast.
+// previous chunk has left.  With less than two chunks for each of two threads the
+// plain copy is as fast.
+//
+// Six images of 4 MB: 888 us with chunks of 2 MB and four threads; 1040 of 1 MB and
+// eight, 1450 of half a MB (each chunk's DMA and event cost about 20 us beside
+// its bytes), 860 of 3 MB, which are slower at 512^2 (420 against 371 us).
+constexpr size_t kBackChunk = (size_t)2 << 20;
+constexpr int kSlots = Context::kCopySlots, kCopyThreads = 4;
+
+// Piece of a host array that is copied to pinned memory and sent.
 constexpr size_t kChunk = (size_t)1 << 20;
-constexpr int kSlots = Context::kCopySlots, kCopyThreads = 8;
 
 int read_back(Context& C, const ReadBack* parts, int nparts, hipStream_t st)
 {
     std::vector<ReadBack> chunks;
     for (int i = 0; i < nparts; ++i)
-        for (size_t o = 0; o < parts[i].bytes; o += kChunk)
+        for (size_t o = 0; o < parts[i].bytes; o += kBackChunk)
             chunks.push_back({static_cast<char*>(parts[i].dst) + o, static_cast<const char*>(parts[i].src) + o,
-                              std::min(kChunk, parts[i].bytes - o)});
+                              std::min(kBackChunk, parts[i].bytes - o)});
     const size_t K = chunks.size();
     const size_t cpus = std::max(1u, std::thread::hardware_concurrency());
     std::vector<std::thread> threads;
@@ -83,7 +90,7 @@ int read_back(Context& C, const ReadBack* parts, int nparts, hipStream_t st)
             FIP_HIP(hipMemcpy(parts[i].dst, parts[i].src, parts[i].bytes, hipMemcpyDeviceToHost));
         return FIP_OK;
     }
-    FIP_HIP(C.staging.ensure(kSlots * kChunk));
+    FIP_HIP(C.staging.ensure(kSlots * kBackChunk));
     if (int rc = C.ensure_copy_events()) return rc;
     char* ring = static_cast<char*>(C.staging.p);
     std::atomic<size_t> enqueued{0};
@@ -106,7 +113,7 @@ int read_back(Context& C, const ReadBack* parts, int nparts, hipStream_t st)
                 failed.store((int)e, std::memory_order_release);
                 return;
             }
-            std::memcpy(chunks[k].dst, ring + (k % kSlots) * kChunk, chunks[k].bytes);
+            std::memcpy(chunks[k].dst, ring + (k % kSlots) * kBackChunk, chunks[k].bytes);
             moved[k % kSlots].fetch_add(1, std::memory_order_release);
         }
     };
@@ -121,7 +128,7 @@ int read_back(Context& C, const ReadBack* parts, int nparts, hipStream_t st)
         const size_t slot = k % kSlots;
         while (moved[slot].load(std::memory_order_acquire) < k / kSlots && !stop()) std::this_thread::yield();
         if (stop()) break;
-        hipError_t e = hipMemcpyAsync(ring + slot * kChunk, chunks[k].src, chunks[k].bytes, hipMemcpyDeviceToHost, st);
+        hipError_t e = hipMemcpyAsync(ring + slot * kBackChunk, chunks[k].src, chunks[k].bytes, hipMemcpyDeviceToHost, st);
         if (e == hipSuccess) e = hipEventRecord(C.copy_events[slot], st);
         if (e != hipSuccess) {
             failed.store((int)e, std::memory_order_release);

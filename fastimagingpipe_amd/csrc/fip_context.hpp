@@ -104,7 +104,7 @@ public:
     hipEvent_t in_ready[3] = {};
     // Slots of the image read-back's ring (in `staging`) and their events,
     // created on first use.
-    static constexpr int kCopySlots = 16;
+    static constexpr int kCopySlots = 8;
     hipEvent_t copy_events[kCopySlots] = {};
     int ensure_copy_events();
     // Preprocessing (projection, collapse and the raw-input chain): device

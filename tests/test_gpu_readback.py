@@ -9,7 +9,7 @@ from tests.inputs import snapshots
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("image,nsnap", [(128, 2), (128, 41), (512, 3), (1024, 3), (2048, 5)])
+@pytest.mark.parametrize("image,nsnap", [(128, 2), (128, 41), (128, 130), (512, 3), (1024, 3), (2048, 5)])
 def test_image_readback_equals_single_snapshots(fip, image, nsnap):
     cell, nbl = 1.45e-5 * 1024 / image, 1500
     vr, vi, B, V = snapshots(50 + image, nsnap, nbl, image, cell)
