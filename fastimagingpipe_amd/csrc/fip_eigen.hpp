@@ -15,18 +15,22 @@ namespace fip {
 // constants once unrolled: on the GPU the matrices stay in registers.
 
 // Cyclic Jacobi on a symmetric 3x3 matrix a (destroyed).  evec columns are
-// the eigenvectors of eval.  It ends once the off-diagonal is below 1e-25 of the
-// diagonal: a further rotation's sine is then far below an ulp of the vectors
-// (unless two eigenvalues agree to 1e-9, where they are not determined by
-// the data).
+// the eigenvectors of eval.  It ends once every rotation left would be by less
+// than 1e-30, which changes no vector in FP64: an off-diagonal entry is compared
+// with the gap of its own two diagonal entries, since one that is small against
+// the largest eigenvalue can still decide the directions of the smaller ones (a
+// nearly linear array).
 __host__ __device__ inline void jacobi3(double a[3][3], double evec[3][3], double eval[3])
 {
 #pragma clang fp contract(off)
     double v[3][3] = {{1, 0, 0}, {0, 1, 0}, {0, 0, 1}};
 #pragma unroll 1
     for (int sweep = 0; sweep < 64; ++sweep) {
-        const double off = std::fabs(a[0][1]) + std::fabs(a[0][2]) + std::fabs(a[1][2]);
-        if (off <= 1e-25 * (std::fabs(a[0][0]) + std::fabs(a[1][1]) + std::fabs(a[2][2]))) break;
+        constexpr double tiny = 1e-30;
+        if (std::fabs(a[0][1]) <= tiny * std::fabs(a[0][0] - a[1][1]) &&
+            std::fabs(a[0][2]) <= tiny * std::fabs(a[0][0] - a[2][2]) &&
+            std::fabs(a[1][2]) <= tiny * std::fabs(a[1][1] - a[2][2]))
+            break;
 #pragma unroll
         for (int p = 0; p < 2; ++p) {
 #pragma unroll

@@ -98,3 +98,15 @@ def test_project_at_block_edges(fip, oracle, nrows, nchan):
     ob, ov = oracle.project(uvw, freqs)
     assert np.abs(V - ov).max() <= 1.2e-7
     assert np.abs(B - ob).max() <= 1.2e-7 * np.abs(ob).max()
+
+
+@pytest.mark.parametrize("log2_ratio", [4, 30, 44, 60])
+def test_project_nearly_linear_array(fip, log2_ratio):
+    """Baselines along u, and far shorter ones along (0, 3, 4): the second axis
+    is decided by covariances 2^-2k of the first one's variance, which cancel
+    exactly against it here.  Tolerance: the rounding to float."""
+    u, s = 2.0 ** 10, 2.0 ** (10 - log2_ratio)
+    uvw = np.array([[u, 0, 0], [-u, 0, 0], [0, 3 * s, 4 * s], [0, -3 * s, -4 * s]])
+    _, V = fip.project(uvw, [299792458.0])
+    expect = np.array([[1, 0, 0], [0, 0.6, 0.8], [0, -0.8, 0.6]])
+    assert np.abs(V - expect).max() <= 6e-8
