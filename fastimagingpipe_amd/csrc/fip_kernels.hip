@@ -945,9 +945,10 @@ __global__ __launch_bounds__(ColShape<G>::NX, ColShape<G>::waves) void k_stage1(
     __shared__ float sc[Sh::NBLK], isc[Sh::NBLK];
     // Column-major over snapshots: the heavily populated low columns of
     // every snapshot are dispatched first, so none of them ends the launch.
-    const int S = (int)(gridDim.x / (G / 2 + 1));
-    const int s = (int)(blockIdx.x % S);
-    const int c = (int)(blockIdx.x / S);
+    // On two axes: one of (g/2 + 1) S workgroups would pass the 2^32 threads
+    // that an axis may hold from 43241 snapshots of 128^2 or 5455 of 1024^2 on.
+    const int s = (int)blockIdx.x;
+    const int c = (int)blockIdx.y;
     // The runs do not depend on the metadata: both loads are in flight
     // together.
     const int4 rg = column_ranges<G>(bstart + (size_t)s * boff_row(G), c);
@@ -1989,8 +1990,8 @@ hipError_t launch_bin(const InputView& in, const WorkView& w, const PlanTables& 
 template <int G, int KR>
 static void stage1_dispatch(const WorkView& w, const PlanTables& p, int S, hipStream_t st)
 {
-    hipLaunchKernelGGL((k_stage1<G, KR>), dim3((G / 2 + 1) * S), dim3(ColShape<G>::NX), 0, st, w.sorted, w.bstart,
-                       w.meta, p.tw_g, w.kt, w.stride);
+    hipLaunchKernelGGL((k_stage1<G, KR>), dim3(S, G / 2 + 1), dim3(ColShape<G>::NX), 0, st, w.sorted, w.bstart, w.meta,
+                       p.tw_g, w.kt, w.stride);
 }
 
 // Records per thread held in registers while a column is gridded.
