@@ -601,7 +601,7 @@ int fip_batch_device(const void* vis_re, const void* vis_im, int vis_type, const
         std::memcpy(&key.cell_bits, &cell_size, 4);
         key.t0 = tu.stage1_records;
         key.t1 = tu.stage2_rows;
-        key.t2 = tu.splat_tile;
+        key.t2 = splat_tile_for(tu, (int)image_size, S);
         key.t3 = tu.persistent;
         key.nmax = nmax;   // sizes the bin/scatter grids baked into the graph
         key.work_gen = C->work.gen;
@@ -723,7 +723,7 @@ int fip_set_tuning(size_t image_size, const int* choice)
     Tuning t;
     t.stage1_records = choice[0];
     t.stage2_rows = choice[1];
-    t.splat_tile = choice[2];
+    t.splat_tile = choice[2] >= 64 ? 64 : 32;
     t.persistent = choice[3];
     C->set_tuning(image_size, t);
     return FIP_OK;

@@ -247,12 +247,7 @@ Tuning default_tuning(size_t image)
     t.stage1_records = 2;
     // Without effect (the row pass takes two rows per workgroup everywhere).
     t.stage2_rows = image <= 4096 ? 2 : 1;
-    // Up to 512^2 a 64-pixel tile leaves most CUs without a workgroup (16 per
-    // image at 256^2) and each one's chain of loads and LDS atomics is the
-    // launch: 32-pixel tiles take a call from 37 to 33 us at 256^2 and from 47
-    // to 44 at 512^2 (2016 and 4000 visibilities); at 1024^2 59 -> 63, where
-    // there are enough and the smaller tiles' borders count.
-    t.splat_tile = image <= 512 ? 32 : 64;
+    t.splat_tile = 0;
     t.persistent = 0;
     return t;
 }

@@ -140,7 +140,7 @@ struct BinView {
 struct Tuning {
     int stage1_records;   // gridding records per thread held in registers (2, 4, 8)
     int stage2_rows;    // accepted and kept; the row pass has one launch form
-    int splat_tile;     // target tile edge of the splat (32 or 64)
+    int splat_tile;     // target tile edge of the splat (32 or 64; 0: splat_tile_for)
     int persistent;     // accepted and kept; the column kernel has one launch form
 };
 
@@ -167,6 +167,9 @@ hipError_t launch_bin(const InputView& in, const WorkView& w, const PlanTables& 
 hipError_t launch_stage1(const WorkView& w, const PlanTables& p, int S, const Tuning& tu,
                          hipStream_t st);
 hipError_t launch_stage2(const WorkView& w, const PlanTables& p, int S, hipStream_t st);
+// Target tile edge of a splat of S snapshots: the tuning's, or by the size of the
+// launch where that leaves it open.
+int splat_tile_for(const Tuning& tu, int I, int S);
 // Splat of snapshots 0..S-1 of the view.
 hipError_t launch_splat(const WorkView& w, const PlanTables& p, int S, const Tuning& tu,
                         hipStream_t st);

@@ -2048,10 +2048,25 @@ hipError_t launch_stage2(const WorkView& w, const PlanTables& p, int S, hipStrea
     return hipGetLastError();
 }
 
+// Two 64-pixel tiles per CU are enough to fill the GPU; with fewer, each
+// workgroup's chain of loads and LDS atomics is the launch, and 32-pixel tiles
+// are shorter although their borders are read twice: a call of three snapshots
+// takes 33 instead of 37 us at 256^2 and 44 instead of 47 at 512^2 (2016 and 4000
+// visibilities).  Batches of 4, 16, 64 and 256 snapshots at 512^2 take 57, 88,
+// 198 and 710 us with 32-pixel tiles and 59, 84, 181 and 618 with 64-pixel
+// ones; the lines cross at 450 to 670 of the larger tiles from 64^2 to 512^2.  From
+// 1024^2 on one image has 256 of them, and a call of three takes 59 us against 63
+// with the smaller ones.
+int splat_tile_for(const Tuning& tu, int I, int S)
+{
+    if (tu.splat_tile != 0) return tu.splat_tile >= 64 ? 64 : 32;
+    return I > 512 || (long)S * (I / 64) * (I / 64) >= 512 ? 64 : 32;
+}
+
 hipError_t launch_splat(const WorkView& w, const PlanTables& p, int S, const Tuning& tu, hipStream_t st)
 {
     if (S <= 0) return hipSuccess;
-    if (tu.splat_tile >= 64 && p.I % 64 == 0) {
+    if (splat_tile_for(tu, p.I, S) == 64) {
         const int nt = (p.I / 64) * (p.I / 64);
         hipLaunchKernelGGL((k_splat<64, false>), dim3(nt, S), dim3(256), 0, st, w.pre, w.meta, w.geom, w.pmax, w.img,
                            p.I, 0, nullptr, nullptr, nullptr, 1);
@@ -2069,7 +2084,7 @@ bool splat_trigger_fusable(const PlanTables& p, const Tuning& tu, int tile)
     // splat over all snapshots with the trigger after it is shorter: 59 against
     // 70 us per call at 1024^2 (8128 visibilities), 105 against 108 at 2048^2
     // (32640), but 311 against 302 at 4096^2 (130816).
-    return p.I >= 4096 && tu.splat_tile >= 64 && p.I % 64 == 0 && tile == 32;
+    return p.I >= 4096 && splat_tile_for(tu, p.I, 1) == 64 && tile == 32;
 }
 
 // The reduced trigger terms go to the K tiles' buffer, which the column and
