@@ -547,8 +547,10 @@ int fip_batch_device(const void* vis_re, const void* vis_im, int vis_type, const
         const int S = (int)nsnap;
         if (int rc = C->work.ensure(S, stride, P->t)) return rc;
         BatchGraph& bg = batch_graph();
-        // Per-snapshot counts: upload only when they change (stream-ordered
-        // before the graph that reads them).
+        // Per-snapshot counts: uploaded only when they change, once every
+        // earlier use of the library has ended, on whichever stream it was:
+        // that may be another batch, which reads the counts it came with.
+        if (int rc = C->order_work(st)) return rc;
         if (bg.nvis_cached.size() != nsnap || !std::equal(nvis, nvis + nsnap, bg.nvis_cached.begin())) {
             FIP_HIP(hipStreamSynchronize(st));
             FIP_HIP(bg.nvis_d.ensure(nsnap * sizeof(int)));
@@ -576,7 +578,6 @@ int fip_batch_device(const void* vis_re, const void* vis_im, int vis_type, const
             // windows (k, k+1, k+2): the run form reads each image once per 8 windows
             return run_trigger_run(*C, *P, C->work, stride, 0, S - 2, (int)unit_size, d_tlisi, st);
         };
-        if (int rc = C->order_work(st)) return rc;
         if (C->profiling) {
             // Eager launches with per-stage events (no graph).
             if (int rc = enqueue()) return rc;

@@ -2,6 +2,7 @@
 import numpy as np
 import pytest
 
+from fastimagingpipe_amd import hip
 from tests.inputs import snapshots
 
 pytestmark = pytest.mark.gpu
@@ -36,3 +37,24 @@ def test_batch_on_both_sides_of_the_splat_tile_rule(fip, image, S):
         q = [(r + j) % 3 for j in range(3)]
         ref = fip.trigger(img[q[0]][0], img[q[1]][0], img[q[2]][0], np.array([mx[j][0] for j in q]), tile)
         assert np.array_equal(got[r::3].view(np.uint32), np.broadcast_to(ref.view(np.uint32), got[r::3].shape))
+
+
+def test_batches_on_two_streams_keep_their_counts(fip):
+    """A batch whose turn has not come yet keeps the counts it was called with,
+    although another one with other counts is called on another stream."""
+    image, nbl, tile, S = 512, 3000, 32, 64
+    cell = 1.45e-5 * 1024 / image
+    vr, vi, B, V = (a[np.arange(S) % 3] for a in snapshots(29, 3, nbl, image, cell))
+    counts = [np.full(S, nbl, np.int32), np.where(np.arange(S) % 3 == 1, nbl // 2, nbl).astype(np.int32)]
+    ref = [fip.batch_host(vr, vi, B, V, nv, nbl, image, cell, tile) for nv in counts]
+    assert not np.array_equal(ref[0], ref[1])
+    dev = [hip.DeviceArray(np.ascontiguousarray(a)) for a in (vr, vi, B, V)]
+    out = [hip.DeviceArray(nbytes=ref[0].nbytes) for _ in range(2)]
+    other = hip.Stream()
+    for which in (0, 0, 1):   # the first two one after the other on the library's stream
+        fip.batch_device(dev[0].addr, dev[1].addr, fip.VIS_F32, dev[2].addr, dev[3].addr, counts[which], nbl, S, nbl,
+                         image, cell, tile, out[which].addr, stream=other.addr if which else 0)
+    hip.synchronize()
+    for which in (0, 1):
+        got = out[which].to_host(np.float32, ref[0].shape)
+        assert np.array_equal(got.view(np.uint32), ref[which].view(np.uint32)), which
