@@ -493,7 +493,7 @@ struct BatchKey {
     size_t stride, nsnap, norm_n, image, tile;
     int vis_type;
     uint32_t cell_bits;
-    int t0, t1, t2, t3;
+    int records, splat_tile;   // what of the tuning the launches depend on
     int nmax;
     unsigned long long work_gen;   // the work buffers' addresses are baked into the graph
     bool operator==(const BatchKey& o) const { return std::memcmp(this, &o, sizeof(BatchKey)) == 0; }
@@ -505,8 +505,7 @@ struct BatchGraph {
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
     std::vector<int> nvis_cached;
-    DevBuf nvis_d, win_d;
-    size_t win_for = 0;
+    DevBuf nvis_d;
 };
 
 BatchGraph& batch_graph()
@@ -557,18 +556,6 @@ int fip_batch_device(const void* vis_re, const void* vis_im, int vis_type, const
             FIP_HIP(hipMemcpy(bg.nvis_d.p, nvis, nsnap * sizeof(int), hipMemcpyHostToDevice));
             bg.nvis_cached.assign(nvis, nvis + nsnap);
         }
-        if (bg.win_for != nsnap) {
-            std::vector<int> w(3 * (nsnap - 2));
-            for (size_t k = 0; k + 2 < nsnap; ++k) {
-                w[3 * k] = (int)k;
-                w[3 * k + 1] = (int)k + 1;
-                w[3 * k + 2] = (int)k + 2;
-            }
-            FIP_HIP(hipStreamSynchronize(st));
-            FIP_HIP(bg.win_d.ensure(w.size() * sizeof(int)));
-            FIP_HIP(hipMemcpy(bg.win_d.p, w.data(), w.size() * sizeof(int), hipMemcpyHostToDevice));
-            bg.win_for = nsnap;
-        }
         const Tuning tu = C->tuning(image_size);
         InputView in{vis_re, vis_im, bin, vin, bg.nvis_d.as<int>(), stride, 0, vis_type};
         const int* norm_dev = norm_n == 0 ? bg.nvis_d.as<int>() : nullptr;
@@ -600,11 +587,9 @@ int fip_batch_device(const void* vis_re, const void* vis_im, int vis_type, const
         key.tile = unit_size;
         key.vis_type = vis_type;
         std::memcpy(&key.cell_bits, &cell_size, 4);
-        key.t0 = tu.stage1_records;
-        key.t1 = tu.stage2_rows;
-        key.t2 = splat_tile_for(tu, (int)image_size, S);
-        key.t3 = tu.persistent;
-        key.nmax = nmax;   // sizes the bin/scatter grids baked into the graph
+        key.records = tu.stage1_records;
+        key.splat_tile = splat_tile_for(tu, (int)image_size, S);
+        key.nmax = nmax;   // picks the front end's segments and grids baked into the graph
         key.work_gen = C->work.gen;
         if (!bg.valid || !(bg.key == key)) {
             if (bg.exec) (void)hipGraphExecDestroy(bg.exec);
@@ -809,7 +794,7 @@ int fip_autotune(size_t image_size, size_t num_baselines, float cell_size, int r
         const int tiles[2] = {32, 64};
         double tm[kStCount];
         best.persistent = 0;
-        best.stage2_rows = default_tuning(image_size).stage2_rows;
+        best.stage2_rows = default_tuning().stage2_rows;
         for (int r : records) {
             Tuning t = best;
             t.stage1_records = r;

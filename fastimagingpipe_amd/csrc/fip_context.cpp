@@ -238,15 +238,14 @@ int Context::plan(size_t image, Plan** out)
     return FIP_OK;
 }
 
-Tuning default_tuning(size_t image)
+Tuning default_tuning()
 {
     Tuning t;
     // Gridding records per thread in registers: 2, the autotuner's choice at
     // 4096^2 and 2048^2 on MI355X (each thread's records stay resident up
     // to 1024 per column; heavier columns take further passes).
     t.stage1_records = 2;
-    // Without effect (the row pass takes two rows per workgroup everywhere).
-    t.stage2_rows = image <= 4096 ? 2 : 1;
+    t.stage2_rows = 2;   // what the row pass takes
     t.splat_tile = 0;
     t.persistent = 0;
     return t;
@@ -256,7 +255,7 @@ Tuning Context::tuning(size_t image) const
 {
     auto it = tunings_.find(image);
     if (it != tunings_.end()) return it->second;
-    return default_tuning(image);
+    return default_tuning();
 }
 
 int Context::order_work(hipStream_t st)

@@ -55,7 +55,7 @@ struct PlanHostTables {
 void plan_host_tables(size_t image, PlanHostTables& t);
 
 // Launch parameters used until the autotuner or fip_set_tuning picks others.
-Tuning default_tuning(size_t image);
+Tuning default_tuning();
 
 // Work buffers in the order rec, sorted, bstart, meta, geom, kt, pre, img,
 // pmax: their byte sizes for S snapshots.

@@ -205,7 +205,7 @@ extern "C" int fip_pipe_device_noalloc(const float* vis_re, const float* vis_im,
         w.stride = num_baselines;
         hipStream_t st = static_cast<hipStream_t>(stream);
         InputView in{vis_re, vis_im, bin, vin, nullptr, num_baselines, (int)num_baselines, FIP_VIS_F32};
-        return pipe_sequence(nullptr, p, w, in, (int)num_baselines, cell_size, default_tuning(image_size),
+        return pipe_sequence(nullptr, p, w, in, (int)num_baselines, cell_size, default_tuning(),
                              reinterpret_cast<const int*>(base + L.win), (int)unit_size, result, st);
     } catch (...) {
         return set_error(FIP_ERR_HIP, "unexpected exception");
