@@ -78,8 +78,7 @@ void PinnedBuf::release()
 
 // ---------------------------------------------------------------- work
 
-// Bytes of each work buffer for S snapshots, in the order rec, sorted,
-// bstart, meta, geom, kt, pre, img, pmax.
+// Bytes of each work buffer for S snapshots, in the order of WorkBuf.
 void work_sizes(int S, size_t stride, const PlanTables& p, size_t out[kWorkBufs])
 {
     const size_t s = (size_t)S;

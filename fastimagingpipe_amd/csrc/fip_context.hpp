@@ -57,9 +57,8 @@ void plan_host_tables(size_t image, PlanHostTables& t);
 // Launch parameters used until the autotuner or fip_set_tuning picks others.
 Tuning default_tuning();
 
-// Work buffers in the order rec, sorted, bstart, meta, geom, kt, pre, img,
-// pmax: their byte sizes for S snapshots.
-constexpr int kWorkBufs = 9;
+// Work buffers and their byte sizes for S snapshots.
+enum WorkBuf { kWorkRec, kWorkSorted, kWorkBstart, kWorkMeta, kWorkGeom, kWorkKt, kWorkPre, kWorkImg, kWorkPmax, kWorkBufs };
 void work_sizes(int S, size_t stride, const PlanTables& p, size_t out[kWorkBufs]);
 
 // Work buffers sized for S snapshots of one image size and stride.

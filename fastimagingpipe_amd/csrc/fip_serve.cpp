@@ -18,9 +18,9 @@
 // next, so its GPU queue does not run dry while the completion thread
 // relaunches.  Other snapshots wait in the stream's queue; when a sequence
 // completes, the completion thread launches the queued snapshots (up to
-// kServeBatch, in consecutive ring slots) as one multi-snapshot sequence.  An idle stream launches a
-// snapshot at once, alone, so the latency at low load is that of one
-// snapshot.
+// kServeBatch, in consecutive ring slots) as one multi-snapshot sequence.  An
+// idle stream launches a snapshot at once, alone, so the latency at low load is
+// that of one snapshot.
 //
 // Admission by HBM budget: at creation every stream's fixed device state
 // (work buffers, ring, window table) plus one snapshot of the largest
@@ -35,6 +35,7 @@
 #include "fip_plan.hpp"
 
 #include <algorithm>
+#include <array>
 #include <atomic>
 #include <chrono>
 #include <cmath>
@@ -100,22 +101,42 @@ BatchLayout batch_layout(const fip_stream_config& c)
     return L;
 }
 
-// Fixed device bytes a stream is admitted with: work buffers and gathered
-// inputs for kServeBatch snapshots, the ring of images with their metadata and
-// max slots, the window table and the tLISI of kServeBatch windows.  The
-// visibilities count 56 bytes each and the grid 8 bytes per row; the front end
-// holds 48 of the one and 2 of the other.
-constexpr size_t kAdmitGeom = 136;   // of a snapshot's geometry
+// Fixed device buffers of one stream, in the order of SubStream::buffers():
+// work buffers and gathered inputs for kServeBatch snapshots, the ring of images
+// with their metadata and max slots, the window table and the tLISI of
+// kServeBatch windows.  The same sizes are admitted and allocated.
+constexpr int kStreamBufs = 12;
+using StreamSizes = std::array<size_t, kStreamBufs>;
+
+StreamSizes stream_sizes(const fip_stream_config& c, int ring)
+{
+    PlanTables p{};
+    p.I = (int)c.image_size;
+    p.G = (int)grid_size_for(c.image_size);
+    p.M = p.G / 2;
+    const size_t un = c.image_size / c.unit_size;
+    size_t batch[kWorkBufs], slots[kWorkBufs];
+    work_sizes(kServeBatch, c.num_baselines, p, batch);
+    work_sizes(ring, c.num_baselines, p, slots);
+    return {batch[kWorkRec],
+            batch[kWorkSorted],
+            batch[kWorkBstart],
+            batch[kWorkGeom],
+            batch[kWorkKt],
+            batch[kWorkPre],
+            batch_layout(c).bytes,
+            slots[kWorkMeta],
+            slots[kWorkImg],
+            slots[kWorkPmax],
+            (size_t)ring * 3 * sizeof(int),
+            kServeBatch * un * un * sizeof(float)};
+}
 
 size_t stream_fixed_bytes(const fip_stream_config& c, int ring)
 {
-    const size_t I = c.image_size, N = c.num_baselines, B = kServeBatch;
-    const size_t G = grid_size_for(I), M = G / 2;
-    const size_t un = I / c.unit_size;
-    const size_t work = N * sizeof(VisRec) * 2 + N * sizeof(int2) + G * 4 + (G + 1) * 4 + I * (M + 1) * 8 + I * I * 4;
-    const size_t ringb = (size_t)ring * (I * I * 4 + sizeof(SnapMeta) + kAdmitGeom) +
-                         pmax_words(ring) * sizeof(unsigned) + 3 * sizeof(int) * (size_t)ring;
-    return B * work + batch_layout(c).bytes + ringb + B * un * un * 4 + 256;
+    size_t sum = 0;
+    for (size_t b : stream_sizes(c, ring)) sum += b;
+    return sum;
 }
 
 // One launch copies the queued snapshots' inputs from their reservations into
@@ -164,10 +185,14 @@ struct SubStream {
     Tuning tu{};
     hipStream_t hs = nullptr;   // launch sequences
     hipStream_t cs = nullptr;   // input copies, so they run under the sequences
-    DevBuf rec, sorted, bstart, kt, pre;                       // kServeBatch snapshots
+    DevBuf rec, sorted, bstart, geom, kt, pre;                 // kServeBatch snapshots
     DevBuf batch_in;                                           // gathered inputs (BatchLayout)
-    DevBuf img, meta, geom, pmax;                              // ring
+    DevBuf meta, img, pmax;                                    // ring
     DevBuf win, out;
+    std::array<DevBuf*, kStreamBufs> buffers()
+    {
+        return {&rec, &sorted, &bstart, &geom, &kt, &pre, &batch_in, &meta, &img, &pmax, &win, &out};
+    }
     InLayout lay{};
     // Admitted snapshots waiting for a launch sequence, and the sequences
     // enqueued and not yet completed (at most kMaxRunning); both guarded by
@@ -178,7 +203,6 @@ struct SubStream {
     long submitted = 0;
     std::vector<float> latest;
     long latest_window = -1;
-    int G = 0, M = 0;
 };
 
 // First-fit allocator over [0, size) with coalescing frees.
@@ -336,7 +360,7 @@ int launch_queued(fip_server* srv, SubStream& ss)
     w.sorted = ss.sorted.as<VisRec>();
     w.bstart = ss.bstart.as<int>();
     w.meta = ss.meta.as<SnapMeta>() + r0;
-    w.geom = ss.geom.as<SnapGeom>() + r0;
+    w.geom = ss.geom.as<SnapGeom>();
     w.kt = ss.kt.as<float2>();
     w.pre = ss.pre.as<float>();
     w.img = ss.img.as<float>() + (size_t)r0 * plane;
@@ -561,35 +585,23 @@ int fip_server_create(const fip_stream_config* streams, int nstreams, int ring, 
             ss->lay = in_layout(streams[k]);
             if (int rc = C->plan(ss->cfg.image_size, &ss->plan)) return fail(rc);
             ss->tu = C->tuning(ss->cfg.image_size);
-            ss->G = ss->plan->t.G;
-            ss->M = ss->plan->t.M;
-            const size_t I = ss->cfg.image_size, N = ss->cfg.num_baselines;
-            const size_t un = I / ss->cfg.unit_size;
+            const size_t un = ss->cfg.image_size / ss->cfg.unit_size;
             SubStream* ssp = ss.get();
             srv->streams.push_back(std::move(ss));
             e = hipStreamCreateWithFlags(&ssp->hs, hipStreamNonBlocking);
             if (e != hipSuccess) return fail(hip_error(e, "hipStreamCreate"));
             e = hipStreamCreateWithFlags(&ssp->cs, hipStreamNonBlocking);
             if (e != hipSuccess) return fail(hip_error(e, "hipStreamCreate"));
-            const size_t G = ssp->G, M = ssp->M, B = kServeBatch;
-            for (auto pr : {std::make_pair(&ssp->rec, B * N * sizeof(VisRec)),
-                            std::make_pair(&ssp->sorted, B * N * sizeof(VisRec)),
-                            std::make_pair(&ssp->bstart, B * bstart_words((int)G) * sizeof(int)),
-                            std::make_pair(&ssp->kt, B * I * (M + 1) * 8), std::make_pair(&ssp->pre, B * I * I * 4),
-                            std::make_pair(&ssp->batch_in, batch_layout(ssp->cfg).bytes),
-                            std::make_pair(&ssp->img, (size_t)ring * I * I * 4),
-                            std::make_pair(&ssp->meta, (size_t)ring * sizeof(SnapMeta)),
-                            std::make_pair(&ssp->geom, (size_t)ring * sizeof(SnapGeom)),
-                            std::make_pair(&ssp->pmax, pmax_words(ring) * sizeof(unsigned)),
-                            std::make_pair(&ssp->win, (size_t)3 * sizeof(int) * ring),
-                            std::make_pair(&ssp->out, B * un * un * 4)}) {
-                e = pr.first->ensure(pr.second);
+            const StreamSizes sizes = stream_sizes(ssp->cfg, ring);
+            for (int i = 0; i < kStreamBufs; ++i) {
+                e = ssp->buffers()[i]->ensure(sizes[i]);
                 if (e != hipSuccess) return fail(hip_error(e, "hipMalloc (server)"));
             }
             // Every buffer is written once here, so the first snapshots after
-            // creation do not pay the first use of freshly allocated memory.
-            for (DevBuf* b : {&ssp->rec, &ssp->sorted, &ssp->bstart, &ssp->kt, &ssp->pre, &ssp->batch_in, &ssp->img,
-                              &ssp->meta, &ssp->geom, &ssp->pmax, &ssp->out}) {
+            // creation do not pay the first use of freshly allocated memory
+            // (the window table by its copy below, on no stream of its own).
+            for (DevBuf* b : ssp->buffers()) {
+                if (b == &ssp->win) continue;
                 e = hipMemsetAsync(b->p, 0, b->cap, ssp->hs);
                 if (e != hipSuccess) return fail(hip_error(e, "hipMemsetAsync (server)"));
             }
@@ -796,8 +808,7 @@ void fip_server_destroy(fip_server* srv)
     srv->pcv.notify_one();
     if (srv->poller.joinable()) srv->poller.join();
     for (auto& ss : srv->streams) {
-        for (DevBuf* b : {&ss->rec, &ss->sorted, &ss->bstart, &ss->kt, &ss->pre,
-                          &ss->batch_in, &ss->img, &ss->meta, &ss->geom, &ss->pmax, &ss->win, &ss->out})
+        for (DevBuf* b : ss->buffers())
             b->release();
         if (ss->hs) (void)hipStreamDestroy(ss->hs);
         if (ss->cs) (void)hipStreamDestroy(ss->cs);

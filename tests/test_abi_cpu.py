@@ -203,3 +203,19 @@ def test_server_argument_errors_before_any_device_use(F):
     cfg[0].image_size = 256
     assert lib.fip_server_create(cfg, 1, 8, 1 << 16, ctypes.byref(out)) == -7     # budget, before any device use
     assert not out.value
+
+
+def test_server_budget_counts_what_is_allocated(F):
+    """The bytes a refused server names are those of its buffers: a ring slot is
+    an image, its metadata (32 bytes), its maxima (128 words) and a row of the
+    window table; a visibility of each of three snapshots is two records of 24
+    bytes and its gathered input, and one snapshot's input is reserved."""
+    def need(nbl, ring, image=64):
+        out = ctypes.c_void_p()
+        cfg = (F._StreamConfig * 1)()
+        cfg[0].num_baselines, cfg[0].image_size, cfg[0].cell_size, cfg[0].unit_size = nbl, image, 5.8e-5, 16
+        assert F.lib.fip_server_create(cfg, 1, ring, 0, ctypes.byref(out)) == -7
+        return int(re.search(rb"below the (\d+) bytes", F.lib.fip_last_error()).group(1))
+
+    assert need(64, 5000) - need(64, 1000) == 4000 * (64 * 64 * 4 + 32 + 128 * 4 + 3 * 4)
+    assert need(6400, 8) - need(640, 8) == 5760 * (3 * (2 * 24 + 16) + 16)
