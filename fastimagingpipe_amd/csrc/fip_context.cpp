@@ -192,15 +192,16 @@ void plan_host_tables(size_t image, PlanHostTables& t)
     const int G = (int)grid_size_for(image);
     const int M = G / 2;
     t.twg.assign(G, make_float2(0.0f, 0.0f));
+    make_stage_twiddles(G, t.twg.data());
+    t.corr = corr_table(image, (size_t)G);
+    if (!row_pass_splits(G)) return;
     t.twm.assign(M, make_float2(0.0f, 0.0f));
     t.wpost.resize(M);
-    make_stage_twiddles(G, t.twg.data());
     make_stage_twiddles(M, t.twm.data());
     for (int k = 0; k < M; ++k) {
         const double a = 2.0 * M_PI * (double)k / (double)G;
         t.wpost[k] = make_float2((float)std::cos(a), (float)std::sin(a));
     }
-    t.corr = corr_table(image, (size_t)G);
 }
 
 int Context::plan(size_t image, Plan** out)
@@ -220,14 +221,17 @@ int Context::plan(size_t image, Plan** out)
     P->t.M = M;
     PlanHostTables h;
     plan_host_tables(image, h);
-    FIP_HIP(P->tw_g.ensure(h.twg.size() * sizeof(float2)));
-    FIP_HIP(P->tw_m.ensure(h.twm.size() * sizeof(float2)));
-    FIP_HIP(P->wpost.ensure(h.wpost.size() * sizeof(float2)));
-    FIP_HIP(P->corr.ensure(h.corr.size() * sizeof(float)));
-    FIP_HIP(hipMemcpy(P->tw_g.p, h.twg.data(), h.twg.size() * sizeof(float2), hipMemcpyHostToDevice));
-    FIP_HIP(hipMemcpy(P->tw_m.p, h.twm.data(), h.twm.size() * sizeof(float2), hipMemcpyHostToDevice));
-    FIP_HIP(hipMemcpy(P->wpost.p, h.wpost.data(), h.wpost.size() * sizeof(float2), hipMemcpyHostToDevice));
-    FIP_HIP(hipMemcpy(P->corr.p, h.corr.data(), h.corr.size() * sizeof(float), hipMemcpyHostToDevice));
+    auto upload = [](DevBuf& b, const void* src, size_t bytes) -> int {
+        FIP_HIP(b.ensure(bytes));
+        FIP_HIP(hipMemcpy(b.p, src, bytes, hipMemcpyHostToDevice));
+        return FIP_OK;
+    };
+    if (int rc = upload(P->tw_g, h.twg.data(), h.twg.size() * sizeof(float2))) return rc;
+    if (int rc = upload(P->corr, h.corr.data(), h.corr.size() * sizeof(float))) return rc;
+    if (!h.wpost.empty()) {
+        if (int rc = upload(P->tw_m, h.twm.data(), h.twm.size() * sizeof(float2))) return rc;
+        if (int rc = upload(P->wpost, h.wpost.data(), h.wpost.size() * sizeof(float2))) return rc;
+    }
     P->t.tw_g = P->tw_g.as<float2>();
     P->t.tw_m = P->tw_m.as<float2>();
     P->t.wpost = P->wpost.as<float2>();

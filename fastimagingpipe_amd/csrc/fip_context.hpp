@@ -46,8 +46,9 @@ struct Plan {
 };
 
 // Host copies of one image size's plan tables (FP64-computed, FP32-stored):
-// stage twiddles of the length-G and length-M transforms, the C2R split
-// factors and the per-axis grid correction.
+// stage twiddles of the length-G transform, the per-axis grid correction, and
+// where the row pass splits its transform (row_pass_splits) the stage twiddles of
+// length M and the split's factors.
 struct PlanHostTables {
     std::vector<float2> twg, twm, wpost;
     std::vector<float> corr;

@@ -103,8 +103,8 @@ struct InputView {
 struct PlanTables {
     int I, G, M;
     float2* tw_g;      // stage twiddles for the length-G transform
-    float2* tw_m;      // stage twiddles for the length-M transform
-    float2* wpost;     // exp(+2 pi i k / G), k < M (split row pass of 8192^2)
+    float2* tw_m;      // stage twiddles for the length-M transform, and
+    float2* wpost;     // exp(+2 pi i k / G), k < M: only where row_pass_splits
     float* corr;       // 1 / (c(t) * norm), t = 0..I/2
 };
 
@@ -166,6 +166,9 @@ hipError_t launch_bin(const InputView& in, const WorkView& w, const PlanTables& 
                       double scale, const int* norm_n_dev, int norm_n_const, hipStream_t st);
 hipError_t launch_stage1(const WorkView& w, const PlanTables& p, int S, const Tuning& tu,
                          hipStream_t st);
+// Whether the row pass of grid G takes two transforms of length G/2 (the only
+// use of tw_m and wpost).
+bool row_pass_splits(int G);
 hipError_t launch_stage2(const WorkView& w, const PlanTables& p, int S, hipStream_t st);
 // Target tile edge of a splat of S snapshots: the tuning's, or by the size of the
 // launch where that leaves it open.

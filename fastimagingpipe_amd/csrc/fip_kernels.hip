@@ -2029,6 +2029,8 @@ static void stage2_dispatch(const WorkView& w, const PlanTables& p, int S, hipSt
                        p.corr, w.pre);
 }
 
+bool row_pass_splits(int G) { return G == 12288; }
+
 hipError_t launch_stage2(const WorkView& w, const PlanTables& p, int S, hipStream_t st)
 {
     switch (p.G) {

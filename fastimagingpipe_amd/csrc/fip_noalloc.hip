@@ -5,9 +5,9 @@
 // nothing.
 //
 // Layout of the array (offsets 256-byte aligned):
-//   [tables]  stage twiddles, C2R split factors and grid-correction tables of
-//             every image size whose work can fit (64..1024), and the window
-//             {0, 1, 2}; written once per device when the device is set up;
+//   [tables]  stage twiddles and grid-correction tables of every image size
+//             whose work can fit (64..1024), and the window {0, 1, 2}; written
+//             once per device when the device is set up;
 //   [work]    the work buffers of one call (rec, sorted, bstart, meta, geom,
 //             kt, pre, img, pmax), laid out per call for its shape.
 // Kernels clear what must start at zero (metadata, max slots) in their
@@ -21,7 +21,6 @@
 
 #include <hip/hip_runtime.h>
 
-#include <algorithm>
 #include <cstring>
 #include <mutex>
 #include <string>
@@ -29,8 +28,8 @@
 namespace fip {
 namespace {
 
-// 64 MiB (67.1 MB): the 1024^2 workload with 130816 baselines is admitted at
-// 66.1 MB (see admitted_bytes).
+// 64 MiB (67.1 MB): the 1024^2 workload with 130816 baselines needs 63.0 MB
+// (records 18.8 MB, K tiles 18.9 MB, two image sets 25.2 MB).
 constexpr size_t kScratchBytes = size_t(64) << 20;
 constexpr size_t kAlign = 256;
 constexpr int kMaxDevices = 64;
@@ -53,7 +52,7 @@ namespace {
 size_t align_up(size_t x) { return (x + kAlign - 1) / kAlign * kAlign; }
 
 struct TableSlot {
-    size_t twg, twm, wpost, corr;   // byte offsets in the array
+    size_t twg, corr;   // byte offsets in the array
 };
 
 struct TableLayout {
@@ -68,13 +67,9 @@ TableLayout table_layout()
     size_t o = 0;
     for (int k = 0; k < kNumTableImages; ++k) {
         const size_t I = kTableImages[k];
-        const size_t G = grid_size_for(I), M = G / 2;
+        const size_t G = grid_size_for(I);
         L.slot[k].twg = o;
         o = align_up(o + G * sizeof(float2));
-        L.slot[k].twm = o;
-        o = align_up(o + M * sizeof(float2));
-        L.slot[k].wpost = o;
-        o = align_up(o + M * sizeof(float2));
         L.slot[k].corr = o;
         o = align_up(o + (I / 2 + 1) * sizeof(float));
     }
@@ -82,21 +77,6 @@ TableLayout table_layout()
     o = align_up(o + 3 * sizeof(int));
     L.end = o;
     return L;
-}
-
-// What a call is admitted by: 168 bytes per baseline (three snapshots' records
-// in and out of column order and their keys), the grid's counters and the
-// images, each part aligned.  The work buffers themselves take less; the
-// limit is the documented one and does not move with them.
-size_t admitted_bytes(const TableLayout& L, size_t nbl, const PlanTables& p)
-{
-    const size_t S = 3, I = (size_t)p.I, G = (size_t)p.G;
-    const size_t parts[] = {S * nbl * 24,       S * nbl * 8,   S * nbl * 24,  S * G * 4,           S * (G + 1) * 4,
-                            S * 32,             S * 136,       S * I * (p.M + 1) * 8, S * I * I * 4, S * I * I * 4,
-                            256,                pmax_words((int)S) * 4};
-    size_t o = L.end;
-    for (size_t b : parts) o = align_up(o + b);
-    return o;
 }
 
 struct DeviceScratch {
@@ -128,10 +108,6 @@ int scratch_base(int device, unsigned char** out)
             PlanHostTables h;
             plan_host_tables(kTableImages[k], h);
             FIP_HIP(hipMemcpy(base + L.slot[k].twg, h.twg.data(), h.twg.size() * sizeof(float2),
-                              hipMemcpyHostToDevice));
-            FIP_HIP(hipMemcpy(base + L.slot[k].twm, h.twm.data(), h.twm.size() * sizeof(float2),
-                              hipMemcpyHostToDevice));
-            FIP_HIP(hipMemcpy(base + L.slot[k].wpost, h.wpost.data(), h.wpost.size() * sizeof(float2),
                               hipMemcpyHostToDevice));
             FIP_HIP(hipMemcpy(base + L.slot[k].corr, h.corr.data(), h.corr.size() * sizeof(float),
                               hipMemcpyHostToDevice));
@@ -178,7 +154,6 @@ extern "C" int fip_pipe_device_noalloc(const float* vis_re, const float* vis_im,
             off[i] = o;
             o = align_up(o + sz[i]);
         }
-        o = std::max(o, admitted_bytes(L, num_baselines, p));
         if (o > kScratchBytes)
             return set_error(FIP_ERR_SIZE, "fip_pipe_device_noalloc: " + std::to_string(num_baselines) +
                                                " baselines at " + std::to_string(image_size) + "^2 need " +
@@ -189,19 +164,17 @@ extern "C" int fip_pipe_device_noalloc(const float* vis_re, const float* vis_im,
         unsigned char* base = nullptr;
         if (int rc = scratch_base(dev, &base)) return rc;
         p.tw_g = reinterpret_cast<float2*>(base + L.slot[k].twg);
-        p.tw_m = reinterpret_cast<float2*>(base + L.slot[k].twm);
-        p.wpost = reinterpret_cast<float2*>(base + L.slot[k].wpost);
         p.corr = reinterpret_cast<float*>(base + L.slot[k].corr);
         WorkView w{};
-        w.rec = reinterpret_cast<VisRec*>(base + off[0]);
-        w.sorted = reinterpret_cast<VisRec*>(base + off[1]);
-        w.bstart = reinterpret_cast<int*>(base + off[2]);
-        w.meta = reinterpret_cast<SnapMeta*>(base + off[3]);
-        w.geom = reinterpret_cast<SnapGeom*>(base + off[4]);
-        w.kt = reinterpret_cast<float2*>(base + off[5]);
-        w.pre = reinterpret_cast<float*>(base + off[6]);
-        w.img = reinterpret_cast<float*>(base + off[7]);
-        w.pmax = reinterpret_cast<unsigned*>(base + off[8]);
+        w.rec = reinterpret_cast<VisRec*>(base + off[kWorkRec]);
+        w.sorted = reinterpret_cast<VisRec*>(base + off[kWorkSorted]);
+        w.bstart = reinterpret_cast<int*>(base + off[kWorkBstart]);
+        w.meta = reinterpret_cast<SnapMeta*>(base + off[kWorkMeta]);
+        w.geom = reinterpret_cast<SnapGeom*>(base + off[kWorkGeom]);
+        w.kt = reinterpret_cast<float2*>(base + off[kWorkKt]);
+        w.pre = reinterpret_cast<float*>(base + off[kWorkPre]);
+        w.img = reinterpret_cast<float*>(base + off[kWorkImg]);
+        w.pmax = reinterpret_cast<unsigned*>(base + off[kWorkPmax]);
         w.stride = num_baselines;
         hipStream_t st = static_cast<hipStream_t>(stream);
         InputView in{vis_re, vis_im, bin, vin, nullptr, num_baselines, (int)num_baselines, FIP_VIS_F32};

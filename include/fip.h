@@ -81,7 +81,7 @@ int fip_pipe_device(const float *vis_re, const float *vis_im, const float *bin,
  * intermediate buffer and plan table lives in one static 64 MiB device array
  * per GPU, held until the process ends; the call makes no hipMalloc,
  * hipFree or other allocating call.  Image sizes 64..1024 whose work fits
- * the array (1024^2 with up to 130816 baselines); larger shapes return
+ * the array (1024^2 with up to 159740 baselines); larger shapes return
  * FIP_ERR_SIZE.  The first call on a device writes the plan tables into the
  * array with synchronous copies; later calls only enqueue kernels on
  * `stream` (NULL: the default stream).  All calls on one GPU share the

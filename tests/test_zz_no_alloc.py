@@ -68,3 +68,15 @@ def test_noalloc_refuses_shapes_beyond_its_array(fip):
         fip.pipe_device_noalloc(big[0].addr, big[1].addr, big[2].addr, big[3].addr, out.addr, n, 1024, 3,
                                 2.9e-5, 32)
     assert e.value.status == -3
+
+
+def test_noalloc_at_the_end_of_its_array(fip):
+    """The most baselines the array holds at 1024^2, and one more."""
+    image, nbl, cell, tile = 1024, 159740, 2.9e-5, 32
+    dev = _device_inputs(*snapshots(710, 3, nbl + 1, image, cell))
+    got = _run(fip, fip.pipe_device_noalloc, dev, nbl, image, cell, tile)
+    ref = _run(fip, fip.pipe_device, dev, nbl, image, cell, tile)
+    assert np.array_equal(got.view(np.uint32), ref.view(np.uint32))
+    with pytest.raises(fip.FipError) as e:
+        _run(fip, fip.pipe_device_noalloc, dev, nbl + 1, image, cell, tile)
+    assert e.value.status == -3
