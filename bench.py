@@ -92,13 +92,17 @@ def stage_bytes(nbl, image, g, rmax, tile, nsnap=3, nwin=1, fused=False):
 
 
 def load_traffic(stage: str):
-    """HBM bytes per launch measured with rocprofv3 --pmc (copy-calibrated), if present."""
+    """HBM bytes per launch measured with rocprofv3 --pmc (copy-calibrated), if present.
+    The front end's time ("bin") is that of up to three kernels, and so are its bytes."""
     if not os.path.exists(TRAFFIC_FILE):
         return None
     try:
         with open(TRAFFIC_FILE) as f:
-            k = json.load(f)["kernels"].get(stage)
-        return None if k is None else int(round(k["bytes"]))
+            kernels = json.load(f)["kernels"]
+        if stage not in kernels:
+            return None
+        parts = ("bin", "offsets", "merge") if stage == "bin" else (stage,)
+        return int(round(sum(kernels[k]["bytes"] for k in parts if k in kernels)))
     except Exception:
         return None
 

@@ -96,3 +96,16 @@ def test_trace_statistics_over_the_last_dispatches(tmp_path):
     assert rows[SPLAT]["median_ns"] == pytest.approx(110000.0)
     assert rows[SPLAT]["min_ns"] == 100000.0 and rows[SPLAT]["max_ns"] == 120000.0
     assert rows[C2R]["calls"] == 2 and rows[C2R]["avg_ns"] == pytest.approx(95000.0)
+
+
+def test_bench_counts_the_bytes_of_the_whole_front_end():
+    """The time of stage "bin" spans bin, offsets and merge; so do its bytes."""
+    import json
+
+    import bench
+    with open(bench.TRAFFIC_FILE) as f:
+        kernels = json.load(f)["kernels"]
+    front = sum(kernels[k]["bytes"] for k in ("bin", "offsets", "merge"))
+    assert bench.load_traffic("bin") == round(front)
+    assert bench.load_traffic("row_c2r") == round(kernels["row_c2r"]["bytes"])
+    assert bench.load_traffic("scan") is None
