@@ -284,11 +284,12 @@ __device__ __forceinline__ void bfly_masked(float2* v)
 // fewest stages that keep a butterfly's registers within occupancy: radix 16
 // and 12 in registers (three stages for 384 to 6144, four for 12288) measured
 // 3-13% faster than radix 8/4/3/2 lists of five or six stages, and 6144 as
-// 32, 16, 12 took the column kernel from 99 to 83 us at 4096^2 against
-// 16, 16, 2, 12 (one LDS round trip less; the radix-32 stage fills three of
-// the eight waves, which the CU's other workgroups cover).  Every list ends in radix 12: the last stage's outputs then lie
-// N/12 apart, so a crop to the central two thirds is four whole outputs
-// dropped per butterfly, and the kept ones leave from registers.
+// 32, 16, 12 takes the column kernel from 82 to 76 us and the row pass from 88 to
+// 85 at 4096^2 against 16, 16, 2, 12 (one LDS round trip less; the radix-32 stage
+// fills three of the eight waves, which the CU's other workgroups cover).  Every
+// list ends in radix 12: the last stage's outputs then lie N/12 apart, so a crop
+// to the central two thirds is four whole outputs dropped per butterfly, and the
+// kept ones leave from registers.
 template <int NT, int... Rs>
 struct PlanDef {
     static constexpr int nt = NT;

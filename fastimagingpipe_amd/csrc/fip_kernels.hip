@@ -297,10 +297,11 @@ __device__ __forceinline__ void set_extent(SnapMeta& m, int k, int v)
 //
 // Latency bound: at 2048^2 with 32640 visibilities 1.2 us of loads, 1.7 of
 // FP64 and LDS atomics, 1.5 of scan and 0.6 of stores; the rest of its 8 us is
-// launch and write-back.  With k_merge 7, 14, 14, 26 and 58 us (rocprofv3, three
+// launch and write-back.  With k_merge 7, 14, 16, 25 and 59 us (rocprofv3, three
 // snapshots) at 256^2, 1024^2, 2048^2, 4096^2 and 8192^2 with 2016, 8128, 32640,
-// 130816 and 523776 visibilities (the last two with k_offsets); clearing, histogram with global atomics, scan
-// and scatter as four launches took 16, 19.5, 22.6, 32 and 74.  (A column
+// 130816 and 523776 visibilities (the last two with k_offsets); clearing,
+// histogram with global atomics, scan and scatter as four launches took 16, 18,
+// 21, 32 and 73.  (A column
 // kernel that took its records from the sorted segments themselves, with no
 // merge, lost more than the merge costs: 95 against 84 us at 4096^2.)
 template <class VT, int VPT>
@@ -765,11 +766,13 @@ __device__ __forceinline__ int4 column_ranges(const int* __restrict__ bst, int c
 // instructions) and by the fullest columns' passes up to 2048^2.  Rows
 // counted from -g/2, so that a record's taps are one address plus constants,
 // the transform reading the integers and storing the crop from registers, and
-// extra waves for full columns took it from 105.6 to 83 us (4096^2, 130816
-// visibilities), 35 to 25 us (2048^2, 32640), 562 to 473 us (8192^2, 523776)
-// and 12.2 to 8 us (256^2, 2016) for three snapshots.  smem: ColShape<G>::bytes of LDS, used in turn as the blocks'
-// masses, the int32 column and the FFT's exchange buffer.  KR records per
-// thread are held in registers at a time.
+// extra waves for full columns took it from 97 to 76 us (4096^2, 130816
+// visibilities), 35 to 25 us (2048^2, 32640), 539 to 459 us (8192^2, 523776)
+// and 12.4 to 7.6 us (256^2, 2016) for three snapshots (rocprofv3).
+//
+// smem: ColShape<G>::bytes of LDS, used in turn as the blocks' masses, the int32
+// column and the FFT's exchange buffer.  KR records per thread are held in
+// registers at a time.
 template <int G, int KR>
 __device__ __forceinline__ void stage1_column(int s, int c, int4 rg, const VisRec* __restrict__ sorted,
                                               const SnapMeta& m, const float2* __restrict__ tw,
@@ -1023,8 +1026,8 @@ struct RowStore {
 // real for exact data; their real parts are taken, so no row leaks into the
 // other.
 //
-// Three images, before and after: 103.8 -> 94.7 us at 4096^2 (339 MB, 3.6 TB/s),
-// 26 -> 24 at 2048^2.  Arithmetic and LDS turns of the waves (52 us of vector
+// Three images, before and after (rocprofv3): 96 -> 86 us at 4096^2 (339 MB, 3.9
+// TB/s), 25 -> 24 at 2048^2.  Arithmetic and LDS turns of the waves (52 us of vector
 // instructions) and the start of each workgroup on cold loads bound it now.
 // Next rows' K loads held across the transform (a persistent loop) took 112
 // registers instead of 70, with fewer waves and no gain.
@@ -1102,7 +1105,7 @@ __global__ __launch_bounds__(FftPlan<G>::nt, G >= 6144 ? 6 : 2) void k_stage2(
 // outputs through the second, so each K entry is read once, 16 bytes for both
 // rows, and a row's columns 2m and 2m + 1 leave as one 8-byte store.
 //
-// Three images: 558 -> 473 us (1.46 GB, 3.1 TB/s) against one row per workgroup
+// Three images: 577 -> 467 us (1.46 GB, 3.1 TB/s) against one row per workgroup
 // as a real transform, whose 8-byte loads each touched a 64-byte piece of the
 // tiles.  119 registers, two workgroups per CU: the transforms' barriers are
 // not always covered.

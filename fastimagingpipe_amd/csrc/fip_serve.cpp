@@ -457,9 +457,14 @@ constexpr int kMaxRunning = 2;
 // takes little longer than one of one (102 against 73 us at 2048^2 with 32640
 // visibilities).  A stream submitted without a pause: 55-61 -> 43-46 us a
 // snapshot at 256^2 (2016 visibilities), 61-70 -> 51-54 at 1024^2 (8128), 83 -> 77
-// at 2048^2 (32640).  From 4096^2 on one snapshot fills the GPU and nothing is
-// held back (held back it took 204 us instead of 199).  The caller holds the context lock and srv->qmu.  A failed launch releases the
-// rest of the queue unlaunched and returns its error (also kept in
+// at 2048^2 (32640).  What arrives now and then loses nothing by the wait: with
+// the direct tLISI below, two snapshots back to back take 137 us at 256^2, 163
+// at 1024^2 and 228 at 2048^2 (182, 203 and 263 when each went out at once and
+// its tLISI by a copy), and Poisson arrivals of 8000/s at 1024^2 a median of 104
+// and a 99th percentile of 230 us (114 and 349).  From 4096^2 on one snapshot
+// fills the GPU and nothing is held back (held back it took 204 us instead of
+// 199).  The caller holds the context lock and srv->qmu.  A failed launch
+// releases the rest of the queue unlaunched and returns its error (also kept in
 // srv->launch_error).
 int launch_ready(fip_server* srv, SubStream& ss)
 {

@@ -241,7 +241,8 @@ int fip_ingest_table(const int *file_index, const double *time,
 /* Enable or disable per-stage event timing for subsequent calls. */
 int fip_set_profiling(int on);
 /* Stage names and accumulated milliseconds / launch counts since the last
- * reset; n_stages <= fip_stage_count(). */
+ * reset; n_stages <= fip_stage_count().  "bin" is the whole front end; "reset",
+ * "scan" and "scatter" keep their places in the list and stay at zero. */
 int fip_stage_count(void);
 const char *fip_stage_name(int stage);
 int fip_stage_times(double *ms, long *counts, int n_stages);
