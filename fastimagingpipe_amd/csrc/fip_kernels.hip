@@ -714,7 +714,7 @@ __device__ __forceinline__ void grid_taps(const ColRec& c, const float* sc, int*
 // Adds the record's magnitude bound (units of amax / 4096, rounded up) to the
 // mass of every scale block its taps touch (at most two).  The mass is 64-bit:
 // a column holds up to two records per visibility (its direct and mirrored
-// buckets), so a 32-bit sum of up to 4096 units per record would wrap after
+// runs), so a 32-bit sum of up to 4096 units per record would wrap after
 // about 2^19 visibilities at one uv point.  Each block's mass is kept in MC
 // copies, one per lane modulo MC: nearly all records of a full column lie in
 // the few blocks around row 0, where a single word per block would serialise
